@@ -249,6 +249,7 @@ extern "C" int bd_destroy(bd_ctx *c) {
     dev_free(c->d_script);
     dev_free(c->d_mlp);
     dev_free(c->d_mlp_ops);
+    dev_free(c->d_mlp_ws);
     if (c->h_ctl) (void)hipHostFree(c->h_ctl);
     for (auto &e : c->ev)
         if (e) (void)hipEventDestroy(e);

@@ -192,6 +192,8 @@ struct bd_ctx {
     uint4 *d_mlp_ops = nullptr;  // the step kernels' per-lane operand table
     int mlp_h1 = 0, mlp_h2 = 0;
     bool has_mlp = false;
+    float *d_mlp_ws = nullptr;   // training and inference workspace
+    size_t mlp_ws_bytes = 0;
     std::vector<float> h_mlp;
 
     // multi-root state

@@ -62,3 +62,42 @@ def test_device_training_matches_oracle_adam(ctx, orc):
     assert loss_dev == pytest.approx(loss_ref, rel=2e-2)
     first, _ = orc.mlp_loss_grad(p, x, t)
     assert loss_dev < first
+
+
+@pytest.mark.parametrize("n,h1,h2", [(1, 32, 32), (31, 1, 1), (32, 32, 32), (33, 5, 17),
+                                     (129, 32, 8), (8192, 32, 32), (8225, 17, 32)])
+def test_grad_and_infer_at_tile_edges(ctx, orc, n, h1, h2):
+    """Samples and hidden units at and beside the 32-wide tiles, the four
+    waves of a workgroup and the largest grid (64 x 4 x 32 samples); the fp32
+    tolerances of the tests above."""
+    p = random_params(orc, 21, h1, h2)
+    x, t = data(n, 22)
+    mask = (np.random.default_rng(23).random((n, 2)) > 0.3).astype(np.float32)
+    mask[0] = 1
+    ctx.mlp_set(p, h1, h2)
+    np.testing.assert_allclose(ctx.mlp_infer(x, mfma=False), orc.mlp_forward(p, x, h1, h2),
+                               rtol=1e-4, atol=1e-5)
+    loss, g = ctx.mlp_loss_grad(x, t, mask)
+    rloss, rg = orc.mlp_loss_grad(p, x, t, mask, h1, h2)
+    assert loss == pytest.approx(rloss, rel=1e-4)
+    np.testing.assert_allclose(g, rg, rtol=1e-3, atol=1e-5 * np.abs(rg).max())
+
+
+def test_grad_with_an_infinite_input_behind_an_idle_unit(ctx, orc):
+    """An infinite activation whose successors are all idle adds nothing to
+    any gradient: the result is that of any other positive input there."""
+    p = random_params(orc, 31)
+    p[:8] = 0
+    p[0] = 1                        # unit 0 of layer 1 sees input 0 alone
+    p[8:256].reshape(31, 8)[:, 0] = 0  # no other unit sees it
+    p[32 * 9:32 * 9 + 1024].reshape(32, 32)[:, 0] = -50  # and it idles all of layer 2
+    x, t = data(70, 32)
+    x[40, 0] = 1000.0
+    ctx.mlp_set(p)
+    loss, g = ctx.mlp_loss_grad(x, t)
+    x[40, 0] = np.inf
+    for k in range(1, 32):          # 0 * inf idles the other units of that sample too
+        assert p[8 * k] == 0
+    loss_inf, g_inf = ctx.mlp_loss_grad(x, t)
+    assert loss_inf == pytest.approx(loss, rel=1e-6)
+    np.testing.assert_allclose(g_inf, g, rtol=1e-6, atol=1e-6 * np.abs(g).max())
