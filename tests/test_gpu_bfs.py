@@ -787,3 +787,30 @@ def test_learned_policy_is_beamer_on_graphs_without_hubs(ctx, orc):
         np.testing.assert_array_equal(ctx.fetch()[0], orc.bfs_depth(off, adj, root))
     finally:
         ctx.set_tuning(**t0)
+
+
+@pytest.mark.parametrize("first", [1023, 1024, 1025, 2048])
+def test_multi_graph_finds_an_edge_between_graphs(ctx, first):
+    """The check reads 1024 list entries per wave: graphs whose lists end at
+    and beside such a cut, edge-free graphs between, and one crossing edge at
+    either end of a graph's lists."""
+    def star(n):  # n leaves: 2n entries
+        return np.concatenate([[0], n + np.arange(n + 1)]).astype(np.int64), np.concatenate(
+            [np.arange(1, n + 1), np.zeros(n)]).astype(np.int32)
+
+    a = (np.arange(first + 1, dtype=np.int64), np.arange(first, dtype=np.int32))  # self-loops
+    empty = (np.zeros(4, np.int64), np.zeros(0, np.int32))
+    off, cols = star(700)
+    graphs = [(*a, first), (*empty, 0), (*empty, 0), (off, cols, 700), (*empty, 0)]
+    o, c, m, vbase = bd.union_csr(graphs)
+    roots = np.zeros(len(graphs), np.int64)
+    ctx.upload_csr(o, c, m)
+    dp, _ = ctx.multi_graph(vbase, roots)
+    assert dp[0] == 0 and dp[1] == -1 and dp[vbase[3]] == 0 and (dp[vbase[3] + 1:vbase[4]] == 1).all()
+    for k in (0, first - 1, first, len(c) - 1):
+        x = c.copy()
+        x[k] = vbase[3] if k < first else 0
+        ctx.upload_csr(o, x, m)
+        with pytest.raises(bd.BeedrillError) as e:
+            ctx.multi_graph(vbase, roots)
+        assert e.value.code == -1
