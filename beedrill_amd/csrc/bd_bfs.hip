@@ -1829,113 +1829,6 @@ __global__ __launch_bounds__(256) void k_check_tree(const int64_t *__restrict__ 
     }
 }
 
-// Head index of the bottom-up step: head[v] = (deg(v) << 32) | the
-// neighbour of v of largest degree, the first in CSR order among equals
-// (degrees saturated at 2^31-1), or 0xffffffff when v has none.  One 8-byte
-// load gives the bottom-up step both the likeliest parent and the degree.  A vertex's highest-degree neighbour is the
-// one most likely to be reached first, so it is the likeliest parent when v
-// is scanned bottom-up; a dense array of them is read in vertex order, where
-// the first entry of each adjacency list costs a cache line per vertex.
-__device__ __forceinline__ unsigned long long head_key(const int64_t *off, int32_t u,
-                                                       int64_t pos) {
-    int64_t d = off[u + 1] - off[u];
-    d = d < 0x7fffffff ? d : 0x7fffffff;
-    return ((unsigned long long)d << 32) | (0xffffffffULL - (unsigned long long)pos);
-}
-
-// One wave per 64 vertices: a lane does its own vertex when the list is
-// shorter than 64, longer lists are done by the whole wave.
-__global__ __launch_bounds__(256) void k_head_index(const int64_t *__restrict__ off,
-                                                    const int32_t *__restrict__ cols, int64_t nv,
-                                                    uint64_t *__restrict__ head,
-                                                    unsigned long long *__restrict__ max_deg) {
-    const int lane = threadIdx.x & 63;
-    const int64_t wave = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-    const int64_t nwaves = ((int64_t)gridDim.x * blockDim.x) >> 6;
-    unsigned long long dmax = 0;
-    for (int64_t base = wave * 64; base < nv; base += nwaves * 64) {
-        const int64_t v = base + lane;
-        const bool valid = v < nv;
-        int64_t b = 0, e = 0;
-        if (valid) {
-            b = off[v];
-            e = off[v + 1];
-            dmax = (unsigned long long)(e - b) > dmax ? (unsigned long long)(e - b) : dmax;
-        }
-        const bool alone = valid && e - b < 64;
-        if (alone) {
-            unsigned long long best = 0;
-            for (int64_t k = b; k < e; ++k) {
-                const unsigned long long key = head_key(off, cols[k], k - b);
-                best = key > best ? key : best;
-            }
-            const uint32_t id =
-                best ? (uint32_t)cols[b + (int64_t)(0xffffffffULL - (best & 0xffffffffULL))]
-                     : 0xffffffffu;
-            head[v] = ((uint64_t)(e - b) << 32) | id;
-        }
-        // lists of kHubBigDeg or more: k_head_big and k_head_big_done
-        const bool big = valid && e - b >= kHubBigDeg;
-        if (big) head[v] = 0;
-        uint64_t lm = __ballot(valid && !alone && !big);
-        while (lm) {
-            const int src = __ffsll((unsigned long long)lm) - 1;
-            lm &= lm - 1;
-            const int64_t kb = lane_bcast(b, src), ke = lane_bcast(e, src);
-            unsigned long long best = 0;
-            for (int64_t k = kb + lane; k < ke; k += 64) {
-                const unsigned long long key = head_key(off, cols[k], k - kb);
-                best = key > best ? key : best;
-            }
-            best = wave_max(best);
-            if (lane == src)
-                head[v] = ((uint64_t)(ke - kb) << 32) |
-                          (uint32_t)cols[kb + (int64_t)(0xffffffffULL - (best & 0xffffffffULL))];
-        }
-    }
-    dmax = wave_max(dmax);
-    if (lane == 0 && dmax) atomicMax(max_deg, dmax);
-}
-
-// The lists of kHubBigDeg entries or more, one hub slice per wave: each
-// slice's best key (degree, then first position) is combined into head[v]
-// (cleared by k_head_index) with a 64-bit atomic maximum.
-__global__ __launch_bounds__(256) void k_head_big(const int64_t *__restrict__ off,
-                                                  const int32_t *__restrict__ cols,
-                                                  const td_task *__restrict__ big, int64_t nbig,
-                                                  uint64_t *__restrict__ head) {
-    const int lane = threadIdx.x & 63;
-    const int64_t wave = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-    const int64_t nwaves = ((int64_t)gridDim.x * blockDim.x) >> 6;
-    for (int64_t t = wave; t < nbig; t += nwaves) {
-        const td_task tk = big[t];
-        const int64_t b = off[tk.src];
-        unsigned long long best = 0;
-        for (int64_t k = tk.beg + lane; k < tk.end; k += 64) {
-            const unsigned long long key = head_key(off, cols[k], k - b);
-            best = key > best ? key : best;
-        }
-        best = wave_max(best);
-        if (lane == 0) atomicMax((unsigned long long *)&head[tk.src], best);
-    }
-}
-
-// Then each such vertex's key becomes its entry: degree and neighbour id
-// (the slice that starts its list does it).
-__global__ void k_head_big_done(const int64_t *__restrict__ off, const int32_t *__restrict__ cols,
-                                const td_task *__restrict__ big, int64_t nbig,
-                                uint64_t *__restrict__ head) {
-    for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < nbig;
-         t += (int64_t)gridDim.x * blockDim.x) {
-        const td_task tk = big[t];
-        const int64_t b = off[tk.src], e = off[tk.src + 1];
-        if (tk.beg != b) continue;
-        const unsigned long long best = head[tk.src];
-        head[tk.src] = ((uint64_t)(e - b) << 32) |
-                       (uint32_t)cols[b + (int64_t)(0xffffffffULL - (best & 0xffffffffULL))];
-    }
-}
-
 // Streams a buffer larger than the last-level cache so a timed step starts
 // from cold caches.
 __global__ void k_scrub(const uint4 *__restrict__ p, int64_t n, uint4 *__restrict__ sink) {
@@ -2191,35 +2084,6 @@ int finish_search(bd_ctx *c, int64_t source, bd_run_stats *out, double event_ms)
 }
 
 }  // namespace
-
-int build_head_index(bd_ctx *c) {
-    if (c->d_head || c->nv == 0) return BD_OK;
-    int rc = dev_alloc(c, (void **)&c->d_head, sizeof(uint64_t) * c->nv, "head index");
-    if (rc) return rc;
-    unsigned long long *d_max = nullptr;
-    if ((rc = dev_alloc(c, (void **)&d_max, sizeof(unsigned long long), "max degree"))) return rc;
-    struct guard {
-        void *p;
-        ~guard() { dev_free(p); }
-    } g{d_max};
-    BD_HIP(c, hipMemsetAsync(d_max, 0, sizeof(unsigned long long), c->stream));
-    hipLaunchKernelGGL(k_head_index, dim3(grid_for(c, c->nv, 256)), dim3(256), 0, c->stream,
-                       c->d_soff, c->d_scols, c->nv, c->d_head, d_max);
-    if (c->n_hub_big) {
-        hipLaunchKernelGGL(k_head_big, dim3(grid_for(c, c->n_hub_big * 64, 256)), dim3(256), 0,
-                           c->stream, c->d_soff, c->d_scols, c->d_hub_big, c->n_hub_big,
-                           c->d_head);
-        hipLaunchKernelGGL(k_head_big_done, dim3(grid_for(c, c->n_hub_big, 256)), dim3(256), 0,
-                           c->stream, c->d_soff, c->d_scols, c->d_hub_big, c->n_hub_big,
-                           c->d_head);
-    }
-    BD_HIP(c, hipGetLastError());
-    unsigned long long h = 0;
-    BD_HIP(c, hipMemcpyAsync(&h, d_max, sizeof(h), hipMemcpyDeviceToHost, c->stream));
-    BD_HIP(c, hipStreamSynchronize(c->stream));
-    c->max_deg = (int64_t)h;
-    return BD_OK;
-}
 
 // A search is k_init, then one k_step launch per level.  Step L publishes
 // the state before it (closing step L-1), so the launch that finds the

@@ -153,8 +153,7 @@ int alloc_search(bd_ctx *c) {
         if ((rc = dev_alloc(c, (void **)&t, sizeof(td_task) * (kSeg * c->tseg_cap + c->task_cap),
                             "tasks")))
             return rc;
-    if ((rc = build_search_layout(c))) return rc;
-    return build_head_index(c);
+    return build_search_layout(c);
 }
 
 }  // namespace bd

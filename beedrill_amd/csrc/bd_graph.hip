@@ -22,6 +22,7 @@
 #include "bd_device.h"
 #include "bd_gen_common.h"
 #include "bd_internal.h"
+#include "bd_mlp.h"
 
 namespace bd {
 
@@ -390,24 +391,47 @@ namespace {
 
 constexpr int64_t kSpreadHubs = 4096;
 
-// keys[v] = (rank class << s) | v, v < 2^s: sorting their low 32 + s bits
-// gives the search order.
-__global__ void k_order_keys(const int64_t *__restrict__ off, int64_t nv, int order, int s,
-                             uint64_t *__restrict__ keys, unsigned long long *__restrict__ active) {
-    unsigned long long n = 0;
+// stat[0] = vertices with edges, stat[1] = the largest degree.  One pair of
+// atomics per workgroup, on a grid of one workgroup per CU at most: with a
+// pair per wave the atomics on the two addresses alone took 110 us.
+__global__ __launch_bounds__(kBlock) void k_degree_stats(const int64_t *__restrict__ off, int64_t nv,
+                                                         unsigned long long *__restrict__ stat) {
+    __shared__ unsigned long long red[2][kBlock / 64];
+    unsigned long long n = 0, mx = 0;
     for (int64_t v = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; v < nv;
          v += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t d = off[v + 1] - off[v];
-        uint64_t cls;
-        if (order == 1 || order == 4)
-            cls = 0xffffffffULL - (uint64_t)(d < 0xffffffffLL ? d : 0xffffffffLL);
-        else
-            cls = d == 0 ? 1 : 0;
-        keys[v] = (cls << s) | (uint64_t)v;
+        const unsigned long long d = (unsigned long long)(off[v + 1] - off[v]);
         n += d > 0;
+        mx = d > mx ? d : mx;
     }
     n = wave_sum(n);
-    if ((threadIdx.x & 63) == 0 && n) atomicAdd(active, n);
+    mx = wave_max(mx);
+    if ((threadIdx.x & 63) == 0) {
+        red[0][threadIdx.x >> 6] = n;
+        red[1][threadIdx.x >> 6] = mx;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < kBlock / 64; ++w) {
+            n += red[0][w];
+            mx = red[1][w] > mx ? red[1][w] : mx;
+        }
+        if (n) atomicAdd(&stat[0], n);
+        if (mx) atomicMax(&stat[1], mx);
+    }
+}
+
+// keys[v] = (rank class << s) | v, v < 2^s: sorting them gives the search
+// order.  Classes run from 0 (the largest degree) to top = the largest
+// degree (capped to 32 bits), so a sort takes only the bits top needs.
+__global__ void k_order_keys(const int64_t *__restrict__ off, int64_t nv, int order, int s,
+                             uint64_t top, uint64_t *__restrict__ keys) {
+    for (int64_t v = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; v < nv;
+         v += (int64_t)gridDim.x * blockDim.x) {
+        const uint64_t d = (uint64_t)(off[v + 1] - off[v]);
+        const uint64_t cls = (order == 1 || order == 4) ? top - (d < top ? d : top) : (d == 0 ? 1 : 0);
+        keys[v] = (cls << s) | (uint64_t)v;
+    }
 }
 
 // Search id of the vertex of rank r (position in the sorted keys).  The
@@ -423,68 +447,170 @@ __device__ __forceinline__ int64_t spread_id(int64_t r, int64_t spread) {
     return r;
 }
 
+// A vertex's record, by graph id: its degree (saturated at 2^31-1) and its
+// search id, which a list pass fetches together.
+__device__ __forceinline__ uint64_t vertex_rec(int64_t deg, int64_t id) {
+    return ((uint64_t)(deg < 0x7fffffff ? deg : 0x7fffffff) << 32) | (uint32_t)id;
+}
+
 // perm[i] = graph vertex of search id i, inv its inverse, sdeg[i] its degree.
 __global__ void k_order_perm(const uint64_t *__restrict__ skeys, const int64_t *__restrict__ off,
                              int64_t nv, int s, int64_t spread, int32_t *__restrict__ perm,
-                             int32_t *__restrict__ inv, int64_t *__restrict__ sdeg) {
+                             int32_t *__restrict__ inv, int64_t *__restrict__ sdeg,
+                             uint64_t *__restrict__ rec) {
     const uint64_t vmask = (1ULL << s) - 1;
     for (int64_t r = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; r < nv;
          r += (int64_t)gridDim.x * blockDim.x) {
         const int32_t v = (int32_t)(skeys[r] & vmask);
         const int64_t i = spread_id(r, spread);
+        const int64_t d = off[v + 1] - off[v];
         perm[i] = v;
         inv[v] = (int32_t)i;
-        sdeg[i] = off[v + 1] - off[v];
+        sdeg[i] = d;
+        rec[v] = vertex_rec(d, i);
     }
 }
 
-// The renumbered lists: one wave per 64 search ids, a lane copying its own
-// list when it is shorter than 64, the whole wave otherwise.
-__global__ __launch_bounds__(256) void k_order_cols(
+// Records of a layout in the graph's own order.
+__global__ void k_own_records(const int64_t *__restrict__ off, int64_t nv,
+                              uint64_t *__restrict__ rec) {
+    for (int64_t v = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; v < nv;
+         v += (int64_t)gridDim.x * blockDim.x)
+        rec[v] = vertex_rec(off[v + 1] - off[v], v);
+}
+
+// No neighbour: the head entry of a vertex of degree 0.
+constexpr uint64_t kNoHead = 0xffffffffULL;
+
+__global__ void k_fill_heads(uint64_t *__restrict__ head, int64_t nv) {
+    for (int64_t v = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; v < nv;
+         v += (int64_t)gridDim.x * blockDim.x)
+        head[v] = kNoHead;
+}
+
+// The last vertex of [lo, nv) whose list starts at or before position k
+// (k < nnz, so it is not empty).
+__device__ __forceinline__ int64_t owner_of(const int64_t *off, int64_t lo, int64_t nv, int64_t k) {
+    int64_t hi = nv;
+    while (hi - lo > 1) {
+        const int64_t mid = (lo + hi) >> 1;
+        if (off[mid] <= k)
+            lo = mid;
+        else
+            hi = mid;
+    }
+    return lo;
+}
+
+// The renumbered lists and the head index in one pass over the adjacency.
+// head[i] = (deg(i) << 32) | the neighbour of i of largest degree, the first
+// in CSR order among equals, or 0xffffffff when i has none.  One 8-byte load
+// gives a bottom-up step both the likeliest parent (the neighbour most likely
+// to be reached first) and the degree; a dense array of them is read in
+// vertex order, where the first entry of each list costs a cache line per
+// vertex.
+//
+// Each wave takes one range of `chunk` consecutive entries of the layout, so
+// no wave gets more than another whatever the degrees are (a wave per 64
+// vertices walked the medium lists of the first vertices one after another).
+// It lists the range 64 vertices at a time, one entry per lane, four in
+// flight: the entry's owner by a search over the lanes' list starts, then
+// cols and the neighbour's record.  A vertex's best key (degree, then first
+// position) is gathered in LDS; a list that the range holds whole gets its
+// entry at once, the others meet in head[] with an atomic maximum and
+// k_heads_across finishes them.  Bound by the random reads of the records.
+// 300007 vertices, 6.0 M entries: 95 us, against 1265 + 1401 us in two passes
+// of a wave per 64 vertices.
+template <bool RENUMBER>
+__global__ __launch_bounds__(256) void k_layout_lists(
     const int64_t *__restrict__ off, const int32_t *__restrict__ cols,
-    const int32_t *__restrict__ perm, const int32_t *__restrict__ inv,
-    const int64_t *__restrict__ soff, int64_t nv, int32_t *__restrict__ scols) {
+    const int32_t *__restrict__ perm, const uint64_t *__restrict__ rec,
+    const int64_t *__restrict__ soff, int64_t nv, int64_t nnz, int64_t chunk,
+    int32_t *__restrict__ scols, uint64_t *__restrict__ head) {
+    __shared__ unsigned long long s_best[4][64];
     const int lane = threadIdx.x & 63;
-    const int64_t wave = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-    const int64_t nwaves = ((int64_t)gridDim.x * blockDim.x) >> 6;
-    for (int64_t base = wave * 64; base < nv; base += nwaves * 64) {
-        const int64_t i = base + lane;
-        const bool valid = i < nv;
-        int64_t b = 0, e = 0, sb = 0;
-        if (valid) {
-            const int32_t v = perm[i];
-            b = off[v];
-            e = off[v + 1];
-            sb = soff[i];
+    unsigned long long *best = s_best[threadIdx.x >> 6];
+    const int64_t c0 = (((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6) * chunk;
+    if (c0 >= nnz) return;
+    const int64_t end = c0 + chunk < nnz ? c0 + chunk : nnz;
+    int64_t v0 = owner_of(soff, 0, nv, c0);
+    for (int64_t k = c0; k < end;) {
+        const int64_t i = v0 + lane;
+        const int64_t b = i < nv ? soff[i] : nnz, e = i < nv ? soff[i + 1] : nnz;
+        const int64_t stop = lane_bcast(e, 63) < end ? lane_bcast(e, 63) : end;
+        if (stop <= k) {  // 64 empty lists
+            v0 = owner_of(soff, v0, nv, k);
+            continue;
         }
-        if (valid && e - b < 64)
-            for (int64_t k = b; k < e; ++k) scols[sb + (k - b)] = inv[cols[k]];
-        // lists of kHubBigDeg or more: k_order_cols_big
-        uint64_t lm = __ballot(valid && e - b >= 64 && e - b < kHubBigDeg);
-        while (lm) {
-            const int src = __ffsll((unsigned long long)lm) - 1;
-            lm &= lm - 1;
-            const int64_t kb = lane_bcast(b, src), ke = lane_bcast(e, src),
-                          so = lane_bcast(sb, src);
-            for (int64_t k = kb + lane; k < ke; k += 64) scols[so + (k - kb)] = inv[cols[k]];
+        // old list start minus new
+        const int64_t shift = RENUMBER && i < nv && e > b ? off[perm[i]] - b : 0;
+        best[lane] = 0;
+        wave_lds_sync();
+        for (int64_t q0 = k; q0 < stop; q0 += 4 * 64) {
+            int o[4];
+            int32_t u[4];
+            uint64_t r[4];
+            int64_t bo[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int64_t q = q0 + 64 * j + lane;
+                const int64_t qa = q < stop ? q : stop - 1;
+                o[j] = 0;
+#pragma unroll
+                for (int st = 32; st > 0; st >>= 1) {
+                    const int mid = o[j] + st;
+                    if (__shfl(b, mid) <= qa) o[j] = mid;
+                }
+                bo[j] = __shfl(b, o[j]);
+                u[j] = __builtin_nontemporal_load(cols + qa + __shfl(shift, o[j]));
+            }
+#pragma unroll
+            for (int j = 0; j < 4; ++j) r[j] = rec[u[j]];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int64_t q = q0 + 64 * j + lane;
+                const bool live = q < stop;
+                if (RENUMBER && live) scols[q] = (int32_t)(uint32_t)r[j];
+                unsigned long long key =
+                    live ? ((r[j] >> 32) << 32) | (0xffffffffULL - (uint64_t)(q - bo[j])) : 0ULL;
+                if (lane_bcast(o[j], 0) == lane_bcast(o[j], 63)) {
+                    // one list: one write instead of 64 on one address
+                    key = wave_max(key);
+                    if (lane == 0 && key) atomicMax(&best[o[j]], key);
+                } else if (live) {
+                    atomicMax(&best[o[j]], key);
+                }
+            }
         }
+        wave_lds_sync();
+        const unsigned long long key = best[lane];
+        if (key) {
+            if (b >= c0 && e <= end)
+                head[i] = ((uint64_t)(e - b) << 32) |
+                          (uint32_t)rec[cols[b + shift + (int64_t)(0xffffffffULL - (key & 0xffffffffULL))]];
+            else
+                atomicMax((unsigned long long *)&head[i], key);
+        }
+        wave_lds_sync();
+        k = stop;
+        v0 += 64;
     }
 }
 
-// The lists of kHubBigDeg entries or more, one slice of the layout's hub
-// slices per wave (in degree order they would share a few waves above).
-__global__ __launch_bounds__(256) void k_order_cols_big(
-    const int64_t *__restrict__ off, const int32_t *__restrict__ cols,
-    const int32_t *__restrict__ perm, const int32_t *__restrict__ inv,
-    const int64_t *__restrict__ soff, const td_task *__restrict__ big, int64_t nbig,
-    int32_t *__restrict__ scols) {
-    const int lane = threadIdx.x & 63;
-    const int64_t wave = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-    const int64_t nwaves = ((int64_t)gridDim.x * blockDim.x) >> 6;
-    for (int64_t t = wave; t < nbig; t += nwaves) {
-        const td_task tk = big[t];
-        const int64_t ob = off[perm[tk.src]] - soff[tk.src];  // old minus new list start
-        for (int64_t k = tk.beg + lane; k < tk.end; k += 64) scols[k] = inv[cols[ob + k]];
+// The lists that lie across ranges: each one's best key becomes its entry,
+// by the thread of the first range that starts inside it.
+__global__ void k_heads_across(const int64_t *__restrict__ off, const int32_t *__restrict__ cols,
+                               const int32_t *__restrict__ perm, const uint64_t *__restrict__ rec,
+                               const int64_t *__restrict__ soff, int64_t nv, int64_t nnz,
+                               int64_t chunk, uint64_t *__restrict__ head) {
+    for (int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x + 1; c * chunk < nnz;
+         c += (int64_t)gridDim.x * blockDim.x) {
+        const int64_t i = owner_of(soff, 0, nv, c * chunk);
+        const int64_t b = soff[i], e = soff[i + 1];
+        if (b == c * chunk || b < (c - 1) * chunk) continue;
+        const uint64_t key = head[i];
+        const int64_t at = (perm ? off[perm[i]] : b) + (int64_t)(0xffffffffULL - (key & 0xffffffffULL));
+        head[i] = ((uint64_t)(e - b) << 32) | (uint32_t)rec[cols[at]];
     }
 }
 
@@ -542,34 +668,76 @@ static int build_hubs(bd_ctx *c) {
     return BD_OK;
 }
 
+// The layout's lists (renumbered when it has an order of its own) and head
+// index, from the vertices' records.
+static int build_lists(bd_ctx *c, const uint64_t *rec) {
+    int rc;
+    if ((rc = dev_alloc(c, (void **)&c->d_head, sizeof(uint64_t) * c->nv, "head index"))) return rc;
+    hipLaunchKernelGGL(k_fill_heads, dim3(grid1d(c, c->nv)), dim3(kBlock), 0, c->stream, c->d_head,
+                       c->nv);
+    if (c->nnz > 0) {
+        // one range per wave of a grid that fills the device; at least 512
+        // entries, since each range starts with a search for its first vertex
+        const int64_t waves = (int64_t)c->cu_count * 16 * (kBlock / 64);
+        const int64_t chunk = std::max<int64_t>((c->nnz + waves - 1) / waves, 512);
+        const int64_t n = (c->nnz + chunk - 1) / chunk;
+        const dim3 grid((unsigned)((n * 64 + kBlock - 1) / kBlock)), block(kBlock);
+        if (c->d_perm)
+            hipLaunchKernelGGL(k_layout_lists<true>, grid, block, 0, c->stream, c->d_off, c->d_cols,
+                               c->d_perm, rec, c->d_soff, c->nv, c->nnz, chunk, c->d_scols,
+                               c->d_head);
+        else
+            hipLaunchKernelGGL(k_layout_lists<false>, grid, block, 0, c->stream, c->d_off,
+                               c->d_cols, c->d_perm, rec, c->d_soff, c->nv, c->nnz, chunk,
+                               c->d_scols, c->d_head);
+        if (n > 1)
+            hipLaunchKernelGGL(k_heads_across, dim3(grid1d(c, n)), block, 0, c->stream, c->d_off,
+                               c->d_cols, c->d_perm, rec, c->d_soff, c->nv, c->nnz, chunk,
+                               c->d_head);
+    }
+    BD_HIP(c, hipGetLastError());
+    return BD_OK;
+}
+
 int build_search_layout(bd_ctx *c) {
     const int order = c->tune.vertex_order;
-    if (c->s_order == order && c->d_soff) return BD_OK;
+    if (c->s_order == order && c->d_soff && c->d_head) return BD_OK;
     free_search_layout(c);
     const int64_t nv = c->nv, nnz = c->nnz;
     int rc;
-    dev_buf keys, skeys, sdeg, cnt, tmp;
-    if ((rc = dev_alloc(c, &cnt.p, sizeof(unsigned long long), "active count"))) return rc;
-    if ((rc = dev_alloc(c, &keys.p, sizeof(uint64_t) * nv, "order keys"))) return rc;
-    BD_HIP(c, hipMemsetAsync(cnt.p, 0, sizeof(unsigned long long), c->stream));
-    const int sh = bits_for(nv);
-    hipLaunchKernelGGL(k_order_keys, dim3(grid1d(c, nv)), dim3(kBlock), 0, c->stream, c->d_off,
-                       nv, order == 2 ? 3 : order, sh, keys.as<uint64_t>(),
-                       cnt.as<unsigned long long>());
+    dev_buf keys, skeys, sdeg, cnt, tmp, rec;
+    if ((rc = dev_alloc(c, &cnt.p, 2 * sizeof(unsigned long long), "degree counts"))) return rc;
+    BD_HIP(c, hipMemsetAsync(cnt.p, 0, 2 * sizeof(unsigned long long), c->stream));
+    hipLaunchKernelGGL(k_degree_stats, dim3(std::min<int64_t>(grid1d(c, nv), c->cu_count)),
+                       dim3(kBlock), 0, c->stream, c->d_off, nv, cnt.as<unsigned long long>());
     BD_HIP(c, hipGetLastError());
-    unsigned long long active = 0;
-    BD_HIP(c, hipMemcpyAsync(&active, cnt.p, sizeof(active), hipMemcpyDeviceToHost, c->stream));
+    unsigned long long stat[2] = {0, 0};
+    BD_HIP(c, hipMemcpyAsync(stat, cnt.p, sizeof(stat), hipMemcpyDeviceToHost, c->stream));
+    if ((rc = dev_alloc(c, &rec.p, sizeof(uint64_t) * nv, "vertex records"))) return rc;
     BD_HIP(c, hipStreamSynchronize(c->stream));
-    c->nv_active = (int64_t)active;
+    c->nv_active = (int64_t)stat[0];
+    c->max_deg = (int64_t)stat[1];
     if (order == 2) {  // the graph's own order
         c->d_soff = c->d_off;
         c->d_scols = c->d_cols;
         c->d_sdead = c->d_dead;
+        hipLaunchKernelGGL(k_own_records, dim3(grid1d(c, nv)), dim3(kBlock), 0, c->stream, c->d_off,
+                           nv, rec.as<uint64_t>());
+        if ((rc = build_hubs(c)) || (rc = build_lists(c, rec.as<uint64_t>()))) return rc;
+        BD_HIP(c, hipStreamSynchronize(c->stream));
         c->s_order = order;
-        return build_hubs(c);
+        return BD_OK;
     }
+    const int sh = bits_for(nv);
+    const uint64_t top = std::min<uint64_t>(stat[1], 0xffffffffULL);
+    const int cls_bits = order == 3 ? 1 : bits_for((int64_t)top + 1);
+    if ((rc = dev_alloc(c, &keys.p, sizeof(uint64_t) * nv, "order keys"))) return rc;
+    hipLaunchKernelGGL(k_order_keys, dim3(grid1d(c, nv)), dim3(kBlock), 0, c->stream, c->d_off, nv,
+                       order, sh, top, keys.as<uint64_t>());
+    BD_HIP(c, hipGetLastError());
     if ((rc = dev_alloc(c, &skeys.p, sizeof(uint64_t) * nv, "sorted order keys"))) return rc;
-    if ((rc = sort_keys_u64(c, keys.as<uint64_t>(), skeys.as<uint64_t>(), nv, 32 + sh))) return rc;
+    if ((rc = sort_keys_u64(c, keys.as<uint64_t>(), skeys.as<uint64_t>(), nv, cls_bits + sh)))
+        return rc;
     if ((rc = dev_alloc(c, &sdeg.p, sizeof(int64_t) * nv, "search degrees"))) return rc;
     // from here the layout owns what it allocates (freed by free_search_layout)
     if ((rc = dev_alloc(c, (void **)&c->d_perm, sizeof(int32_t) * nv, "search order"))) return rc;
@@ -585,7 +753,7 @@ int build_search_layout(bd_ctx *c) {
     const int64_t spread = order == 1 ? std::min<int64_t>(kSpreadHubs, c->nv_active / 64) : 0;
     hipLaunchKernelGGL(k_order_perm, dim3(grid1d(c, nv)), dim3(kBlock), 0, c->stream,
                        skeys.as<uint64_t>(), c->d_off, nv, sh, spread, c->d_perm, c->d_inv,
-                       sdeg.as<int64_t>());
+                       sdeg.as<int64_t>(), rec.as<uint64_t>());
     BD_HIP(c, hipGetLastError());
     BD_HIP(c, hipMemsetAsync(c->d_soff, 0, sizeof(int64_t), c->stream));
     size_t tb = 0;
@@ -594,13 +762,7 @@ int build_search_layout(bd_ctx *c) {
     if ((rc = dev_alloc(c, &tmp.p, tb, "scan temp"))) return rc;
     BD_HIP(c, rocprim::inclusive_scan(tmp.p, tb, sdeg.as<int64_t>(), c->d_soff + 1, (size_t)nv,
                                       rocprim::plus<int64_t>(), c->stream));
-    if ((rc = build_hubs(c))) return rc;
-    hipLaunchKernelGGL(k_order_cols, dim3(grid1d(c, nv)), dim3(kBlock), 0, c->stream, c->d_off,
-                       c->d_cols, c->d_perm, c->d_inv, c->d_soff, nv, c->d_scols);
-    if (c->n_hub_big)
-        hipLaunchKernelGGL(k_order_cols_big, dim3(grid1d(c, c->n_hub_big * 64)), dim3(kBlock), 0,
-                           c->stream, c->d_off, c->d_cols, c->d_perm, c->d_inv, c->d_soff,
-                           c->d_hub_big, c->n_hub_big, c->d_scols);
+    if ((rc = build_hubs(c)) || (rc = build_lists(c, rec.as<uint64_t>()))) return rc;
     hipLaunchKernelGGL(k_dead_bitmap, dim3(grid1d(c, c->nwords * 64)), dim3(kBlock), 0, c->stream,
                        c->d_soff, nv, c->nwords, c->d_sdead);
     BD_HIP(c, hipGetLastError());

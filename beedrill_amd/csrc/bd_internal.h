@@ -118,7 +118,7 @@ struct bd_ctx {
     int32_t *d_cols = nullptr;
     uint64_t *d_dead = nullptr;   // 1 = vertex of degree 0, or padding bit
     uint64_t *d_head = nullptr;   // bottom-up head index, in search ids (built with the layout)
-    int64_t max_deg = 0;          // largest degree (found with the head index)
+    int64_t max_deg = 0;          // largest degree (found with the layout)
     uint64_t *d_el = nullptr;     // el64 order, packed (src << 32) | dst
     int64_t el_m = 0;
 
@@ -227,13 +227,12 @@ int dev_alloc(bd_ctx *c, void **p, size_t bytes, const char *what);
 void dev_free(void *p);
 // Release all graph-dependent buffers.
 void free_graph(bd_ctx *c);
-// (Re)allocate search buffers for the resident graph (and build its head
-// index if it has none).
+// (Re)allocate search buffers for the resident graph (and build its search
+// layout if it has none in the tuned order).
 int alloc_search(bd_ctx *c);
-// Head index of the bottom-up step for the resident graph.
-int build_head_index(bd_ctx *c);
-// Search layout of the resident graph in the tuned vertex order (no-op when
-// it is built in that order); frees it first when the order changed.
+// Search layout of the resident graph in the tuned vertex order, with the
+// bottom-up head index (no-op when it is built in that order); frees it first
+// when the order changed.
 int build_search_layout(bd_ctx *c);
 void free_search_layout(bd_ctx *c);
 // Drop the bit-parallel search's captured graph (its buffers are going).

@@ -814,3 +814,31 @@ def test_multi_graph_finds_an_edge_between_graphs(ctx, first):
         with pytest.raises(bd.BeedrillError) as e:
             ctx.multi_graph(vbase, roots)
         assert e.value.code == -1
+
+
+@pytest.mark.parametrize("order", [2, 4])
+@pytest.mark.parametrize("hub", [511, 513, 1024, 1537])
+def test_head_index_of_lists_across_ranges(ctx, orc, hub, order):
+    """The layout pass takes 512 consecutive list entries per wave: hubs whose
+    lists cross those cuts, whose best neighbours tie within and across
+    ranges (the first in CSR order is the head), and runs of over 64 isolated
+    vertices between them.  Bottom-up edges_examined counts depend on every
+    head entry and equal the oracle's."""
+    rng = np.random.default_rng(hub)
+    nv = 4 * hub + 900
+    ids = rng.choice(nv - 300, 2 * hub + 40, replace=False)  # the rest are isolated
+    hubs, leaves = ids[:2], ids[2:]
+    s = np.concatenate([np.full(hub, hubs[0]), np.full(hub, hubs[1]), leaves[:-1], leaves[::7]])
+    d = np.concatenate([leaves[:hub], leaves[-hub:], leaves[1:], leaves[::-1][::7]])
+    k = rng.permutation(len(s))
+    s, d = s[k].astype(np.int64), d[k].astype(np.int64)
+    t0 = ctx.get_tuning()
+    try:
+        ctx.set_tuning(vertex_order=order)
+        ctx.from_edges(nv, s, d)
+        off, adj, m = oracle_csr(orc, nv, s, d)
+        for root in (int(hubs[0]), int(leaves[5])):
+            for alpha, beta in ((15, 18), (1000000, 1000000)):
+                run_and_compare(ctx, orc, off, adj, m, root, alpha=alpha, beta=beta)
+    finally:
+        ctx.set_tuning(**t0)
