@@ -69,6 +69,9 @@ constexpr int64_t kPrecheckEdges = 1 << 16;  // top-down steps this heavy pre-ch
 // the bitmap costs less than staging, flushing and reading the lists (a
 // 4096 x 4096 lattice, 6278 levels: 68 ms against 92 ms).
 constexpr int64_t kListEdges = 1 << 14;
+// A top-down step ranks a bitmap frontier of this many vertices in ranges
+// that give every workgroup one (td_bitmap_body).
+constexpr int64_t kEvenRanges = 4096;
 // Top-down rounds of 64 edges a wave visits together (see td_visit_n).
 constexpr int kTdRounds = 2;
 // Largest bottom-up chunk (visited words per wave): a chunk's unvisited
@@ -633,10 +636,18 @@ __device__ __forceinline__ void td_bitmap_body(const step_args &a, step_smem<BLO
                                unsigned long long &dsum, unsigned long long &dmax) {
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
     const bool hubs = s.st.max_frontier_deg >= kHubDeg && s.st.frontier_deg >= kHubPassEdges;
-    const int64_t nranges = (a.live_nwords + BLOCK - 1) / BLOCK;
-    for (int64_t r = blockIdx.x; r < nranges; r += gridDim.x) {
-        const int64_t wi = r * BLOCK + tid;
-        uint64_t w = wi < a.live_nwords ? a.front[wi] : 0ULL;
+    // Words of a range: BLOCK, or, for a frontier of kEvenRanges vertices or
+    // more, a bottom-up chunk for each wave, which gives every workgroup a
+    // range when there are as many chunks as waves.  Late frontiers hold vertices
+    // of equal, low degree, which are neighbours in degree order, and one
+    // workgroup had up to 64 * BLOCK of them to expand (scale 20: 38 k
+    // vertices of 45 k edges in 44.8 us, 13.7 with even ranges).  For a light
+    // frontier the ranks of the empty ranges cost more than they spread (a
+    // lattice's levels: 9.8 us, 11.8 with even ranges).
+    const int rw = s.st.frontier >= kEvenRanges ? a.bu_words * (BLOCK / 64) : BLOCK;
+    for (int64_t w0 = (int64_t)blockIdx.x * rw; w0 < a.live_nwords; w0 += (int64_t)gridDim.x * rw) {
+        const int64_t wi = w0 + tid;
+        uint64_t w = tid < rw && wi < a.live_nwords ? a.front[wi] : 0ULL;
         if (hubs && w) w &= ~a.hub_bm[wi];
         const int32_t c = __popcll(w);
         s.w_bits[tid] = w;
@@ -661,7 +672,7 @@ __device__ __forceinline__ void td_bitmap_body(const step_args &a, step_smem<BLO
                     else
                         hi = mid;
                 }
-                v = (int32_t)((r * BLOCK + lo) * 64 +
+                v = (int32_t)((w0 + lo) * 64 +
                               select_bit(s.w_bits[lo], i - s.w_pref[lo]));
             }
             td_tile<BLOCK>(a, s, tdw, v, cnt, dsum, dmax);
@@ -1938,7 +1949,7 @@ void launch_step_block(bd_ctx *c, const step_args &a, int dirs, int64_t grid, hi
 // Launch the step kernel carrying `dirs` (kStepTD, kStepBU or kStepBoth);
 // grid <= 0 takes the tuned workgroups per CU of that kernel.  With events,
 // the launch stamps e0 at the kernel's start and e1 at its end.
-int launch_step(bd_ctx *c, const step_args &a, int dirs, int64_t grid = 0,
+int launch_step(bd_ctx *c, step_args a, int dirs, int64_t grid = 0,
                 hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr) {
     const int blk = norm_block(c->tune.block);
     if (grid <= 0) {
@@ -1947,6 +1958,13 @@ int launch_step(bd_ctx *c, const step_args &a, int dirs, int64_t grid = 0,
                                                                          : c->tune.grid_per_cu;
         grid = (int64_t)c->cu_count * std::max(1, per_cu);
     }
+    // Words of a wave's chunk: bu_words, or fewer when there are not enough
+    // words to give every wave that many.  A wave walks its chunk's vertices
+    // in rounds of 64, so on a graph smaller than the grid a level lasts as
+    // long as one chunk: at scale 16, 16 words kept 45 of 5120 waves busy
+    // (level 1 bottom-up 32.0 us, 13.0 with one word each).
+    const int64_t waves = grid * (blk / 64);
+    a.bu_words = (int32_t)std::min<int64_t>((a.live_nwords + waves - 1) / waves, a.bu_words);
     switch (blk) {
     case 128:
         launch_step_block<128>(c, a, dirs, grid, e0, e1);

@@ -842,3 +842,29 @@ def test_head_index_of_lists_across_ranges(ctx, orc, hub, order):
                 run_and_compare(ctx, orc, off, adj, m, root, alpha=alpha, beta=beta)
     finally:
         ctx.set_tuning(**t0)
+
+
+@pytest.mark.parametrize("block,bu_words", [(128, 16), (256, 1), (512, 32), (512, 3)])
+@pytest.mark.parametrize("nv", [65536, 100003])
+def test_even_ranges_and_chunks(ctx, orc, nv, block, bu_words):
+    """A top-down step over a bitmap frontier of at least 4096 vertices ranks
+    it in ranges of one chunk per wave, and chunks shrink on graphs smaller
+    than the grid: scripted bottom-up then top-down steps (and claims after a
+    remote write) over frontiers of tens of thousands of vertices."""
+    t0 = ctx.get_tuning()
+    try:
+        ctx.set_tuning(block=block, bu_words=bu_words)
+        ctx.generate_er(nv, 5 * nv, seed=nv)
+        off, adj = ctx.csr()
+        root = int(ctx.pick_roots(1)[0])
+        ref = orc.bfs_depth(off, adj, root)
+        for split in (1 << 30, 1 << 16):
+            ctx.set_tuning(td_split_edges=split)
+            for script in ([0, 0, 0, 0, 1, 0], [0, 0, 0, 1, 0, 1, 0], [1, 0]):
+                ctx.set_script(script)
+                ctx.bfs(root, policy="script")
+                np.testing.assert_array_equal(ctx.fetch()[0], ref)
+                assert ctx.check(root)
+                assert max(r["frontier"] for r in ctx.levels()) >= 4096
+    finally:
+        ctx.set_tuning(**t0)
