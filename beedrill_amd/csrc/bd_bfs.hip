@@ -47,6 +47,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <chrono>
 #include <type_traits>
 #include <vector>
 
@@ -118,7 +119,8 @@ struct step_args {
     int64_t n_hub_med, n_hub_big;
     ctl_block *c;
     seg_counters *seg;
-    bd_level_rec *log;
+    bd_level_rec *log;     // pinned host memory, as is res
+    search_result *res;
     const int32_t *script;
     const float *mlp;
     const uint4 *mlp_ops;  // the network's operands in MFMA lane order
@@ -137,6 +139,7 @@ struct step_args {
     int32_t wave_t, task_t, task_edges;
     int32_t bu_words, bu_cap, bu_head, bu_batch;
     int32_t policy, script_len, log_cap;
+    uint32_t seq;          // the search's number
     int32_t mlp_h1, mlp_h2, has_mlp;
     float mlp_margin;      // log2-cost margin for the network to override Beamer
     int64_t mlp_near;      // also consulted at top-down steps this close to Beamer's switch
@@ -1407,9 +1410,26 @@ __device__ __forceinline__ void publish_state(const step_args &a, step_smem<BLOC
     if (l == 0) {
         g->qlen[(L + 2) % 3][kSeg][0] = 0;
         g->tlen[(L + 2) % 3][kSeg][0] = 0;
-        // the first launch to publish "done" stamps the end (the step
-        // kernel of the other direction republishes the same state)
-        if (done && g->t_end == 0) g->t_end = wall_clock64();
+    }
+    if (done) {
+        // the result, straight into host memory; its number last, once
+        // everything before it has arrived.  (Four copies and their waits
+        // took about 100 us after a search of 130 us at scale 20.)
+        const uint64_t *src = (const uint64_t *)&s.st;
+        uint64_t *dst = (uint64_t *)&a.res->ctl;
+        for (int i = l; i < kCtlWords; i += 64) dst[i] = src[i];
+        if (l == 0) {
+            // the first launch to publish "done" stamps the end (the step
+            // kernel of the other direction republishes the same state)
+            if (g->t_end == 0) g->t_end = wall_clock64();
+            a.res->t_start = g->t_start;
+            a.res->t_end = g->t_end;
+            a.res->task_overflow = g->task_overflow;
+        }
+        __threadfence_system();
+        wave_lds_sync();
+        if (l == 0)
+            __hip_atomic_store(&a.res->seq, a.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
     }
 }
 
@@ -1879,7 +1899,9 @@ step_args make_args(bd_ctx *c, int32_t level, int64_t alpha, int64_t beta, int p
     a.n_hub_big = c->n_hub_big;
     a.c = c->d_ctl;
     a.seg = c->d_seg;
-    a.log = c->d_log;
+    a.log = c->h_log;
+    a.res = c->h_res;
+    a.seq = c->search_seq;
     a.script = c->d_script;
     a.mlp = c->d_mlp;
     a.mlp_ops = c->d_mlp_ops;
@@ -2038,6 +2060,7 @@ int check_run_args(bd_ctx *c, int64_t source, int64_t alpha, int64_t beta, int p
 int start_search(bd_ctx *c, int64_t source, int64_t alpha, int64_t beta, int policy,
                  const int64_t *srcs = nullptr, int64_t nsrc = 1, hipEvent_t init_end = nullptr) {
     const int64_t n = std::max(c->nv, c->nwords);
+    ++c->search_seq;
     const step_args ca = make_args(c, 0, alpha, beta, policy);
     hipLaunchKernelGGL(k_clear, dim3(grid_for(c, n, 256)), dim3(256), 0, c->stream, ca,
                        c->d_parent, c->nv, c->d_sdead, c->d_bm[0], c->d_bm[1], c->d_bm[2],
@@ -2064,30 +2087,38 @@ int read_ctl(bd_ctx *c) {
     return BD_OK;
 }
 
-// The final state: once the search is done both copies hold it.
-const ctl_block *final_ctl(const bd_ctx *c) {
-    return c->h_ctl[0].done ? &c->h_ctl[0] : (c->h_ctl[1].done ? &c->h_ctl[1] : nullptr);
+bool search_done(const bd_ctx *c) {
+    return __atomic_load_n(&c->h_res->seq, __ATOMIC_ACQUIRE) == c->search_seq;
 }
 
-int finish_search(bd_ctx *c, int64_t source, bd_run_stats *out, double event_ms) {
-    const ctl_block *hp = final_ctl(c);
-    if (!hp) return set_err(c, BD_EHIP, "search state not final");
-    const ctl_block &h = *hp;
-    struct {
-        unsigned long long task_overflow;
-        uint64_t t_start, t_end;
-    } tail;
-    BD_HIP(c, hipMemcpy(&tail, &c->d_seg->task_overflow, sizeof(tail), hipMemcpyDeviceToHost));
+// Wait until the search's result is there, or every launch queued so far has
+// ended without it.  The host watches the result's number, which arrives
+// before the launches queued past the search's end have run; they only look
+// at the done flag, and what is queued after them is ordered behind them.
+int wait_search(bd_ctx *c) {
+    for (unsigned n = 1;; ++n) {
+        if (search_done(c)) return BD_OK;
+        if ((n & 255) == 0) {
+            const hipError_t e = hipStreamQuery(c->stream);
+            if (e == hipSuccess) return BD_OK;
+            (void)hipGetLastError();
+            if (e != hipErrorNotReady) return hip_err(c, e, "hipStreamQuery");
+        }
+        __builtin_ia32_pause();
+    }
+}
+
+int finish_search(bd_ctx *c, int64_t source, bd_run_stats *out, double host_ms) {
+    if (!search_done(c)) return set_err(c, BD_EHIP, "search state not final");
+    const search_result &tail = *c->h_res;
+    const ctl_block &h = tail.ctl;
     if (tail.task_overflow) return set_err(c, BD_EHIP, "task list overflow");
     c->last_steps = h.steps;
     c->last_source = source;
     c->have_result = true;
     c->cand_clean = true;  // every write half was followed by its claim sweep
     const int64_t n = std::min<int64_t>(h.steps, c->log_cap);
-    c->last_log.resize(n);
-    if (n)
-        BD_HIP(c, hipMemcpy(c->last_log.data(), c->d_log, sizeof(bd_level_rec) * n,
-                            hipMemcpyDeviceToHost));
+    c->last_log.assign(c->h_log, c->h_log + n);
     if (out) {
         out->source = source;
         out->steps = h.steps;
@@ -2096,7 +2127,7 @@ int finish_search(bd_ctx *c, int64_t source, bd_run_stats *out, double event_ms)
         out->reached = h.reached;
         out->traversed_edges = h.reached_deg / 2;
         const double dev_ms = (double)(tail.t_end - tail.t_start) / (double)c->wall_khz;
-        out->ms = (tail.t_end >= tail.t_start && dev_ms > 0) ? dev_ms : event_ms;
+        out->ms = (tail.t_end >= tail.t_start && dev_ms > 0) ? dev_ms : host_ms;
     }
     return BD_OK;
 }
@@ -2118,7 +2149,7 @@ int run_search(bd_ctx *c, int64_t source, int64_t alpha, int64_t beta, int polic
     if ((rc = start_search(c, source, alpha, beta, policy, srcs, nsrc,
                            per_chunk ? c->ev_pool[0] : nullptr)))
         return rc;
-    BD_HIP(c, hipEventRecord(c->ev[0], c->stream));
+    const auto host_start = std::chrono::steady_clock::now();
     // launches: a level takes one, or two when it writes remotely
     const int64_t max_levels = 2 * c->nv + 4;
     int32_t L = 0;
@@ -2168,7 +2199,8 @@ int run_search(bd_ctx *c, int64_t source, int64_t alpha, int64_t beta, int polic
                 }
                 if ((rc = launch_level(c, a, e0, e1))) return rc;
             }
-            if ((rc = read_ctl(c))) return rc;
+            if ((rc = wait_search(c))) return rc;
+            if (per_launch || per_chunk) BD_HIP(c, hipStreamSynchronize(c->stream));
             for (int k = 0; per_launch && k < chunk; ++k) {
                 float ms = 0;
                 BD_HIP(c, hipEventElapsedTime(&ms, c->ev_pool[2 * k], c->ev_pool[2 * k + 1]));
@@ -2179,17 +2211,15 @@ int run_search(bd_ctx *c, int64_t source, int64_t alpha, int64_t beta, int polic
                 BD_HIP(c, hipEventElapsedTime(&ms, c->ev_pool[0], c->ev_pool[1]));
                 for (int k = 0; k < chunk; ++k) c->last_launch_ms.push_back(ms / chunk);
             }
-            if (final_ctl(c)) break;
+            if (search_done(c)) break;
             if (L > max_levels) return set_err(c, BD_EHIP, "search did not terminate");
             chunk = std::min(chunk * 2, kMaxLevelsPerSync);
         }
     }
-    BD_HIP(c, hipEventRecord(c->ev[1], c->stream));
-    BD_HIP(c, hipEventSynchronize(c->ev[1]));
-    float ev_ms = 0;
-    BD_HIP(c, hipEventElapsedTime(&ev_ms, c->ev[0], c->ev[1]));
-    if ((rc = read_ctl(c))) return rc;
-    if ((rc = finish_search(c, source, out, ev_ms))) return rc;
+    const double host_ms = std::chrono::duration<double, std::milli>(
+                               std::chrono::steady_clock::now() - host_start)
+                               .count();
+    if ((rc = finish_search(c, source, out, host_ms))) return rc;
     if (!c->last_log.empty() && (int64_t)c->last_log.size() == c->last_steps) {
         const bd_level_rec &r = c->last_log.back();
         // its level launches and the launch that found the frontier empty

@@ -220,8 +220,16 @@ extern "C" int bd_create(bd_ctx **out, int device) {
     if (e == hipSuccess) e = hipMalloc((void **)&c->d_ctl, 2 * sizeof(ctl_block));
     if (e == hipSuccess) e = hipMalloc((void **)&c->d_seg, sizeof(seg_counters));
     if (e == hipSuccess) e = hipHostMalloc((void **)&c->h_ctl, 2 * sizeof(ctl_block), hipHostMallocDefault);
+    const unsigned shared = hipHostMallocMapped | hipHostMallocCoherent;
+    if (e == hipSuccess) {
+        e = hipHostMalloc((void **)&c->h_res, sizeof(search_result), shared);
+        if (e == hipSuccess) c->h_res->seq = 0;
+    }
     if (e == hipSuccess) {
         c->log_cap = 1 << 16;
+        e = hipHostMalloc((void **)&c->h_log, sizeof(bd_level_rec) * c->log_cap, shared);
+    }
+    if (e == hipSuccess) {
         e = hipMalloc((void **)&c->d_log, sizeof(bd_level_rec) * c->log_cap);
     }
     if (e != hipSuccess) {
@@ -250,6 +258,8 @@ extern "C" int bd_destroy(bd_ctx *c) {
     dev_free(c->d_mlp_ops);
     dev_free(c->d_mlp_ws);
     if (c->h_ctl) (void)hipHostFree(c->h_ctl);
+    if (c->h_res) (void)hipHostFree(c->h_res);
+    if (c->h_log) (void)hipHostFree(c->h_log);
     for (auto &e : c->ev)
         if (e) (void)hipEventDestroy(e);
     for (auto &e : c->ev_pool)

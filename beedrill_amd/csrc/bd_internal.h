@@ -101,7 +101,16 @@ struct ctl_block {
     int64_t reached_deg;
 };
 
-struct ctx_state;
+// What a search leaves for the host, in pinned memory that the device writes:
+// the launch that finds the search done fills it and sets seq, last, to the
+// search's number, so the host reads the result without a copy or a
+// synchronisation of its own.
+struct search_result {
+    ctl_block ctl;
+    unsigned long long task_overflow;
+    uint64_t t_start, t_end;
+    uint32_t seq;
+};
 
 }  // namespace bd
 
@@ -171,7 +180,10 @@ struct bd_ctx {
     bd::seg_counters *d_seg = nullptr;
     bd::ctl_block *d_ctl = nullptr;  // two published copies (see ctl_block)
     bd::ctl_block *h_ctl = nullptr;  // pinned mirror of both copies
-    bd_level_rec *d_log = nullptr;
+    bd::search_result *h_res = nullptr;  // pinned, written by the device
+    bd_level_rec *h_log = nullptr;       // pinned: step records, written by the device
+    uint32_t search_seq = 0;             // number of the last search started
+    bd_level_rec *d_log = nullptr;       // level records of the bit-parallel search
     int64_t log_cap = 0;
     int32_t *d_script = nullptr;
     int64_t script_len = 0;
