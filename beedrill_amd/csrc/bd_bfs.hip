@@ -201,14 +201,15 @@ struct step_smem {
 // Reserve n slots of the output list for this workgroup's segment; returns
 // how many fit there (at *pos) and where the rest goes in the overflow
 // segment (at *opos).
-__device__ __forceinline__ int64_t seg_reserve(unsigned long long (*len)[kLine], int64_t seg_cap,
-                                               int64_t n, int64_t *pos, int64_t *opos) {
+__device__ __forceinline__ int64_t seg_reserve(seg_line *lines, unsigned long long seg_line::*len,
+                                               int64_t seg_cap, int64_t n, int64_t *pos,
+                                               int64_t *opos) {
     const int sidx = blockIdx.x % kSeg;
-    *pos = (int64_t)atomicAdd(&len[sidx][0], (unsigned long long)n);
+    *pos = (int64_t)atomicAdd(&(lines[sidx].*len), (unsigned long long)n);
     int64_t fit = seg_cap - *pos;
     fit = fit < 0 ? 0 : (fit > n ? n : fit);
     *opos = 0;
-    if (fit < n) *opos = (int64_t)atomicAdd(&len[kSeg][0], (unsigned long long)(n - fit));
+    if (fit < n) *opos = (int64_t)atomicAdd(&(lines[kSeg].*len), (unsigned long long)(n - fit));
     return fit;
 }
 
@@ -229,7 +230,8 @@ __device__ __forceinline__ void emit_tasks(const step_args &a, bool huge, int32_
     long long pos = 0, opos = 0, fit = 0;
     if (lane == 0) {
         int64_t ps, ops;
-        fit = seg_reserve(a.seg->tlen[(a.level + 1) % 3], a.tseg_cap, total, &ps, &ops);
+        fit = seg_reserve(a.seg->line[(a.level + 1) % 3], &seg_line::tlen, a.tseg_cap, total, &ps,
+                          &ops);
         pos = ps;
         opos = ops;
     }
@@ -294,7 +296,8 @@ __device__ __forceinline__ void emit_next(const step_args &a, step_smem<BLOCK> &
     if (in_lds < cnt) {
         if (lane == leader) {
             int64_t ps, ops;
-            fit = seg_reserve(a.seg->qlen[(a.level + 1) % 3], a.qseg_cap, cnt - in_lds, &ps, &ops);
+            fit = seg_reserve(a.seg->line[(a.level + 1) % 3], &seg_line::qlen, a.qseg_cap,
+                              cnt - in_lds, &ps, &ops);
             pos = ps;
             opos = ops;
         }
@@ -324,8 +327,8 @@ __device__ __forceinline__ void flush_queue(const step_args &a, step_smem<BLOCK>
     if (n > 0) {
         if (threadIdx.x == 0) {
             int64_t pos, opos;
-            s.qfit = (int32_t)seg_reserve(a.seg->qlen[(a.level + 1) % 3], a.qseg_cap, n, &pos,
-                                          &opos);
+            s.qfit = (int32_t)seg_reserve(a.seg->line[(a.level + 1) % 3], &seg_line::qlen,
+                                          a.qseg_cap, n, &pos, &opos);
             s.qpos = pos;
             s.qopos = opos;
         }
@@ -1285,15 +1288,15 @@ __device__ __forceinline__ bool rebuild_state(const step_args &a, step_smem<BLOC
     const int l = lane_id();
     seg_counters *g = a.seg;
     const uint64_t *src = (const uint64_t *)&a.c[(L - 1) & 1];
-    const int pa = (L - 1) % 3, pq = L % 3;
+    const seg_line *ln = g->line[L % 3];
     uint64_t cw[3];
 #pragma unroll
     for (int i = 0; i < 3; ++i) cw[i] = l + 64 * i < kCtlWords ? src[l + 64 * i] : 0;
     unsigned long long ac[4];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) ac[k] = g->acc[pa][l][k];
-    const int64_t ql = (int64_t)g->qlen[pq][l][0], qo = (int64_t)g->qlen[pq][kSeg][0];
-    const int64_t tl = (int64_t)g->tlen[pq][l][0], to = (int64_t)g->tlen[pq][kSeg][0];
+    for (int k = 0; k < 4; ++k) ac[k] = ln[l].acc[k];
+    const int64_t ql = (int64_t)ln[l].qlen, qo = (int64_t)ln[kSeg].qlen;
+    const int64_t tl = (int64_t)ln[l].tlen, to = (int64_t)ln[kSeg].tlen;
     {
         uint64_t *dst = (uint64_t *)&s.st;
 #pragma unroll
@@ -1385,10 +1388,21 @@ __device__ __forceinline__ bool rebuild_state(const step_args &a, step_smem<BLOC
     return false;
 }
 
+// Clear one copy of the lines (one wave).
+__device__ __forceinline__ void clear_lines(seg_line *ln, int l) {
+    ln[l].qlen = 0;
+    ln[l].tlen = 0;
+    for (int k = 0; k < 4; ++k) ln[l].acc[k] = 0;
+    if (l == 0) {
+        ln[kSeg].qlen = 0;
+        ln[kSeg].tlen = 0;
+    }
+}
+
 // Workgroup 0, first wave: publish the state before step L as copy L&1 (both
 // copies once the search is done, so later launches see it), and clear the
-// counters the next step fills: acc[(L+1)%3] and the segment lengths
-// [(L+2)%3], neither of which anyone reads or writes during step L.
+// lines the next step fills, [(L+2)%3], which nobody reads or writes during
+// step L.
 template <int BLOCK>
 __device__ __forceinline__ void publish_state(const step_args &a, step_smem<BLOCK> &s) {
     const int L = a.level;
@@ -1404,13 +1418,7 @@ __device__ __forceinline__ void publish_state(const step_args &a, step_smem<BLOC
             if (done) d1[i] = src[i];
         }
     }
-    for (int k = 0; k < 4; ++k) g->acc[(L + 1) % 3][l][k] = 0;
-    g->qlen[(L + 2) % 3][l][0] = 0;
-    g->tlen[(L + 2) % 3][l][0] = 0;
-    if (l == 0) {
-        g->qlen[(L + 2) % 3][kSeg][0] = 0;
-        g->tlen[(L + 2) % 3][kSeg][0] = 0;
-    }
+    clear_lines(g->line[(L + 2) % 3], l);
     if (done) {
         // the result, straight into host memory; its number last, once
         // everything before it has arrived.  (Four copies and their waits
@@ -1460,7 +1468,7 @@ __device__ __forceinline__ void block_flush_counters(const step_args &a, step_sm
             exam += s.red[2][w];
             dmax = s.red[3][w] > dmax ? s.red[3][w] : dmax;
         }
-        unsigned long long *slot = a.seg->acc[a.level % 3][blockIdx.x % kSlots];
+        unsigned long long *slot = a.seg->line[(a.level + 1) % 3][blockIdx.x % kSlots].acc;
         if (cnt) atomicAdd(&slot[0], cnt);
         if (dsum) atomicAdd(&slot[1], dsum);
         if (exam) atomicAdd(&slot[2], exam);
@@ -1537,13 +1545,7 @@ __global__ __launch_bounds__(64) void k_init(step_args a, int64_t source,
     // (hybrid_bfs.cc:157-167, hybrid_bfs_main.cc:267-282)
     if (l == 0) g->t_start = wall_clock64();
     const uint64_t below = (1ULL << l) - 1;
-    for (int w = 0; w < 3; ++w) {
-        for (int i = l; i <= kSeg; i += 64) {
-            g->qlen[w][i][0] = 0;
-            g->tlen[w][i][0] = 0;
-        }
-        for (int k = 0; k < 4; ++k) g->acc[w][l][k] = 0;
-    }
+    for (int w = 0; w < 3; ++w) clear_lines(g->line[w], l);
     // the state is built in LDS and published with one coalesced copy
     ctl_block *c = &s.st;
     for (int i = l; i < kCtlWords; i += 64) ((uint64_t *)&s.st)[i] = 0;
@@ -1686,14 +1688,7 @@ __global__ void k_fill_cand(int32_t *__restrict__ cand, int64_t nv, uint8_t *__r
 // Profiling: undo the first direction's step at level L (its counters and
 // the lengths of the list it filled) before timing the other direction.
 __global__ __launch_bounds__(64) void k_reset_step(seg_counters *g, int32_t level) {
-    const int l = threadIdx.x;
-    for (int k = 0; k < 4; ++k) g->acc[level % 3][l][k] = 0;
-    g->qlen[(level + 1) % 3][l][0] = 0;
-    g->tlen[(level + 1) % 3][l][0] = 0;
-    if (l == 0) {
-        g->qlen[(level + 1) % 3][kSeg][0] = 0;
-        g->tlen[(level + 1) % 3][kSeg][0] = 0;
-    }
+    clear_lines(g->line[(level + 1) % 3], threadIdx.x);
 }
 
 // count_num_traversed_edges (hybrid_bfs.cc:401-414): sum of degrees over
@@ -2519,7 +2514,7 @@ extern "C" int bd_bfs_profile(bd_ctx *c, int64_t source, int64_t alpha, int64_t 
     if ((rc = start_search(c, source, alpha, beta, policy))) return rc;
     if ((rc = read_ctl(c))) return rc;
     std::vector<std::pair<double, double>> times;
-    std::vector<unsigned long long> acc(kSlots * kLine);
+    std::vector<seg_line> lines(kSlots);
     double total = 0;
     for (int32_t L = 0;; ++L) {
         if (L > c->nv + 2) return set_err(c, BD_EHIP, "search did not terminate");
@@ -2549,9 +2544,9 @@ extern "C" int bd_bfs_profile(bd_ctx *c, int64_t source, int64_t alpha, int64_t 
             if ((rc = launch_step(c, a, a.force_dir, 0, c->ev[2], c->ev[3]))) return rc;
             BD_HIP(c, hipEventSynchronize(c->ev[3]));
             BD_HIP(c, hipEventElapsedTime(&ms[pass], c->ev[2], c->ev[3]));
-            BD_HIP(c, hipMemcpy(acc.data(), c->d_seg->acc[L % 3],
-                                sizeof(unsigned long long) * acc.size(), hipMemcpyDeviceToHost));
-            for (int s = 0; s < kSlots; ++s) found[pass] += acc[s * kLine];
+            BD_HIP(c, hipMemcpy(lines.data(), c->d_seg->line[(L + 1) % 3],
+                                sizeof(seg_line) * lines.size(), hipMemcpyDeviceToHost));
+            for (const seg_line &x : lines) found[pass] += x.acc[0];
         }
         if (found[0] != found[1])
             return set_err(c, BD_EHIP, "profile: directions disagree on the next frontier");
