@@ -159,6 +159,14 @@ __device__ __forceinline__ int seg_of(const int64_t *pref, int64_t i) {
     return s;
 }
 
+// The state of a search that predict_costs reads, copied before the closing
+// of the step changes it, and the counters of that step.
+struct step_close {
+    int64_t edges_to_check, old_awake, alpha, unvisited, unvisited_deg, steps;
+    int64_t nnew, nnew_deg, max_deg;
+    int32_t dir, in_bu_loop, done;
+};
+
 // Per-workgroup LDS state.  The top-down staging and tile arrays and the
 // bottom-up found words, pending lists and first hits share one union, sized
 // by the workgroup.
@@ -168,7 +176,8 @@ struct step_smem {
     long long s_new, s_new_deg;
     int s_dir;
     int s_split;  // the step closed was a top-down step with remote writes
-    float x[8];
+    float x[8], y[2];  // the network's inputs and outputs
+    step_close pre;    // what predict_costs starts from
     unsigned long long red[4][BLOCK / 64];
     int32_t qn;
     int64_t qpos, qopos;
@@ -1211,18 +1220,8 @@ __device__ __forceinline__ void choose_dir(const step_args &a, step_smem<BLOCK> 
          (a.mlp_near > 1 && last_dir == BD_DIR_TD && c->dir == BD_DIR_TD &&
           gt_quotient(c->scout, c->edges_to_check + c->scout,
                       c->alpha > (1LL << 46) ? (1LL << 62) : c->alpha * a.mlp_near)))) {
-        // the operands are loaded only here: every workgroup loading the
-        // 6 KB table at every step cost more than a consultation
-        mlp_wave_regs w;
-        mlp_load(a.mlp_ops, w);
-        const int l = lane_id();
-        if (l < kMlpIn)
-            s.x[l] = mlp_feature_k(l, c->frontier, c->frontier_deg, c->max_frontier_deg,
-                                   c->unvisited, c->unvisited_deg, c->level, c->nv, a.m,
-                                   last_dir);
-        wave_lds_sync();
-        float y[2];
-        mlp_eval(w, s.x, y);
+        // evaluated by the second wave meanwhile (predict_costs)
+        const float y[2] = {s.y[0], s.y[1]};
         // y = predicted log2 cost of (top-down, bottom-up).  The network
         // overrides Beamer only when it predicts the other direction cheaper
         // by more than the margin; a NaN prediction keeps Beamer's choice.
@@ -1283,6 +1282,9 @@ static_assert(kCtlWords <= 3 * 64, "ctl_block is copied as three words per lane"
 // before any is used, so the rebuild costs one memory round trip.  Returns
 // true, having changed nothing, when the search ended before this level.
 template <int BLOCK>
+__device__ __forceinline__ void predict_costs(const step_args &a, step_smem<BLOCK> &s);
+
+template <int BLOCK>
 __device__ __forceinline__ bool rebuild_state(const step_args &a, step_smem<BLOCK> &s, bool publish) {
     const int L = a.level;
     const int l = lane_id();
@@ -1304,15 +1306,39 @@ __device__ __forceinline__ bool rebuild_state(const step_args &a, step_smem<BLOC
             if (l + 64 * i < kCtlWords) dst[l + 64 * i] = cw[i];
     }
     wave_lds_sync();
+    const bool learned = a.policy == BD_POLICY_LEARNED && a.has_mlp;
     // the search ended before this level: leave everything as it is (the
     // launch only has to see the flag, which is part of the state it loaded)
-    if (s.st.done) return true;
+    if (s.st.done) {
+        if (learned) {
+            if (l == 0) s.pre.done = 1;
+            __syncthreads();
+        }
+        return true;
+    }
     const unsigned long long nn = wave_sum(ac[0]);
     const unsigned long long nd = wave_sum(ac[1]);
     const unsigned long long ex = wave_sum(ac[2]);
     const unsigned long long mx = wave_max(ac[3]);
     wave_lds_sync();
     ctl_block *c = &s.st;
+    if (learned) {
+        if (l == 0) {
+            s.pre.edges_to_check = c->edges_to_check;
+            s.pre.old_awake = c->old_awake;
+            s.pre.alpha = c->alpha;
+            s.pre.unvisited = c->unvisited;
+            s.pre.unvisited_deg = c->unvisited_deg;
+            s.pre.steps = c->steps;
+            s.pre.nnew = (int64_t)nn;
+            s.pre.nnew_deg = (int64_t)nd;
+            s.pre.max_deg = (int64_t)mx;
+            s.pre.dir = c->dir;
+            s.pre.in_bu_loop = c->in_bu_loop;
+            s.pre.done = 0;
+        }
+        __syncthreads();  // the second wave starts predict_costs
+    }
     if (l == 0) {
         const int32_t dir = c->dir;
         s.s_dir = dir;
@@ -1378,14 +1404,54 @@ __device__ __forceinline__ bool rebuild_state(const step_args &a, step_smem<BLOC
         seg_prefix(ql, qo, a.qseg_cap, a.nv, c->qpref);
         seg_prefix(tl, to, a.tseg_cap, a.task_cap, c->tpref);
         wave_lds_sync();
+    }
+    return false;
+}
+
+// Second half of the rebuild: the direction of the step.
+template <int BLOCK>
+__device__ __forceinline__ void rebuild_dir(const step_args &a, step_smem<BLOCK> &s) {
+    if (s.s_dir != kDirTDWrite) {
         // the remote-write steps of REMOTE_WRITES_HYBRID are its bottom-up
         // phase (hybrid_bfs.cc:262-268)
         const int32_t last = (a.policy == BD_POLICY_REMOTE_WRITES_HYBRID && s.s_split)
                                  ? BD_DIR_BU
                                  : s.s_dir;
-        if (s.s_new > 0) choose_dir(a, s, c, last, s.s_new, s.s_new_deg);
+        if (s.s_new > 0) choose_dir(a, s, &s.st, last, s.s_new, s.s_new_deg);
     }
-    return false;
+}
+
+// LEARNED: the network's prediction for the step, on the workgroup's second
+// wave while the first closes the step before.  From the same inputs it
+// derives what the closing will find, and evaluates the network only when
+// choose_dir may consult it: after a top-down step within the factor mlp_near
+// of the switch, or a bottom-up step that Beamer's rules may leave.  The
+// operands (6 KB a workgroup) are loaded only then.
+template <int BLOCK>
+__device__ __forceinline__ void predict_costs(const step_args &a, step_smem<BLOCK> &s) {
+    const step_close &p = s.pre;
+    const int l = lane_id();
+    const int64_t nn = p.nnew, nd = p.nnew_deg;
+    if (p.done || p.dir == kDirTDWrite || nn == 0) return;
+    const int32_t last = step_dir(p.dir);
+    const bool maybe =
+        last == BD_DIR_TD
+            ? gt_quotient(nd, p.edges_to_check,
+                          p.alpha > (1LL << 46) ? (1LL << 62) : p.alpha * a.mlp_near)
+            : !p.in_bu_loop || (nn < p.old_awake && nn <= a.nv_beta);
+    if (!maybe) return;
+    mlp_wave_regs w;
+    mlp_load(a.mlp_ops, w);
+    const float x = mlp_feature_lane(l, nn, nd, p.max_deg, p.unvisited - nn, p.unvisited_deg - nd,
+                                     (int32_t)(p.steps + 1), a.nv, a.m, last);
+    if (l < kMlpIn) s.x[l] = x;
+    wave_lds_sync();
+    float y[2];
+    mlp_eval(w, s.x, y);
+    if (l == 0) {
+        s.y[0] = y[0];
+        s.y[1] = y[1];
+    }
 }
 
 // Clear one copy of the lines (one wave).
@@ -1490,6 +1556,7 @@ template <int BLOCK, int DIRS>
 __global__ __launch_bounds__(BLOCK) void k_step(step_args a) {
     const int L = a.level;
     __shared__ step_smem<BLOCK> s;
+    const bool learned = a.policy == BD_POLICY_LEARNED && a.has_mlp;
     if (threadIdx.x < 64) {
         if (L == 0) {
             const uint64_t *src = (const uint64_t *)&a.c[0];
@@ -1499,8 +1566,16 @@ __global__ __launch_bounds__(BLOCK) void k_step(step_args a) {
             // one round trip: the previous state (done flag included) and the
             // counters are loaded together; a finished search stops there
             const bool was_done = rebuild_state(a, s, blockIdx.x == 0);
-            if (blockIdx.x == 0 && !was_done) publish_state(a, s);
+            if (learned) __syncthreads();  // the prediction is there
+            if (!was_done) {
+                rebuild_dir(a, s);
+                if (blockIdx.x == 0) publish_state(a, s);
+            }
         }
+    } else if (learned && L > 0) {
+        __syncthreads();  // the state and counters of the step before are there
+        if (threadIdx.x < 128) predict_costs(a, s);
+        __syncthreads();
     }
     if (threadIdx.x == 0) s.qn = 0;
     __syncthreads();

@@ -42,25 +42,42 @@ __host__ __device__ inline void mlp_features_dev(int64_t frontier, int64_t front
     x[7] = prev_dir == 1 ? 1.0f : 0.0f;
 }
 
-// Feature `k` (0..7) of mlp_features_dev alone, so that lanes 0-7 of a wave
-// compute the eight features side by side; the same arithmetic, in the same
-// order, as mlp_features_dev.
-__device__ inline float mlp_feature_k(int k, int64_t frontier, int64_t frontier_deg,
-                                      int64_t max_frontier_deg, int64_t unvisited,
-                                      int64_t unvisited_deg, int64_t level, int64_t nv, int64_t m,
-                                      int64_t prev_dir) {
-    const float lv = lg1p((float)nv);
-    const float le = lg1p(2.0f * (float)m);
-    switch (k) {
-    case 0: return lg1p((float)frontier) / lv;
-    case 1: return lg1p((float)frontier_deg) / le;
-    case 2: return lg1p((float)unvisited) / lv;
-    case 3: return lg1p((float)unvisited_deg) / le;
-    case 4: return (float)(level < 64 ? level : 64) / 64.0f;
-    case 5: return lg1p((float)max_frontier_deg) / lv;
-    case 6: return lg1p(2.0f * (float)m / (float)(nv > 0 ? nv : 1)) / 8.0f;
-    default: return prev_dir == 1 ? 1.0f : 0.0f;
+__device__ __forceinline__ float lane_f32(float v, int lane) {
+    return __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(v), lane));
+}
+
+// Feature l of mlp_features_dev in lanes l = 0..7 of a wave, the same
+// arithmetic: the arguments of all the logarithms (lanes 8 and 9 take the two
+// in the denominators) are chosen first, so that one logarithm and one
+// division serve every lane.  A switch over the features ran its eight cases
+// one after another, on the critical path of a step.
+__device__ inline float mlp_feature_lane(int l, int64_t frontier, int64_t frontier_deg,
+                                         int64_t max_frontier_deg, int64_t unvisited,
+                                         int64_t unvisited_deg, int64_t level, int64_t nv,
+                                         int64_t m, int64_t prev_dir) {
+    const int64_t n = l == 0   ? frontier
+                      : l == 1 ? frontier_deg
+                      : l == 2 ? unvisited
+                      : l == 3 ? unvisited_deg
+                      : l == 5 ? max_frontier_deg
+                      : l == 8 ? nv
+                               : m;
+    float arg = (float)n;
+    if (l == 6 || l == 9) arg = 2.0f * arg;
+    if (l == 6) arg = arg / (float)(nv > 0 ? nv : 1);
+    const float lg = lg1p(arg);
+    const float lv = lane_f32(lg, 8), le = lane_f32(lg, 9);
+    float num = lg, den = l == 1 || l == 3 ? le : lv;
+    if (l == 6) den = 8.0f;
+    if (l == 4) {
+        num = (float)(level < 64 ? level : 64);
+        den = 64.0f;
     }
+    if (l == 7) {
+        num = prev_dir == 1 ? 1.0f : 0.0f;
+        den = 1.0f;
+    }
+    return num / den;
 }
 
 // Orders LDS accesses among the lanes of one wave.  The network code below
@@ -180,18 +197,26 @@ __device__ inline void mlp_prefetch(const float *p, int h1, int h2, mlp_wave_reg
 // one wave, from prefetched weights.  Row 0 of each 16-row tile carries the
 // sample.  The result tile holds row 0 in lanes 0..15 (column = lane), so a
 // layer's activations reach the next layer's A operand (row 0, k = 4 (l/16)
-// + j of tile kt) by a shuffle from lane 4 (l/16) + j.  Same rounding as
+// + j of tile kt) by a shuffle from lane 4 (l/16) + j; every row gets it,
+// and the rows past row 0 are not read.  Same rounding as
 // mlp_forward_rows_mfma: bf16 operands, fp32 sums, bias and ReLU in fp32.
 // Every lane returns y.
+__device__ __forceinline__ bf16x4 bf16x4_of(float v0, float v1, float v2, float v3) {
+    // the hardware's conversion, round to nearest even as f32_to_bf16
+    typedef __bf16 hbf16x4 __attribute__((ext_vector_type(4)));
+    union {
+        hbf16x4 h;
+        bf16x4 s;
+    } u;
+    u.h = hbf16x4{(__bf16)v0, (__bf16)v1, (__bf16)v2, (__bf16)v3};
+    return u.s;
+}
+
 __device__ inline void mlp_eval(const mlp_wave_regs &w, const float *x, float *y) {
     const int l = threadIdx.x & 63, r = l & 15, q = l >> 4;
-    bf16x4 a;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const int kk = 4 * q + j;
-        a[j] = f32_to_bf16((r == 0 && kk < kMlpIn) ? x[kk] : 0.f);
-    }
     const f32x4 z = {0.f, 0.f, 0.f, 0.f};
+    bf16x4 a = bf16x4{0, 0, 0, 0};
+    if (r == 0 && q < 2) a = bf16x4_of(x[4 * q], x[4 * q + 1], x[4 * q + 2], x[4 * q + 3]);
     float h[2];
 #pragma unroll
     for (int nt = 0; nt < 2; ++nt) {
@@ -199,14 +224,15 @@ __device__ inline void mlp_eval(const mlp_wave_regs &w, const float *x, float *y
         const float v = d[0] + w.b1[nt];
         h[nt] = v > 0.f ? v : 0.f;
     }
+    // row 0 of the next A operand; the other rows' results are not used
+    auto carry = [&](bf16x4 (&a2)[2]) {
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt)
+            a2[kt] = bf16x4_of(__shfl(h[kt], 4 * q), __shfl(h[kt], 4 * q + 1),
+                               __shfl(h[kt], 4 * q + 2), __shfl(h[kt], 4 * q + 3));
+    };
     bf16x4 a2[2];
-#pragma unroll
-    for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const float v = __shfl(h[kt], 4 * q + j);
-            a2[kt][j] = f32_to_bf16(r == 0 ? v : 0.f);
-        }
+    carry(a2);
 #pragma unroll
     for (int nt = 0; nt < 2; ++nt) {
         f32x4 d = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a2[0], w.w2[nt][0], z, 0, 0, 0);
@@ -214,18 +240,12 @@ __device__ inline void mlp_eval(const mlp_wave_regs &w, const float *x, float *y
         const float v = d[0] + w.b2[nt];
         h[nt] = v > 0.f ? v : 0.f;
     }
-#pragma unroll
-    for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const float v = __shfl(h[kt], 4 * q + j);
-            a2[kt][j] = f32_to_bf16(r == 0 ? v : 0.f);
-        }
+    carry(a2);
     f32x4 d = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a2[0], w.w3[0], z, 0, 0, 0);
     d = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a2[1], w.w3[1], d, 0, 0, 0);
     const float out = d[0] + w.b3;
-    y[0] = __shfl(out, 0);
-    y[1] = __shfl(out, 1);
+    y[0] = lane_f32(out, 0);
+    y[1] = lane_f32(out, 1);
 }
 
 // The prefetched weights as a table in device memory, 96 bytes per lane,
