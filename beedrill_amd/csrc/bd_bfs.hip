@@ -1779,35 +1779,63 @@ __global__ void k_count_traversed(const int32_t *__restrict__ parent,
     if ((threadIdx.x & 63) == 0 && s) atomicAdd(&out[(blockIdx.x % kSlots) * kLine], s);
 }
 
-// A search's result in graph ids: vertex v is search id inv[v], and a parent
-// p (a search id) is graph vertex perm[p].  Either output may be null.
-__global__ void k_to_graph_ids(const int32_t *__restrict__ inv, const int32_t *__restrict__ perm,
-                               const int32_t *__restrict__ sparent,
-                               const int32_t *__restrict__ sdepth, int64_t nv,
-                               int32_t *__restrict__ parent, int32_t *__restrict__ depth) {
-    for (int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; v < nv;
-         v += (int64_t)gridDim.x * blockDim.x) {
-        const int32_t i = inv[v];
-        if (parent) {
-            const int32_t p = sparent[i];
-            parent[v] = p < 0 ? -1 : perm[p];
-        }
-        if (depth) depth[v] = sdepth[i];
-    }
-}
-
 // Depths from the parent tree.  The steps write parents only, as
 // hybrid_bfs::run_beamer does; a vertex's depth is its distance to the
 // source its parent chain ends at (a source is its own parent).
-// t[v] = (k << 32) | x names an ancestor x of v, k levels up, starting from
-// the parent (k = 1, or k = 0 for a source).  Each round of pointer jumping
-// replaces (x, k) by (y, k + j) where t[x] = (j << 32) | y, until every x is
-// a source.  Entries are single 8-byte words, read and written whole, so a
-// jump that reads a word another thread has already advanced in this round
-// still gets an ancestor and its distance; such reads only shorten the
-// rounds, which are no more than with separate buffers (log2 of the depth).
-// err[1] is set when a parent is itself unreached, err[2] when a chain
-// closes on a vertex that is not a source.
+//
+// A search's result in graph ids: vertex v is search id inv[v], and a parent
+// p (a search id) is graph vertex perm[p] (no inv: ids are as they are).
+// Either output may be null.  Depths come from sdepth, or, when that is null,
+// from walking the chain: a search of few levels has short chains whose upper
+// ends are shared and cached, and one launch replaces the rounds of pointer
+// jumping, their host waits and the mapping (scale 16: 12 launches and copies,
+// 190 us a fetch).  flags (host memory, written only on a fault): [0] a chain
+// longer than limit, [1] an unreached or out-of-range ancestor.
+template <typename P>
+__global__ void k_result(const int32_t *__restrict__ inv, const int32_t *__restrict__ perm,
+                         const int32_t *__restrict__ sparent, const int32_t *__restrict__ sdepth,
+                         int64_t nv, int64_t limit, P *__restrict__ parent,
+                         int32_t *__restrict__ depth, int32_t *__restrict__ flags) {
+    for (int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; v < nv;
+         v += (int64_t)gridDim.x * blockDim.x) {
+        const int32_t i = inv ? inv[v] : (int32_t)v;
+        const int32_t p = sparent[i];
+        if (parent) parent[v] = p < 0 ? -1 : (P)(perm ? perm[p] : p);
+        if (!depth) continue;
+        if (sdepth) {
+            depth[v] = sdepth[i];
+            continue;
+        }
+        int32_t d = -1;
+        if (p >= 0) {
+            d = 0;
+            for (int32_t x = i, y = p; y != x;) {
+                const int32_t z = (int64_t)y < nv ? sparent[y] : -1;
+                if (z < 0) {
+                    flags[1] = 1;
+                    break;
+                }
+                if (++d > limit) {
+                    flags[0] = 1;
+                    break;
+                }
+                x = y;
+                y = z;
+            }
+        }
+        depth[v] = d;
+    }
+}
+
+// Deep trees: t[v] = (k << 32) | x names an ancestor x of v, k levels up,
+// starting from the parent (k = 1, or k = 0 for a source).  Each round of
+// pointer jumping replaces (x, k) by (y, k + j) where t[x] = (j << 32) | y,
+// until every x is a source.  Entries are single 8-byte words, read and
+// written whole, so a jump that reads a word another thread has already
+// advanced in this round still gets an ancestor and its distance; such reads
+// only shorten the rounds, which are no more than with separate buffers (log2
+// of the depth).  flags[1] is set when a parent is itself unreached, flags[0]
+// when a chain has not ended at a source after the rounds.
 constexpr uint64_t kNoTree = ~0ULL;
 
 __global__ void k_tree_init(const int32_t *__restrict__ parent, uint64_t *__restrict__ t,
@@ -1819,30 +1847,31 @@ __global__ void k_tree_init(const int32_t *__restrict__ parent, uint64_t *__rest
     }
 }
 
-__global__ void k_tree_jump(uint64_t *t, int64_t nv, int32_t *__restrict__ err) {
+__global__ void k_tree_jump(uint64_t *t, int64_t nv, int32_t *__restrict__ flags,
+                            int32_t *__restrict__ moved) {
     for (int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; v < nv;
          v += (int64_t)gridDim.x * blockDim.x) {
         const uint64_t x = __hip_atomic_load(t + v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         if (x == kNoTree) continue;
         const uint32_t a = (uint32_t)x;
         if ((int64_t)a >= nv) {
-            err[1] = 1;
+            flags[1] = 1;
             continue;
         }
         const uint64_t y = __hip_atomic_load(t + a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         if (y == kNoTree) {
-            err[1] = 1;
+            flags[1] = 1;
             continue;
         }
         if ((uint32_t)y == a) continue;  // a is a source (or closes a cycle)
         __hip_atomic_store(t + v, (((x >> 32) + (y >> 32)) << 32) | (uint32_t)y, __ATOMIC_RELAXED,
                            __HIP_MEMORY_SCOPE_WORKGROUP);
-        err[0] = 1;  // a jump was made: another round
+        if (moved) *moved = 1;  // a jump was made: another round
     }
 }
 
 __global__ void k_tree_depth(const uint64_t *__restrict__ t, int32_t *__restrict__ depth,
-                             int64_t nv, int32_t *__restrict__ err) {
+                             int64_t nv, int32_t *__restrict__ flags) {
     for (int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; v < nv;
          v += (int64_t)gridDim.x * blockDim.x) {
         const uint64_t x = t[v];
@@ -1850,7 +1879,8 @@ __global__ void k_tree_depth(const uint64_t *__restrict__ t, int32_t *__restrict
             depth[v] = -1;
             continue;
         }
-        if (t[(uint32_t)x] != (uint64_t)(uint32_t)x) err[2] = 1;  // ends at a non-source
+        const uint32_t a = (uint32_t)x;
+        if ((int64_t)a >= nv || t[a] != (uint64_t)a) flags[0] = 1;  // ends at a non-source
         depth[v] = (int32_t)(x >> 32);
     }
 }
@@ -1870,64 +1900,85 @@ __global__ void k_tree_depth(const uint64_t *__restrict__ t, int32_t *__restrict
 // distance.  Conversely a tree the reference accepts has BFS depths, which
 // pass every test.  err[0]: a parent is not a neighbour, err[1]: an edge
 // spans two levels or leaves the reached set, err[2]: a second root, or the
-// source unreached or not its own parent.  One wave per 64 vertices; lists
-// of 64 or more are scanned by the whole wave.
-__global__ __launch_bounds__(256) void k_check_tree(const int64_t *__restrict__ off,
-                                                    const int32_t *__restrict__ cols,
-                                                    const int32_t *__restrict__ parent,
-                                                    const int32_t *__restrict__ depth, int64_t nv,
-                                                    int64_t source, int32_t *__restrict__ err) {
-    const int lane = threadIdx.x & 63;
-    const int64_t wave = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-    const int64_t nwaves = ((int64_t)gridDim.x * blockDim.x) >> 6;
-    for (int64_t base = wave * 64; base < nv; base += nwaves * 64) {
-        const int64_t v = base + lane;
-        const bool valid = v < nv;
-        const int32_t d = valid ? depth[v] : -1;
-        const int32_t p = valid ? parent[v] : -1;
-        bool bad_root = false, bad_par = false, bad_edge = false;
-        if (valid && v == source && (d != 0 || p != (int32_t)v)) bad_root = true;
+// source unreached or not its own parent (host memory, written on a fault).
+// Each wave takes a range of `chunk` entries (walk_range).  A list that lies
+// across ranges is known to all of them as range b / chunk + 1, the first that
+// starts inside it, where marks[] gathers whether its parent was found;
+// k_check_roots looks at those, and at each vertex's own entries.  Bound by
+// the random reads of the neighbours' depths.
+__global__ __launch_bounds__(256) void k_check_edges(const int64_t *__restrict__ off,
+                                                     const int32_t *__restrict__ cols,
+                                                     const int32_t *__restrict__ parent,
+                                                     const int32_t *__restrict__ depth, int64_t nv,
+                                                     int64_t nnz, int64_t chunk, int64_t source,
+                                                     uint8_t *__restrict__ marks,
+                                                     int32_t *__restrict__ err) {
+    __shared__ uint8_t s_found[4][64];
+    const int lane = lane_id();
+    uint8_t *found = s_found[threadIdx.x >> 6];
+    const int64_t c0 = (((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6) * chunk;
+    if (c0 >= nnz) return;
+    const int64_t end = c0 + chunk < nnz ? c0 + chunk : nnz;
+    bool bad_par = false, bad_edge = false;
+    int32_t d = -1, p = -1;
+    walk_range(
+        off, nv, nnz, c0, end,
+        [&](int64_t v, int64_t, int64_t) {
+            d = v < nv ? depth[v] : -1;
+            p = v < nv ? parent[v] : -1;
+            found[lane] = 0;
+            wave_lds_sync();
+        },
+        [&](const int (&o)[kRangeRounds], const int64_t (&q)[kRangeRounds],
+            const bool (&live)[kRangeRounds]) {
+            int32_t u[kRangeRounds], du[kRangeRounds];
+#pragma unroll
+            for (int j = 0; j < kRangeRounds; ++j) u[j] = __builtin_nontemporal_load(cols + q[j]);
+#pragma unroll
+            for (int j = 0; j < kRangeRounds; ++j) du[j] = depth[u[j]];
+#pragma unroll
+            for (int j = 0; j < kRangeRounds; ++j) {
+                const int32_t dv = __shfl(d, o[j]), pv = __shfl(p, o[j]);
+                if (!live[j] || dv < 0) continue;
+                if (u[j] == pv) found[o[j]] = 1;
+                if (du[j] < 0 || du[j] > dv + 1 || du[j] < dv - 1) bad_edge = true;
+            }
+        },
+        [&](int64_t v, int64_t b, int64_t e) {
+            wave_lds_sync();
+            if (d >= 0 && e > b && v != source) {
+                if (b >= c0 && e <= end)
+                    bad_par |= !found[lane];
+                else if (found[lane])
+                    marks[b / chunk + 1] = 1;
+            }
+            wave_lds_sync();
+        });
+    if (__ballot(bad_par) && lane == 0) err[0] = 1;
+    if (__ballot(bad_edge) && lane == 0) err[1] = 1;
+}
+
+__global__ __launch_bounds__(256) void k_check_roots(const int64_t *__restrict__ off,
+                                                     const int32_t *__restrict__ parent,
+                                                     const int32_t *__restrict__ depth, int64_t nv,
+                                                     int64_t chunk, int64_t source,
+                                                     const uint8_t *__restrict__ marks,
+                                                     int32_t *__restrict__ err) {
+    bool bad_root = false, bad_par = false;
+    for (int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; v < nv;
+         v += (int64_t)gridDim.x * blockDim.x) {
+        const int32_t d = depth[v], p = parent[v];
+        if (v == source && (d != 0 || p != (int32_t)v)) bad_root = true;
         if (d >= 0 && p == (int32_t)v && v != source) bad_root = true;
-        int64_t b = 0, e = 0;
-        const bool scan = d >= 0;
-        if (scan) {
-            b = off[v];
-            e = off[v + 1];
-        }
-        const bool alone = scan && e - b < 64;
-        bool found = !scan || v == source;
-        if (alone) {
-            for (int64_t k = b; k < e; ++k) {
-                const int32_t u = cols[k];
-                const int32_t du = depth[u];
-                found |= u == p;
-                if (du < 0 || du > d + 1 || du < d - 1) bad_edge = true;
-            }
-        }
-        uint64_t lm = __ballot(scan && !alone);
-        while (lm) {
-            const int src = __ffsll((unsigned long long)lm) - 1;
-            lm &= lm - 1;
-            const int64_t kb = lane_bcast(b, src), ke = lane_bcast(e, src);
-            const int32_t ds = lane_bcast(d, src), ps = lane_bcast(p, src);
-            bool f = false, be = false;
-            for (int64_t k = kb + lane; k < ke; k += 64) {
-                const int32_t u = cols[k];
-                const int32_t du = depth[u];
-                f |= u == ps;
-                if (du < 0 || du > ds + 1 || du < ds - 1) be = true;
-            }
-            const bool fw = __ballot(f) != 0, bw = __ballot(be) != 0;
-            if (lane == src) {
-                found |= fw;
-                bad_edge |= bw;
-            }
-        }
-        bad_par = scan && !found;
-        if (__ballot(bad_par) && lane == 0) err[0] = 1;
-        if (__ballot(bad_edge) && lane == 0) err[1] = 1;
-        if (__ballot(bad_root) && lane == 0) err[2] = 1;
+        if (d < 0 || v == source) continue;
+        const int64_t b = off[v], e = off[v + 1];
+        if (e == b)
+            bad_par = true;  // reached, with no neighbour to be reached from
+        else if (const int64_t r = b / chunk + 1; r * chunk < e)
+            bad_par |= !marks[r];
     }
+    if (__ballot(bad_root) && lane_id() == 0) err[2] = 1;
+    if (__ballot(bad_par) && lane_id() == 0) err[0] = 1;
 }
 
 // Streams a buffer larger than the last-level cache so a timed step starts
@@ -2330,114 +2381,120 @@ extern "C" int bd_bfs_set_script(bd_ctx *c, const int32_t *dirs, int64_t n) {
     return BD_OK;
 }
 
-// Depths of the parent tree `parent` (nv entries, -1 unreached) into
-// `depth` (k_tree_*).  *why is null when the tree is well formed, else the
-// reason it is not: a reached vertex with an unreached or out-of-range
-// parent, a chain that never ends (a cycle), or one that ends at a vertex
-// that is not its own parent.  Returns a status only for runtime errors.
-int tree_depths(bd_ctx *c, const int32_t *parent, int32_t *depth, const char **why) {
-    *why = nullptr;
+// Readout results: parents (and depths) in graph ids, d_out's halves.
+struct readout {
+    int64_t *parent;
+    int32_t *depth;
+};
+
+int out_buffers(bd_ctx *c, readout *r) {
+    if (!c->d_out) {
+        int rc = dev_alloc(c, (void **)&c->d_out, (sizeof(int64_t) + sizeof(int32_t)) * c->nv,
+                           "results in graph ids");
+        if (rc) return rc;
+    }
+    r->parent = c->d_out;
+    r->depth = (int32_t *)(c->d_out + c->nv);
+    return BD_OK;
+}
+
+// Wait for the stream and read the readout kernels' faults.  *why is null
+// when the tree is well formed.
+int read_flags(bd_ctx *c, const char **why) {
+    BD_HIP(c, hipStreamSynchronize(c->stream));
+    *why = c->h_flags[1]   ? "parent tree: a reached vertex has an unreached parent"
+           : c->h_flags[0] ? "parent tree: chains do not end at a source"
+                           : nullptr;
+    return BD_OK;
+}
+
+void clear_flags(bd_ctx *c) {
+    for (int i = 0; i < 4; ++i) c->h_flags[i] = 0;
+}
+
+// Searches of at most this many levels have their depths read by walking the
+// parent chains (k_result), deeper ones by pointer jumping, whose rounds grow
+// with the logarithm of the depth.
+constexpr int64_t kWalkLevels = 24;
+
+// Depths of the tree `parent` (nv entries, -1 unreached) into `depth` by
+// pointer jumping, from trees of any depth up to max_depth (0: unknown, for a
+// caller's tree; then batches of rounds run until none moves).  Faults go to
+// h_flags.
+int tree_depths(bd_ctx *c, const int32_t *parent, int32_t *depth, int64_t max_depth) {
     const int64_t nv = c->nv;
-    uint64_t *t = nullptr;
-    // nv tree words, then err[4]
-    int rc = dev_alloc(c, (void **)&t, sizeof(uint64_t) * (nv + 2), "parent tree");
-    if (rc) return rc;
-    struct guard {
-        uint64_t *p;
-        ~guard() { dev_free(p); }
-    } g{t};
-    int32_t *err = (int32_t *)(t + nv);
+    int rc;
+    // nv tree words, then the moved flag
+    if (!c->d_tree &&
+        (rc = dev_alloc(c, (void **)&c->d_tree, sizeof(uint64_t) * (nv + 1), "parent tree")))
+        return rc;
+    uint64_t *t = c->d_tree;
+    int32_t *moved = (int32_t *)(t + nv);
     const dim3 grid(grid_for(c, nv, 256)), block(256);
     hipLaunchKernelGGL(k_tree_init, grid, block, 0, c->stream, parent, t, nv);
-    BD_HIP(c, hipGetLastError());
-    int32_t h[4] = {1, 0, 0, 0};
-    // a chain of length D takes ceil(log2 D) + 1 rounds; ids are 31 bits
-    for (int r = 0; r < 40 && h[0]; ++r) {
-        BD_HIP(c, hipMemsetAsync(err, 0, sizeof(h), c->stream));
-        hipLaunchKernelGGL(k_tree_jump, grid, block, 0, c->stream, t, nv, err);
-        BD_HIP(c, hipGetLastError());
-        BD_HIP(c, hipMemcpyAsync(h, err, sizeof(h), hipMemcpyDeviceToHost, c->stream));
-        BD_HIP(c, hipStreamSynchronize(c->stream));
-        if (h[1]) {
-            *why = "parent tree: a reached vertex has an unreached parent";
-            return BD_OK;
+    if (max_depth > 0) {
+        // a chain of length D takes ceil(log2 D) rounds
+        for (int64_t d = 1; d < max_depth; d *= 2)
+            hipLaunchKernelGGL(k_tree_jump, grid, block, 0, c->stream, t, nv, c->h_flags, nullptr);
+    } else {
+        int32_t h = 1;
+        // ids are 31 bits: chains that end do so within 32 rounds
+        for (int r = 0; r < 36 && h && !c->h_flags[1]; r += 6) {
+            for (int k = 0; k < 5; ++k)
+                hipLaunchKernelGGL(k_tree_jump, grid, block, 0, c->stream, t, nv, c->h_flags,
+                                   nullptr);
+            BD_HIP(c, hipMemsetAsync(moved, 0, sizeof(int32_t), c->stream));
+            hipLaunchKernelGGL(k_tree_jump, grid, block, 0, c->stream, t, nv, c->h_flags, moved);
+            BD_HIP(c, hipGetLastError());
+            BD_HIP(c, hipMemcpyAsync(&h, moved, sizeof(h), hipMemcpyDeviceToHost, c->stream));
+            BD_HIP(c, hipStreamSynchronize(c->stream));
         }
     }
-    if (h[0]) {
-        *why = "parent tree: chains do not end";
-        return BD_OK;
-    }
-    hipLaunchKernelGGL(k_tree_depth, grid, block, 0, c->stream, t, depth, nv, err);
+    hipLaunchKernelGGL(k_tree_depth, grid, block, 0, c->stream, t, depth, nv, c->h_flags);
     BD_HIP(c, hipGetLastError());
-    BD_HIP(c, hipMemcpyAsync(h, err, sizeof(h), hipMemcpyDeviceToHost, c->stream));
-    BD_HIP(c, hipStreamSynchronize(c->stream));
-    if (h[2]) *why = "parent tree: a chain closes on a non-source";
     return BD_OK;
 }
 
-// Depths of the last search into d_depth, from its parent tree.
-int derive_depth(bd_ctx *c) {
-    if (c->depth_valid) return BD_OK;
-    const char *why = nullptr;
-    int rc = tree_depths(c, c->d_parent, c->d_depth, &why);
-    if (rc) return rc;
-    if (why) return set_err(c, BD_EHIP, why);
-    c->depth_valid = true;
-    return BD_OK;
-}
-
-// check() of the parent tree `parent` from `source` on the device; `depth`
-// holds its depths when have_depth, else receives them (scratch of nv
-// entries when the tree is not the last search's).  *ok = 1 PASS, 0 FAIL.
-int check_tree(bd_ctx *c, const int32_t *parent, int32_t *depth, bool have_depth,
-               int64_t source, int *ok) {
+// Queue the last search's result in graph ids: parents as P (int64 for a
+// caller, int32 for check()) and depths; either may be null.  Faults in the
+// tree go to h_flags.
+template <typename P>
+int queue_result(bd_ctx *c, P *parent, int32_t *depth) {
     int rc;
-    if (!have_depth) {
-        const char *why = nullptr;
-        if ((rc = tree_depths(c, parent, depth, &why))) return rc;
-        if (why) {
-            *ok = 0;
-            return BD_OK;
-        }
+    const bool deep = depth && c->last_steps > kWalkLevels;
+    if (deep && !c->depth_valid) {
+        if (!c->d_depth &&
+            (rc = dev_alloc(c, (void **)&c->d_depth, sizeof(int32_t) * c->nv, "depth")))
+            return rc;
+        if ((rc = tree_depths(c, c->d_parent, c->d_depth, c->last_steps + 1))) return rc;
     }
-    int32_t *err = nullptr;
-    if ((rc = dev_alloc(c, (void **)&err, sizeof(int32_t) * 4, "check flags"))) return rc;
-    struct guard {
-        int32_t *p;
-        ~guard() { dev_free(p); }
-    } g{err};
-    int32_t h[4] = {0, 0, 0, 0};
-    BD_HIP(c, hipMemsetAsync(err, 0, sizeof(h), c->stream));
-    hipLaunchKernelGGL(k_check_tree, dim3(grid_for(c, c->nv, 256)), dim3(256), 0, c->stream,
-                       c->d_off, c->d_cols, parent, depth, c->nv, source, err);
+    hipLaunchKernelGGL(k_result<P>, dim3(grid_for(c, c->nv, 256)), dim3(256), 0, c->stream,
+                       (const int32_t *)c->d_inv, (const int32_t *)c->d_perm,
+                       (const int32_t *)c->d_parent, (const int32_t *)(deep ? c->d_depth : nullptr),
+                       c->nv, c->last_steps + 1, parent, depth, c->h_flags);
     BD_HIP(c, hipGetLastError());
-    BD_HIP(c, hipMemcpyAsync(h, err, sizeof(h), hipMemcpyDeviceToHost, c->stream));
-    BD_HIP(c, hipStreamSynchronize(c->stream));
-    *ok = (h[0] | h[1] | h[2]) ? 0 : 1;
     return BD_OK;
 }
 
-// The last search's parents (and, with want_depth, depths) in graph ids on
-// the device: the search's own arrays when it ran on graph ids, else mapped
-// into `buf` (allocated here, 2 nv entries; the caller frees it).
-int graph_id_result(bd_ctx *c, bool want_depth, int32_t **buf, const int32_t **parent,
-                    const int32_t **depth) {
+// check() of a tree in graph ids whose parents and depths are on the device
+// (or being written on the stream), against the resident graph.  *ok = 1 PASS,
+// 0 FAIL; a fault already in h_flags is a FAIL.
+int check_tree(bd_ctx *c, const int32_t *parent, const int32_t *depth, int64_t source, int *ok) {
     int rc;
-    *buf = nullptr;
-    if (want_depth && (rc = derive_depth(c))) return rc;
-    if (!c->d_perm) {
-        *parent = c->d_parent;
-        *depth = c->d_depth;
-        return BD_OK;
-    }
-    if ((rc = dev_alloc(c, (void **)buf, sizeof(int32_t) * 2 * c->nv, "results in graph ids")))
-        return rc;
-    hipLaunchKernelGGL(k_to_graph_ids, dim3(grid_for(c, c->nv, 256)), dim3(256), 0, c->stream,
-                       c->d_inv, c->d_perm, c->d_parent, c->d_depth, c->nv, *buf,
-                       want_depth ? *buf + c->nv : nullptr);
+    const int64_t chunk = range_entries(c);
+    const int64_t n = (c->nnz + chunk - 1) / chunk;
+    if (!c->d_marks && (rc = dev_alloc(c, (void **)&c->d_marks, n + 2, "check marks"))) return rc;
+    BD_HIP(c, hipMemsetAsync(c->d_marks, 0, n + 2, c->stream));
+    if (n > 0)
+        hipLaunchKernelGGL(k_check_edges, dim3((unsigned)((n * 64 + 255) / 256)), dim3(256), 0,
+                           c->stream, (const int64_t *)c->d_off, (const int32_t *)c->d_cols, parent,
+                           depth, c->nv, c->nnz, chunk, source, c->d_marks, c->h_flags);
+    hipLaunchKernelGGL(k_check_roots, dim3(grid_for(c, c->nv, 256)), dim3(256), 0, c->stream,
+                       (const int64_t *)c->d_off, parent, depth, c->nv, chunk, source,
+                       (const uint8_t *)c->d_marks, c->h_flags);
     BD_HIP(c, hipGetLastError());
-    *parent = *buf;
-    *depth = *buf + c->nv;
+    BD_HIP(c, hipStreamSynchronize(c->stream));
+    *ok = (c->h_flags[0] | c->h_flags[1] | c->h_flags[2]) ? 0 : 1;
     return BD_OK;
 }
 
@@ -2446,25 +2503,22 @@ extern "C" int bd_bfs_fetch(bd_ctx *c, int32_t *depth, int64_t *parent) {
     if (!c->have_result) return set_err(c, BD_ESTATE, "no search has run");
     if (!depth && !parent) return BD_OK;
     BD_HIP(c, hipSetDevice(c->device));
-    int32_t *buf = nullptr;
-    const int32_t *dp = nullptr, *dd = nullptr;
-    int rc = graph_id_result(c, depth != nullptr, &buf, &dp, &dd);
-    struct guard {
-        int32_t *p;
-        ~guard() { dev_free(p); }
-    } g{buf};
+    readout r;
+    int rc = out_buffers(c, &r);
     if (rc) return rc;
+    clear_flags(c);
+    if ((rc = queue_result<int64_t>(c, parent ? r.parent : nullptr, depth ? r.depth : nullptr)))
+        return rc;
     if (depth)
-        BD_HIP(c, hipMemcpyAsync(depth, dd, sizeof(int32_t) * c->nv, hipMemcpyDeviceToHost,
+        BD_HIP(c, hipMemcpyAsync(depth, r.depth, sizeof(int32_t) * c->nv, hipMemcpyDeviceToHost,
                                  c->stream));
-    std::vector<int32_t> p;
-    if (parent) {
-        p.resize(c->nv);
-        BD_HIP(c, hipMemcpyAsync(p.data(), dp, sizeof(int32_t) * c->nv, hipMemcpyDeviceToHost,
+    if (parent)
+        BD_HIP(c, hipMemcpyAsync(parent, r.parent, sizeof(int64_t) * c->nv, hipMemcpyDeviceToHost,
                                  c->stream));
-    }
-    BD_HIP(c, hipStreamSynchronize(c->stream));
-    for (int64_t v = 0; parent && v < c->nv; ++v) parent[v] = p[v];
+    const char *why = nullptr;
+    if ((rc = read_flags(c, &why))) return rc;
+    if (why) return set_err(c, BD_EHIP, why);
+    if (depth && c->last_steps > kWalkLevels) c->depth_valid = true;
     return BD_OK;
 }
 
@@ -2502,37 +2556,22 @@ extern "C" int bd_bfs_count_traversed(bd_ctx *c, int64_t *out) {
 }
 
 // hybrid_bfs::check (hybrid_bfs.cc:281-379) of the last search, on the
-// device (k_check_tree: the same PASS/FAIL as the reference's textbook-BFS
+// device (k_check_edges: the same PASS/FAIL as the reference's textbook-BFS
 // comparison, without a host copy of the graph).
 extern "C" int bd_bfs_check(bd_ctx *c, int64_t source, int *ok) {
     if (!c || !ok) return BD_EINVAL;
     if (!c->have_result) return set_err(c, BD_ESTATE, "no search has run");
     if (source < 0 || source >= c->nv) return set_err(c, BD_ERANGE, "source out of range");
     BD_HIP(c, hipSetDevice(c->device));
-    if (c->d_perm) {
-        // the tree as the caller reads it (graph ids), checked on the graph
-        int32_t *buf = nullptr;
-        const int32_t *dp = nullptr, *dd = nullptr;
-        int rc = graph_id_result(c, false, &buf, &dp, &dd);
-        struct guard {
-            int32_t *p;
-            ~guard() { dev_free(p); }
-        } g{buf};
-        if (rc) return rc;
-        return check_tree(c, dp, buf + c->nv, false, source, ok);
-    }
-    if (!c->depth_valid) {
-        // a malformed tree is a FAIL, not an error
-        const char *why = nullptr;
-        int rc = tree_depths(c, c->d_parent, c->d_depth, &why);
-        if (rc) return rc;
-        if (why) {
-            *ok = 0;
-            return BD_OK;
-        }
-        c->depth_valid = true;
-    }
-    return check_tree(c, c->d_parent, c->d_depth, true, source, ok);
+    // the tree as the caller reads it (graph ids), checked on the graph; a
+    // malformed tree is a FAIL, not an error
+    readout r;
+    int rc = out_buffers(c, &r);
+    if (rc) return rc;
+    clear_flags(c);
+    int32_t *parent = (int32_t *)r.parent;
+    if ((rc = queue_result<int32_t>(c, parent, r.depth))) return rc;
+    return check_tree(c, parent, r.depth, source, ok);
 }
 
 // hybrid_bfs::check of a caller's parent array (nv entries, negative =
@@ -2547,15 +2586,20 @@ extern "C" int bd_bfs_check_parents(bd_ctx *c, int64_t source, const int64_t *pa
     std::vector<int32_t> p(nv);
     for (int64_t v = 0; v < nv; ++v)
         p[v] = parent[v] < 0 ? -1 : (parent[v] >= nv ? (int32_t)nv : (int32_t)parent[v]);
-    int32_t *d = nullptr;
-    int rc = dev_alloc(c, (void **)&d, sizeof(int32_t) * 2 * nv, "checked tree");
+    readout r;
+    int rc = out_buffers(c, &r);
     if (rc) return rc;
-    struct guard {
-        int32_t *p;
-        ~guard() { dev_free(p); }
-    } g{d};
-    BD_HIP(c, hipMemcpy(d, p.data(), sizeof(int32_t) * nv, hipMemcpyHostToDevice));
-    return check_tree(c, d, d + nv, false, source, ok);
+    int32_t *d = (int32_t *)r.parent;
+    BD_HIP(c, hipMemcpyAsync(d, p.data(), sizeof(int32_t) * nv, hipMemcpyHostToDevice, c->stream));
+    clear_flags(c);
+    if ((rc = tree_depths(c, d, r.depth, 0))) return rc;
+    const char *why = nullptr;
+    if ((rc = read_flags(c, &why))) return rc;
+    if (why) {  // before the edges: an out-of-range parent has no depth to look up
+        *ok = 0;
+        return BD_OK;
+    }
+    return check_tree(c, d, r.depth, source, ok);
 }
 
 // Time both directions at every step from the same state; the search follows

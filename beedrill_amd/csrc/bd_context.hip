@@ -40,6 +40,13 @@ void dev_free(void *p) {
 static void free_search(bd_ctx *c) {
     dev_free(c->d_depth);
     dev_free(c->d_parent);
+    dev_free(c->d_tree);
+    dev_free(c->d_out);
+    dev_free(c->d_marks);
+    c->d_tree = nullptr;
+    c->d_out = nullptr;
+    c->d_marks = nullptr;
+    c->depth_valid = false;
     dev_free(c->d_cand);
     dev_free(c->d_dirty);
     c->d_dirty = nullptr;
@@ -126,7 +133,6 @@ int alloc_search(bd_ctx *c) {
     c->cand_clean = false;  // the first search fills the candidate array
     int rc;
     const int64_t nv = c->nv, nw = c->nwords;
-    if ((rc = dev_alloc(c, (void **)&c->d_depth, sizeof(int32_t) * nv, "depth"))) return rc;
     if ((rc = dev_alloc(c, (void **)&c->d_parent, sizeof(int32_t) * nv, "parent"))) return rc;
     if ((rc = dev_alloc(c, (void **)&c->d_cand, sizeof(int32_t) * nv, "candidate parents")))
         return rc;
@@ -225,6 +231,7 @@ extern "C" int bd_create(bd_ctx **out, int device) {
         e = hipHostMalloc((void **)&c->h_res, sizeof(search_result), shared);
         if (e == hipSuccess) c->h_res->seq = 0;
     }
+    if (e == hipSuccess) e = hipHostMalloc((void **)&c->h_flags, 4 * sizeof(int32_t), shared);
     if (e == hipSuccess) {
         c->log_cap = 1 << 16;
         e = hipHostMalloc((void **)&c->h_log, sizeof(bd_level_rec) * c->log_cap, shared);
@@ -259,6 +266,7 @@ extern "C" int bd_destroy(bd_ctx *c) {
     dev_free(c->d_mlp_ws);
     if (c->h_ctl) (void)hipHostFree(c->h_ctl);
     if (c->h_res) (void)hipHostFree(c->h_res);
+    if (c->h_flags) (void)hipHostFree(c->h_flags);
     if (c->h_log) (void)hipHostFree(c->h_log);
     for (auto &e : c->ev)
         if (e) (void)hipEventDestroy(e);

@@ -95,4 +95,63 @@ __device__ __forceinline__ int select_bit(uint64_t x, int k) {
     return pos;
 }
 
+// The last vertex of [lo, nv) whose list starts at or before position k
+// (k < nnz, so that list is not empty).
+__device__ __forceinline__ int64_t owner_of(const int64_t *off, int64_t lo, int64_t nv, int64_t k) {
+    int64_t hi = nv;
+    while (hi - lo > 1) {
+        const int64_t mid = (lo + hi) >> 1;
+        if (off[mid] <= k)
+            lo = mid;
+        else
+            hi = mid;
+    }
+    return lo;
+}
+
+// Walk the list entries [c0, end) on one wave, whatever the degrees: 64
+// vertices at a time, their entries one per lane and kRangeRounds rounds in
+// flight.  open(v, b, e) starts a window (lane i: vertex v = first + i, list
+// [b, e), empty past nv); visit(o, q, live) takes kRangeRounds entries a lane:
+// position q, owner lane o; close(v, b, e) ends the window.  Wave-collective.
+constexpr int kRangeRounds = 4;
+template <typename Open, typename Visit, typename Close>
+__device__ __forceinline__ void walk_range(const int64_t *off, int64_t nv, int64_t nnz, int64_t c0,
+                                           int64_t end, Open open, Visit visit, Close close) {
+    const int lane = lane_id();
+    int64_t v0 = owner_of(off, 0, nv, c0);
+    for (int64_t k = c0; k < end;) {
+        const int64_t v = v0 + lane;
+        const int64_t b = v < nv ? off[v] : nnz, e = v < nv ? off[v + 1] : nnz;
+        const int64_t last = lane_bcast(e, 63);
+        const int64_t stop = last < end ? last : end;
+        if (stop <= k) {  // 64 empty lists
+            v0 = owner_of(off, v0, nv, k);
+            continue;
+        }
+        open(v, b, e);
+        for (int64_t q0 = k; q0 < stop; q0 += kRangeRounds * 64) {
+            int o[kRangeRounds];
+            int64_t q[kRangeRounds];
+            bool live[kRangeRounds];
+#pragma unroll
+            for (int j = 0; j < kRangeRounds; ++j) {
+                q[j] = q0 + 64 * j + lane;
+                live[j] = q[j] < stop;
+                if (!live[j]) q[j] = stop - 1;
+                o[j] = 0;
+#pragma unroll
+                for (int st = 32; st > 0; st >>= 1) {
+                    const int mid = o[j] + st;
+                    if (__shfl(b, mid) <= q[j]) o[j] = mid;
+                }
+            }
+            visit(o, q, live);
+        }
+        close(v, b, e);
+        k = stop;
+        v0 += 64;
+    }
+}
+
 }  // namespace bd

@@ -26,6 +26,13 @@
 
 namespace bd {
 
+// One range per wave of a grid that fills the device; at least 512 entries,
+// since each range starts with a search for its first vertex.
+int64_t range_entries(const bd_ctx *c) {
+    const int64_t waves = (int64_t)c->cu_count * 64;
+    return std::max<int64_t>((c->nnz + waves - 1) / waves, 512);
+}
+
 namespace {
 
 constexpr int kBlock = 256;
@@ -488,20 +495,6 @@ __global__ void k_fill_heads(uint64_t *__restrict__ head, int64_t nv) {
         head[v] = kNoHead;
 }
 
-// The last vertex of [lo, nv) whose list starts at or before position k
-// (k < nnz, so it is not empty).
-__device__ __forceinline__ int64_t owner_of(const int64_t *off, int64_t lo, int64_t nv, int64_t k) {
-    int64_t hi = nv;
-    while (hi - lo > 1) {
-        const int64_t mid = (lo + hi) >> 1;
-        if (off[mid] <= k)
-            lo = mid;
-        else
-            hi = mid;
-    }
-    return lo;
-}
-
 // The renumbered lists and the head index in one pass over the adjacency.
 // head[i] = (deg(i) << 32) | the neighbour of i of largest degree, the first
 // in CSR order among equals, or 0xffffffff when i has none.  One 8-byte load
@@ -533,68 +526,52 @@ __global__ __launch_bounds__(256) void k_layout_lists(
     const int64_t c0 = (((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6) * chunk;
     if (c0 >= nnz) return;
     const int64_t end = c0 + chunk < nnz ? c0 + chunk : nnz;
-    int64_t v0 = owner_of(soff, 0, nv, c0);
-    for (int64_t k = c0; k < end;) {
-        const int64_t i = v0 + lane;
-        const int64_t b = i < nv ? soff[i] : nnz, e = i < nv ? soff[i + 1] : nnz;
-        const int64_t stop = lane_bcast(e, 63) < end ? lane_bcast(e, 63) : end;
-        if (stop <= k) {  // 64 empty lists
-            v0 = owner_of(soff, v0, nv, k);
-            continue;
-        }
-        // old list start minus new
-        const int64_t shift = RENUMBER && i < nv && e > b ? off[perm[i]] - b : 0;
-        best[lane] = 0;
-        wave_lds_sync();
-        for (int64_t q0 = k; q0 < stop; q0 += 4 * 64) {
-            int o[4];
-            int32_t u[4];
-            uint64_t r[4];
-            int64_t bo[4];
+    int64_t shift = 0, start = 0;  // old list start minus new; list start
+    walk_range(
+        soff, nv, nnz, c0, end,
+        [&](int64_t i, int64_t b, int64_t e) {
+            shift = RENUMBER && i < nv && e > b ? off[perm[i]] - b : 0;
+            start = b;
+            best[lane] = 0;
+            wave_lds_sync();
+        },
+        [&](const int (&o)[kRangeRounds], const int64_t (&q)[kRangeRounds],
+            const bool (&live)[kRangeRounds]) {
+            int32_t u[kRangeRounds];
+            uint64_t r[kRangeRounds];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int64_t q = q0 + 64 * j + lane;
-                const int64_t qa = q < stop ? q : stop - 1;
-                o[j] = 0;
+            for (int j = 0; j < kRangeRounds; ++j)
+                u[j] = __builtin_nontemporal_load(cols + q[j] + __shfl(shift, o[j]));
 #pragma unroll
-                for (int st = 32; st > 0; st >>= 1) {
-                    const int mid = o[j] + st;
-                    if (__shfl(b, mid) <= qa) o[j] = mid;
-                }
-                bo[j] = __shfl(b, o[j]);
-                u[j] = __builtin_nontemporal_load(cols + qa + __shfl(shift, o[j]));
-            }
+            for (int j = 0; j < kRangeRounds; ++j) r[j] = rec[u[j]];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) r[j] = rec[u[j]];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int64_t q = q0 + 64 * j + lane;
-                const bool live = q < stop;
-                if (RENUMBER && live) scols[q] = (int32_t)(uint32_t)r[j];
+            for (int j = 0; j < kRangeRounds; ++j) {
+                if (RENUMBER && live[j]) scols[q[j]] = (int32_t)(uint32_t)r[j];
+                const int64_t pos = q[j] - __shfl(start, o[j]);
                 unsigned long long key =
-                    live ? ((r[j] >> 32) << 32) | (0xffffffffULL - (uint64_t)(q - bo[j])) : 0ULL;
+                    live[j] ? ((r[j] >> 32) << 32) | (0xffffffffULL - (uint64_t)pos) : 0ULL;
                 if (lane_bcast(o[j], 0) == lane_bcast(o[j], 63)) {
                     // one list: one write instead of 64 on one address
                     key = wave_max(key);
                     if (lane == 0 && key) atomicMax(&best[o[j]], key);
-                } else if (live) {
+                } else if (live[j]) {
                     atomicMax(&best[o[j]], key);
                 }
             }
-        }
-        wave_lds_sync();
-        const unsigned long long key = best[lane];
-        if (key) {
-            if (b >= c0 && e <= end)
-                head[i] = ((uint64_t)(e - b) << 32) |
-                          (uint32_t)rec[cols[b + shift + (int64_t)(0xffffffffULL - (key & 0xffffffffULL))]];
-            else
-                atomicMax((unsigned long long *)&head[i], key);
-        }
-        wave_lds_sync();
-        k = stop;
-        v0 += 64;
-    }
+        },
+        [&](int64_t i, int64_t b, int64_t e) {
+            wave_lds_sync();
+            const unsigned long long key = best[lane];
+            if (key) {
+                if (b >= c0 && e <= end)
+                    head[i] = ((uint64_t)(e - b) << 32) |
+                              (uint32_t)rec[cols[b + shift +
+                                                 (int64_t)(0xffffffffULL - (key & 0xffffffffULL))]];
+                else
+                    atomicMax((unsigned long long *)&head[i], key);
+            }
+            wave_lds_sync();
+        });
 }
 
 // The lists that lie across ranges: each one's best key becomes its entry,
@@ -676,10 +653,7 @@ static int build_lists(bd_ctx *c, const uint64_t *rec) {
     hipLaunchKernelGGL(k_fill_heads, dim3(grid1d(c, c->nv)), dim3(kBlock), 0, c->stream, c->d_head,
                        c->nv);
     if (c->nnz > 0) {
-        // one range per wave of a grid that fills the device; at least 512
-        // entries, since each range starts with a search for its first vertex
-        const int64_t waves = (int64_t)c->cu_count * 16 * (kBlock / 64);
-        const int64_t chunk = std::max<int64_t>((c->nnz + waves - 1) / waves, 512);
+        const int64_t chunk = range_entries(c);
         const int64_t n = (c->nnz + chunk - 1) / chunk;
         const dim3 grid((unsigned)((n * 64 + kBlock - 1) / kBlock)), block(kBlock);
         if (c->d_perm)

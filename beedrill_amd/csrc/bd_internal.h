@@ -161,7 +161,7 @@ struct bd_ctx {
     int s_order = 0;              // vertex_order the layout was built with (0: none yet)
 
     // search state
-    int32_t *d_depth = nullptr;
+    int32_t *d_depth = nullptr;   // deep searches' depths, in search ids (k_tree_*)
     int32_t *d_parent = nullptr;
     int32_t *d_cand = nullptr;    // candidate parents of a remote-write top-down step (-1 = none)
     uint8_t *d_dirty = nullptr;   // per visited word: a candidate was written into it (0 = none)
@@ -201,6 +201,11 @@ struct bd_ctx {
     // results of the last run
     bool have_result = false;
     bool depth_valid = false;  // d_depth holds the last search's depths
+    // readout workspaces, allocated when first needed and kept with the graph
+    uint64_t *d_tree = nullptr;   // ancestors of a deep parent tree
+    int64_t *d_out = nullptr;     // results in graph ids: nv parents, then nv depths
+    uint8_t *d_marks = nullptr;   // check: per range, its spanning list's parent was found
+    int32_t *h_flags = nullptr;   // pinned: faults a readout kernel found
     bool split_off = false;    // profiling: top-down steps never run with remote writes
     bool cand_clean = false;   // d_cand is all -1 (set when a search finishes)
     int chunk_hint = 0;        // first chunk of device-driven launches (0: 16)
@@ -266,6 +271,8 @@ int refresh_mlp_ops(bd_ctx *c);
 // Build device CSR from a device edge list (packed src<<32|dst, el order).
 int build_csr_from_el(bd_ctx *c, int64_t nv, int64_t m);
 int64_t grid_for(const bd_ctx *c, int64_t work_items, int block);
+// Entries of a wave's range of the adjacency (walk_range).
+int64_t range_entries(const bd_ctx *c);
 
 }  // namespace bd
 

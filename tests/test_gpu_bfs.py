@@ -868,3 +868,57 @@ def test_even_ranges_and_chunks(ctx, orc, nv, block, bu_words):
                 assert max(r["frontier"] for r in ctx.levels()) >= 4096
     finally:
         ctx.set_tuning(**t0)
+
+
+@pytest.mark.parametrize("n", [24, 25, 26, 64, 65])
+@pytest.mark.parametrize("order", [2, 4])
+def test_depths_on_both_sides_of_the_walk_rule(ctx, orc, n, order):
+    """Depths of searches of up to 24 levels are read by walking the parent
+    chains, of deeper ones by pointer jumping: paths at and beside the cut and
+    at powers of two, fetched twice, checked, with and without parents."""
+    t0 = ctx.get_tuning()
+    try:
+        ctx.set_tuning(vertex_order=order)
+        _, s, d = path_graph(n)
+        nv = n + 3  # and isolated vertices
+        ctx.from_edges(nv, s, d)
+        off, adj, m = oracle_csr(orc, nv, s, d)
+        for root in (0, n // 2, nv - 1):
+            ctx.bfs(root)
+            ref = orc.bfs_depth(off, adj, root)
+            for _ in range(2):
+                np.testing.assert_array_equal(ctx.fetch(parent=False)[0], ref)
+                depth, parent = ctx.fetch()
+                np.testing.assert_array_equal(depth, ref)
+                assert parent.dtype == np.int64 and orc.check(off, adj, root, parent)
+                np.testing.assert_array_equal(ctx.fetch(depth=False)[1], parent)
+            assert ctx.check(root) and ctx.check_parents(root, parent)
+            assert not ctx.check((root + 1) % nv)
+            if root < n:
+                bad = parent.copy()
+                bad[root], bad[(root + 1) % n] = (root + 1) % n, root  # a cycle
+                assert not ctx.check_parents(root, bad)
+    finally:
+        ctx.set_tuning(**t0)
+
+
+@pytest.mark.parametrize("hub", [510, 511, 512, 1024, 1300])
+def test_check_of_lists_across_ranges(ctx, orc, hub):
+    """check() reads 512 list entries per wave: a hub whose list crosses those
+    cuts, reached through its first, last or middle neighbour, passes, and
+    fails once its parent is not a neighbour or a depth is off by one."""
+    s = np.concatenate([np.zeros(hub, np.int64), [hub + 1, hub + 2]])
+    d = np.concatenate([np.arange(1, hub + 1), [1, hub + 1]])
+    nv = hub + 4
+    ctx.from_edges(nv, s, d)
+    off, adj, m = oracle_csr(orc, nv, s, d)
+    for root in (1, hub // 2, hub, hub + 2):
+        parent, depth, _ = orc.beamer(off, adj, m, root)
+        ctx.bfs(root)
+        assert ctx.check(root) and ctx.check_parents(root, parent)
+        for v, p in ((0, hub + 1), (0, hub + 2), (hub // 2 + 1, hub // 2 + 2), (nv - 1, 0)):
+            bad = np.where(parent < 0, -1, parent)
+            if bad[v] == p or v == root:
+                continue
+            bad[v] = p
+            assert ctx.check_parents(root, bad) == orc.check(off, adj, root, bad), (root, v, p)
