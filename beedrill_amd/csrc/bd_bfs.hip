@@ -119,8 +119,8 @@ struct step_args {
     int64_t n_hub_med, n_hub_big;
     ctl_block *c;
     seg_counters *seg;
-    bd_level_rec *log;     // pinned host memory, as is res
-    search_result *res;
+    bd_level_rec *hlog, *log;  // the first kHostRecs records (host memory), the others
+    search_result *res;    // host memory
     const int32_t *script;
     const float *mlp;
     const uint4 *mlp_ops;  // the network's operands in MFMA lane order
@@ -1374,7 +1374,7 @@ __device__ __forceinline__ bool rebuild_state(const step_args &a, step_smem<BLOC
                 r.ms_other = -1.0;
                 r.launches = dir == kDirTDClaim ? 2 : 1;
                 r.launch = L - r.launches;
-                a.log[idx] = r;
+                (idx < kHostRecs ? a.hlog : a.log)[idx] = r;
             }
             c->steps += 1;
             if (sd == BD_DIR_TD)
@@ -2020,7 +2020,8 @@ step_args make_args(bd_ctx *c, int32_t level, int64_t alpha, int64_t beta, int p
     a.n_hub_big = c->n_hub_big;
     a.c = c->d_ctl;
     a.seg = c->d_seg;
-    a.log = c->h_log;
+    a.hlog = c->h_log;
+    a.log = c->d_log;
     a.res = c->h_res;
     a.seq = c->search_seq;
     a.script = c->d_script;
@@ -2239,7 +2240,14 @@ int finish_search(bd_ctx *c, int64_t source, bd_run_stats *out, double host_ms) 
     c->have_result = true;
     c->cand_clean = true;  // every write half was followed by its claim sweep
     const int64_t n = std::min<int64_t>(h.steps, c->log_cap);
-    c->last_log.assign(c->h_log, c->h_log + n);
+    c->last_log.assign(c->h_log, c->h_log + std::min(n, kHostRecs));
+    if (n > kHostRecs) {
+        c->last_log.resize(n);
+        BD_HIP(c, hipMemcpyAsync(c->last_log.data() + kHostRecs, c->d_log + kHostRecs,
+                                 sizeof(bd_level_rec) * (n - kHostRecs), hipMemcpyDeviceToHost,
+                                 c->stream));
+        BD_HIP(c, hipStreamSynchronize(c->stream));
+    }
     if (out) {
         out->source = source;
         out->steps = h.steps;

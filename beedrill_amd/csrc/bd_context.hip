@@ -234,7 +234,7 @@ extern "C" int bd_create(bd_ctx **out, int device) {
     if (e == hipSuccess) e = hipHostMalloc((void **)&c->h_flags, 4 * sizeof(int32_t), shared);
     if (e == hipSuccess) {
         c->log_cap = 1 << 16;
-        e = hipHostMalloc((void **)&c->h_log, sizeof(bd_level_rec) * c->log_cap, shared);
+        e = hipHostMalloc((void **)&c->h_log, sizeof(bd_level_rec) * kHostRecs, shared);
     }
     if (e == hipSuccess) {
         e = hipMalloc((void **)&c->d_log, sizeof(bd_level_rec) * c->log_cap);

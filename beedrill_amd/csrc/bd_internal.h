@@ -110,6 +110,11 @@ struct ctl_block {
     int64_t reached_deg;
 };
 
+// Step records the device writes straight to host memory; a deeper search's
+// are copied when it ends.  (Pinning memory for all 65536 took 0.4 ms of
+// making a context.)
+constexpr int64_t kHostRecs = 512;
+
 // What a search leaves for the host, in pinned memory that the device writes:
 // the launch that finds the search done fills it and sets seq, last, to the
 // search's number, so the host reads the result without a copy or a
@@ -190,9 +195,9 @@ struct bd_ctx {
     bd::ctl_block *d_ctl = nullptr;  // two published copies (see ctl_block)
     bd::ctl_block *h_ctl = nullptr;  // pinned mirror of both copies
     bd::search_result *h_res = nullptr;  // pinned, written by the device
-    bd_level_rec *h_log = nullptr;       // pinned: step records, written by the device
+    bd_level_rec *h_log = nullptr;       // pinned: the first kHostRecs step records
     uint32_t search_seq = 0;             // number of the last search started
-    bd_level_rec *d_log = nullptr;       // level records of the bit-parallel search
+    bd_level_rec *d_log = nullptr;       // records past those, and the bit-parallel search's
     int64_t log_cap = 0;
     int32_t *d_script = nullptr;
     int64_t script_len = 0;
