@@ -2213,22 +2213,8 @@ bool search_done(const bd_ctx *c) {
     return __atomic_load_n(&c->h_res->seq, __ATOMIC_ACQUIRE) == c->search_seq;
 }
 
-// Wait until the search's result is there, or every launch queued so far has
-// ended without it.  The host watches the result's number, which arrives
-// before the launches queued past the search's end have run; they only look
-// at the done flag, and what is queued after them is ordered behind them.
-int wait_search(bd_ctx *c) {
-    for (unsigned n = 1;; ++n) {
-        if (search_done(c)) return BD_OK;
-        if ((n & 255) == 0) {
-            const hipError_t e = hipStreamQuery(c->stream);
-            if (e == hipSuccess) return BD_OK;
-            (void)hipGetLastError();
-            if (e != hipErrorNotReady) return hip_err(c, e, "hipStreamQuery");
-        }
-        __builtin_ia32_pause();
-    }
-}
+// Wait for the search's result (or for the launches queued so far).
+int wait_search(bd_ctx *c) { return wait_host_flag(c, &c->h_res->seq, c->search_seq); }
 
 int finish_search(bd_ctx *c, int64_t source, bd_run_stats *out, double host_ms) {
     if (!search_done(c)) return set_err(c, BD_EHIP, "search state not final");

@@ -53,17 +53,6 @@ static void free_search(bd_ctx *c) {
     dev_free(c->d_comp);
     dev_free(c->d_cc_flag);
     dev_free(c->d_cc_tasks);
-    dev_free(c->d_cc_chg);
-    dev_free(c->d_cc_bcols);
-    dev_free(c->d_cc_bend);
-    dev_free(c->d_cc_pieces);
-    dev_free(c->d_cc_pbase);
-    c->d_cc_pieces = nullptr;
-    c->d_cc_pbase = nullptr;
-    c->d_cc_chg = nullptr;
-    c->d_cc_bcols = nullptr;
-    c->d_cc_bend = nullptr;
-    c->cc_bshift = 0;
     c->d_comp = nullptr;
     c->d_cc_flag = nullptr;
     c->d_cc_tasks = nullptr;
@@ -119,6 +108,22 @@ void free_graph(bd_ctx *c) {
     c->d_el = nullptr;
     c->el_m = 0;
     c->nv = c->nnz = c->m = c->nwords = 0;
+}
+
+// The host watches the flag, which arrives before the launches queued past the
+// end have run; those only look at a done flag, and what is queued after them
+// is ordered behind them.
+int wait_host_flag(bd_ctx *c, const uint32_t *flag, uint32_t value) {
+    for (unsigned n = 1;; ++n) {
+        if (__atomic_load_n(flag, __ATOMIC_ACQUIRE) == value) return BD_OK;
+        if ((n & 255) == 0) {
+            const hipError_t e = hipStreamQuery(c->stream);
+            if (e == hipSuccess) return BD_OK;
+            (void)hipGetLastError();
+            if (e != hipErrorNotReady) return hip_err(c, e, "hipStreamQuery");
+        }
+        __builtin_ia32_pause();
+    }
 }
 
 int64_t grid_for(const bd_ctx *c, int64_t work_items, int block) {
@@ -267,6 +272,7 @@ extern "C" int bd_destroy(bd_ctx *c) {
     if (c->h_ctl) (void)hipHostFree(c->h_ctl);
     if (c->h_res) (void)hipHostFree(c->h_res);
     if (c->h_flags) (void)hipHostFree(c->h_flags);
+    if (c->h_cc) (void)hipHostFree(c->h_cc);
     if (c->h_log) (void)hipHostFree(c->h_log);
     for (auto &e : c->ev)
         if (e) (void)hipEventDestroy(e);

@@ -171,14 +171,10 @@ struct bd_ctx {
     int32_t *d_cand = nullptr;    // candidate parents of a remote-write top-down step (-1 = none)
     uint8_t *d_dirty = nullptr;   // per visited word: a candidate was written into it (0 = none)
     int32_t *d_comp = nullptr;    // connected-component labels (components_)
-    int32_t *d_cc_flag = nullptr; // [0] an edge pass changed a label, [1..] counters
+    int32_t *d_cc_flag = nullptr; // a component run's state and counters
     bool have_cc = false;         // d_comp holds a finished run
-    uint64_t *d_cc_chg = nullptr;       // two bitmaps of vertices whose label changed
-    int32_t *d_cc_bcols = nullptr;      // short lists regrouped by column block
-    uint64_t *d_cc_bend = nullptr;      // per vertex: end of each block's run (one byte each)
-    int cc_bshift = 0;                  // column blocks of 2^cc_bshift vertices
-    bd::td_task *d_cc_pieces = nullptr; // long-list pieces by (row block, column block)
-    int64_t *d_cc_pbase = nullptr;      // [65] start of each bucket's pieces
+    void *h_cc = nullptr;         // pinned: a component run's result, written by the device
+    int32_t cc_hub = 0;           // the vertex of largest degree
     bd::td_task *d_cc_tasks = nullptr;  // slices of the long lists of the edge pass
     int64_t cc_ntasks = -1;             // -1: not built for the resident graph
     double cc_prep_ms = 0;              // device time of that one-time build
@@ -276,6 +272,9 @@ int refresh_mlp_ops(bd_ctx *c);
 // Build device CSR from a device edge list (packed src<<32|dst, el order).
 int build_csr_from_el(bd_ctx *c, int64_t nv, int64_t m);
 int64_t grid_for(const bd_ctx *c, int64_t work_items, int block);
+// Wait until the device has set *flag (pinned host memory) to value, or every
+// launch queued so far has ended without that.
+int wait_host_flag(bd_ctx *c, const uint32_t *flag, uint32_t value);
 // Entries of a wave's range of the adjacency (walk_range).
 int64_t range_entries(const bd_ctx *c);
 

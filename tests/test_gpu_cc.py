@@ -107,3 +107,41 @@ def test_cli_components_check():
     out = r.stdout + r.stderr
     assert r.returncode == 0, out
     assert out.count("Found ") == 2 and "PASS" in out and "FAIL" not in out, out
+
+
+@pytest.mark.parametrize("order", [2, 4])
+def test_passes_that_skip_the_largest_label(ctx, orc, order):
+    """From the second pass on, vertices carrying the label of the vertex of
+    largest degree read nothing: components whose smallest ids lie on either
+    side of that label, joined to it through short lists, through lists cut
+    into slices, and through chains that need several passes, with components
+    and isolated vertices it never meets; twice, to reuse the slices."""
+    rng = np.random.default_rng(17)
+    nv, hub = 60000, 30000
+    near = rng.choice(np.arange(20000, 50000), 9000, replace=False)
+    near = near[near != hub]
+    src = [np.full(len(near), hub)]
+    dst = [near]
+    # a long list below the hub's labels, touching the hub's set at its end
+    src.append(np.full(3000, 7))
+    dst.append(np.concatenate([np.arange(100, 3099), near[:1]]))
+    # chains that start low, wander through high ids, and end at the hub's set
+    for k in range(8):
+        chain = np.concatenate([[10 + k], rng.choice(np.arange(50000, 59000), 120, replace=False),
+                                near[10 + k:11 + k]])
+        src.append(chain[:-1])
+        dst.append(chain[1:])
+    # components of their own, below and above the hub
+    src.append(np.arange(4000, 5000)); dst.append(np.arange(4001, 5001))
+    src.append(np.arange(59100, 59900)); dst.append(np.arange(59101, 59901))
+    s, d = np.concatenate(src).astype(np.int64), np.concatenate(dst).astype(np.int64)
+    t0 = ctx.get_tuning()
+    try:
+        ctx.set_tuning(vertex_order=order)
+        ctx.from_edges(nv, s, d)
+        off, adj = orc.build_csr(nv, s, d)
+        for _ in range(2):
+            st = compare(ctx, orc, off, adj)
+        assert st["num_components"] > 1000
+    finally:
+        ctx.set_tuning(**t0)
