@@ -592,12 +592,35 @@ __global__ void k_ms_hubs(const int64_t *__restrict__ off, int64_t nv, int32_t *
     }
 }
 
-// Row r of the depths in graph ids: out[v] = depth[r * nv + inv[v]].
-__global__ void k_ms_row(const int32_t *__restrict__ depth, const int32_t *__restrict__ inv,
-                         int64_t nv, int32_t *__restrict__ out) {
-    for (int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; v < nv;
-         v += (int64_t)gridDim.x * blockDim.x)
-        out[v] = depth[inv[v]];
+// Depths in graph ids, elements [first, first + n) of the root-major rows
+// (element r * nv + v is depth[r * nv + inv[v]]), into host memory: as bytes,
+// 255 unreached, four to a thread, or as they are.
+__device__ __forceinline__ int32_t ms_read(const int32_t *depth, const int32_t *inv, int64_t nv,
+                                           int64_t at) {
+    if (!inv) return depth[at];
+    const int64_t row = at / nv * nv;
+    return depth[row + inv[at - row]];
+}
+
+__global__ void k_ms_read(const int32_t *__restrict__ depth, const int32_t *__restrict__ inv,
+                          int64_t nv, int64_t first, int64_t n, int32_t *__restrict__ out) {
+    for (int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; k < n;
+         k += (int64_t)gridDim.x * blockDim.x)
+        out[k] = ms_read(depth, inv, nv, first + k);
+}
+
+__global__ void k_ms_read_bytes(const int32_t *__restrict__ depth, const int32_t *__restrict__ inv,
+                                int64_t nv, int64_t first, int64_t n, uint32_t *__restrict__ out) {
+    for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q * 4 < n;
+         q += (int64_t)gridDim.x * blockDim.x) {
+        uint32_t w = 0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int64_t k = q * 4 + j;
+            if (k < n) w |= (uint32_t)(uint8_t)ms_read(depth, inv, nv, first + k) << (8 * j);
+        }
+        out[q] = w;  // the ring's chunks end on a multiple of 4
+    }
 }
 
 // Masks, bitmaps, three counter copies with the control block, and (nrows
@@ -822,24 +845,24 @@ int run_multi_root(bd_ctx *c, const int64_t *roots, int n, int32_t *depths, doub
     for (int64_t i = 0; i < nrec && i < (int64_t)level_ms.size(); ++i) c->last_log[i].ms = level_ms[i];
     c->have_result = false;  // bd_bfs_levels now describes this search, not the last single one
     if (depths) {
-        if (!c->d_inv) {
-            BD_HIP(c, hipMemcpy(depths, a.depth, sizeof(int32_t) * n * nv, hipMemcpyDeviceToHost));
-        } else {
-            int32_t *row = nullptr;
-            if ((rc = dev_alloc(c, (void **)&row, sizeof(int32_t) * nv, "depth row"))) return rc;
-            struct rguard {
-                void *p;
-                ~rguard() { dev_free(p); }
-            } rg{row};
-            for (int r = 0; r < n; ++r) {
-                hipLaunchKernelGGL(k_ms_row, dim3(grid_for(c, nv, 256)), dim3(256), 0, c->stream,
-                                   a.depth + (int64_t)r * nv, c->d_inv, nv, row);
-                BD_HIP(c, hipGetLastError());
-                BD_HIP(c, hipMemcpyAsync(depths + (int64_t)r * nv, row, sizeof(int32_t) * nv,
-                                         hipMemcpyDeviceToHost, c->stream));
-            }
-            BD_HIP(c, hipStreamSynchronize(c->stream));
-        }
+        const bool bytes = h.levels <= 250;  // depths fit a byte
+        rc = carry_out(c, bytes ? carry::u8_i32 : carry::i32_i32, depths, (int64_t)n * nv,
+                       [&](int64_t first, int64_t cnt, void *out) -> int {
+                           if (bytes)
+                               hipLaunchKernelGGL(k_ms_read_bytes,
+                                                  dim3(grid_for(c, (cnt + 3) / 4, 256)), dim3(256),
+                                                  0, c->stream, (const int32_t *)a.depth,
+                                                  (const int32_t *)c->d_inv, nv, first, cnt,
+                                                  (uint32_t *)out);
+                           else
+                               hipLaunchKernelGGL(k_ms_read, dim3(grid_for(c, cnt, 256)), dim3(256),
+                                                  0, c->stream, (const int32_t *)a.depth,
+                                                  (const int32_t *)c->d_inv, nv, first, cnt,
+                                                  (int32_t *)out);
+                           BD_HIP(c, hipGetLastError());
+                           return BD_OK;
+                       });
+        if (rc) return rc;
     }
     return BD_OK;
 }

@@ -1785,45 +1785,82 @@ __global__ void k_count_traversed(const int32_t *__restrict__ parent,
 //
 // A search's result in graph ids: vertex v is search id inv[v], and a parent
 // p (a search id) is graph vertex perm[p] (no inv: ids are as they are).
-// Either output may be null.  Depths come from sdepth, or, when that is null,
-// from walking the chain: a search of few levels has short chains whose upper
-// ends are shared and cached, and one launch replaces the rounds of pointer
-// jumping, their host waits and the mapping (scale 16: 12 launches and copies,
-// 190 us a fetch).  flags (host memory, written only on a fault): [0] a chain
-// longer than limit, [1] an unreached or out-of-range ancestor.
-template <typename P>
-__global__ void k_result(const int32_t *__restrict__ inv, const int32_t *__restrict__ perm,
-                         const int32_t *__restrict__ sparent, const int32_t *__restrict__ sdepth,
-                         int64_t nv, int64_t limit, P *__restrict__ parent,
-                         int32_t *__restrict__ depth, int32_t *__restrict__ flags) {
-    for (int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; v < nv;
+// Depths come from sdepth, or, when that is null, from walking the chain: a
+// search of few levels has short chains whose upper ends are shared and
+// cached, and one launch replaces the rounds of pointer jumping, their host
+// waits and the mapping (scale 16: 12 launches and copies, 190 us a fetch).
+// flags (host memory, written only on a fault): [0] a chain longer than
+// limit, [1] an unreached or out-of-range ancestor.
+struct tree_args {
+    const int32_t *inv, *perm, *sparent, *sdepth;
+    int64_t nv, limit;
+    int32_t *flags;
+};
+
+__device__ __forceinline__ int32_t result_depth(const tree_args &a, int32_t i) {
+    if (a.sdepth) return a.sdepth[i];
+    const int32_t p = a.sparent[i];
+    if (p < 0) return -1;
+    int32_t d = 0;
+    for (int32_t x = i, y = p; y != x;) {
+        const int32_t z = (int64_t)y < a.nv ? a.sparent[y] : -1;
+        if (z < 0) {
+            a.flags[1] = 1;
+            break;
+        }
+        if (++d > a.limit) {
+            a.flags[0] = 1;
+            break;
+        }
+        x = y;
+        y = z;
+    }
+    return d;
+}
+
+__device__ __forceinline__ int32_t result_parent(const tree_args &a, int32_t i) {
+    const int32_t p = a.sparent[i];
+    return p < 0 ? -1 : (a.perm ? a.perm[p] : p);
+}
+
+// Both, of every vertex, for check().
+__global__ void k_result(tree_args a, int32_t *__restrict__ parent, int32_t *__restrict__ depth) {
+    for (int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; v < a.nv;
          v += (int64_t)gridDim.x * blockDim.x) {
-        const int32_t i = inv ? inv[v] : (int32_t)v;
-        const int32_t p = sparent[i];
-        if (parent) parent[v] = p < 0 ? -1 : (P)(perm ? perm[p] : p);
-        if (!depth) continue;
-        if (sdepth) {
-            depth[v] = sdepth[i];
-            continue;
+        const int32_t i = a.inv ? a.inv[v] : (int32_t)v;
+        parent[v] = result_parent(a, i);
+        depth[v] = result_depth(a, i);
+    }
+}
+
+// The parents of n vertices from `first`, into host memory.
+__global__ void k_read_parents(tree_args a, int64_t first, int64_t n, int32_t *__restrict__ out) {
+    for (int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; k < n;
+         k += (int64_t)gridDim.x * blockDim.x)
+        out[k] = result_parent(a, a.inv ? a.inv[first + k] : (int32_t)(first + k));
+}
+
+// Their depths; as bytes (255: unreached) four to a thread, so that a wave's
+// store still covers 256 bytes.
+__global__ void k_read_depths(tree_args a, int64_t first, int64_t n, int32_t *__restrict__ out) {
+    for (int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; k < n;
+         k += (int64_t)gridDim.x * blockDim.x)
+        out[k] = result_depth(a, a.inv ? a.inv[first + k] : (int32_t)(first + k));
+}
+
+__global__ void k_read_depth_bytes(tree_args a, int64_t first, int64_t n,
+                                   uint32_t *__restrict__ out) {
+    for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q * 4 < n;
+         q += (int64_t)gridDim.x * blockDim.x) {
+        uint32_t w = 0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int64_t k = q * 4 + j;
+            if (k >= n) break;
+            const int64_t v = first + k;
+            w |= (uint32_t)(uint8_t)result_depth(a, a.inv ? a.inv[v] : (int32_t)v) << (8 * j);
         }
-        int32_t d = -1;
-        if (p >= 0) {
-            d = 0;
-            for (int32_t x = i, y = p; y != x;) {
-                const int32_t z = (int64_t)y < nv ? sparent[y] : -1;
-                if (z < 0) {
-                    flags[1] = 1;
-                    break;
-                }
-                if (++d > limit) {
-                    flags[0] = 1;
-                    break;
-                }
-                x = y;
-                y = z;
-            }
-        }
-        depth[v] = d;
+        out[q] = w;  // the ring's chunks end on a multiple of 4
     }
 }
 
@@ -2375,20 +2412,20 @@ extern "C" int bd_bfs_set_script(bd_ctx *c, const int32_t *dirs, int64_t n) {
     return BD_OK;
 }
 
-// Readout results: parents (and depths) in graph ids, d_out's halves.
+// check()'s tree: parents and depths in graph ids, d_out's halves.
 struct readout {
-    int64_t *parent;
+    int32_t *parent;
     int32_t *depth;
 };
 
 int out_buffers(bd_ctx *c, readout *r) {
     if (!c->d_out) {
-        int rc = dev_alloc(c, (void **)&c->d_out, (sizeof(int64_t) + sizeof(int32_t)) * c->nv,
+        int rc = dev_alloc(c, (void **)&c->d_out, 2 * sizeof(int32_t) * c->nv,
                            "results in graph ids");
         if (rc) return rc;
     }
     r->parent = c->d_out;
-    r->depth = (int32_t *)(c->d_out + c->nv);
+    r->depth = c->d_out + c->nv;
     return BD_OK;
 }
 
@@ -2449,24 +2486,22 @@ int tree_depths(bd_ctx *c, const int32_t *parent, int32_t *depth, int64_t max_de
     return BD_OK;
 }
 
-// Queue the last search's result in graph ids: parents as P (int64 for a
-// caller, int32 for check()) and depths; either may be null.  Faults in the
-// tree go to h_flags.
-template <typename P>
-int queue_result(bd_ctx *c, P *parent, int32_t *depth) {
-    int rc;
+// Searches of at most this many levels have depths that fit a byte.
+constexpr int64_t kByteLevels = 250;
+
+// What the readout kernels need of the last search; with depth, a deep
+// search's depths are found first.  Faults in the tree go to h_flags.
+int result_args(bd_ctx *c, bool depth, tree_args *a) {
     const bool deep = depth && c->last_steps > kWalkLevels;
     if (deep && !c->depth_valid) {
+        int rc;
         if (!c->d_depth &&
             (rc = dev_alloc(c, (void **)&c->d_depth, sizeof(int32_t) * c->nv, "depth")))
             return rc;
         if ((rc = tree_depths(c, c->d_parent, c->d_depth, c->last_steps + 1))) return rc;
     }
-    hipLaunchKernelGGL(k_result<P>, dim3(grid_for(c, c->nv, 256)), dim3(256), 0, c->stream,
-                       (const int32_t *)c->d_inv, (const int32_t *)c->d_perm,
-                       (const int32_t *)c->d_parent, (const int32_t *)(deep ? c->d_depth : nullptr),
-                       c->nv, c->last_steps + 1, parent, depth, c->h_flags);
-    BD_HIP(c, hipGetLastError());
+    *a = tree_args{c->d_inv, c->d_perm, c->d_parent, deep ? c->d_depth : nullptr,
+                   c->nv, c->last_steps + 1, c->h_flags};
     return BD_OK;
 }
 
@@ -2497,18 +2532,36 @@ extern "C" int bd_bfs_fetch(bd_ctx *c, int32_t *depth, int64_t *parent) {
     if (!c->have_result) return set_err(c, BD_ESTATE, "no search has run");
     if (!depth && !parent) return BD_OK;
     BD_HIP(c, hipSetDevice(c->device));
-    readout r;
-    int rc = out_buffers(c, &r);
-    if (rc) return rc;
     clear_flags(c);
-    if ((rc = queue_result<int64_t>(c, parent ? r.parent : nullptr, depth ? r.depth : nullptr)))
-        return rc;
-    if (depth)
-        BD_HIP(c, hipMemcpyAsync(depth, r.depth, sizeof(int32_t) * c->nv, hipMemcpyDeviceToHost,
-                                 c->stream));
-    if (parent)
-        BD_HIP(c, hipMemcpyAsync(parent, r.parent, sizeof(int64_t) * c->nv, hipMemcpyDeviceToHost,
-                                 c->stream));
+    tree_args a;
+    int rc = result_args(c, depth != nullptr, &a);
+    if (rc) return rc;
+    const auto grid = [&](int64_t n) { return dim3((unsigned)grid_for(c, n, 256)); };
+    if (depth) {
+        const bool bytes = c->last_steps <= kByteLevels;
+        rc = carry_out(c, bytes ? carry::u8_i32 : carry::i32_i32, depth, c->nv,
+                       [&](int64_t first, int64_t n, void *out) -> int {
+                           if (bytes)
+                               hipLaunchKernelGGL(k_read_depth_bytes, grid((n + 3) / 4), dim3(256),
+                                                  0, c->stream, a, first, n, (uint32_t *)out);
+                           else
+                               hipLaunchKernelGGL(k_read_depths, grid(n), dim3(256), 0, c->stream,
+                                                  a, first, n, (int32_t *)out);
+                           BD_HIP(c, hipGetLastError());
+                           return BD_OK;
+                       });
+        if (rc) return rc;
+    }
+    if (parent) {
+        rc = carry_out(c, carry::i32_i64, parent, c->nv,
+                       [&](int64_t first, int64_t n, void *out) -> int {
+                           hipLaunchKernelGGL(k_read_parents, grid(n), dim3(256), 0, c->stream, a,
+                                              first, n, (int32_t *)out);
+                           BD_HIP(c, hipGetLastError());
+                           return BD_OK;
+                       });
+        if (rc) return rc;
+    }
     const char *why = nullptr;
     if ((rc = read_flags(c, &why))) return rc;
     if (why) return set_err(c, BD_EHIP, why);
@@ -2563,9 +2616,12 @@ extern "C" int bd_bfs_check(bd_ctx *c, int64_t source, int *ok) {
     int rc = out_buffers(c, &r);
     if (rc) return rc;
     clear_flags(c);
-    int32_t *parent = (int32_t *)r.parent;
-    if ((rc = queue_result<int32_t>(c, parent, r.depth))) return rc;
-    return check_tree(c, parent, r.depth, source, ok);
+    tree_args a;
+    if ((rc = result_args(c, true, &a))) return rc;
+    hipLaunchKernelGGL(k_result, dim3(grid_for(c, c->nv, 256)), dim3(256), 0, c->stream, a,
+                       r.parent, r.depth);
+    BD_HIP(c, hipGetLastError());
+    return check_tree(c, r.parent, r.depth, source, ok);
 }
 
 // hybrid_bfs::check of a caller's parent array (nv entries, negative =
@@ -2583,7 +2639,7 @@ extern "C" int bd_bfs_check_parents(bd_ctx *c, int64_t source, const int64_t *pa
     readout r;
     int rc = out_buffers(c, &r);
     if (rc) return rc;
-    int32_t *d = (int32_t *)r.parent;
+    int32_t *d = r.parent;
     BD_HIP(c, hipMemcpyAsync(d, p.data(), sizeof(int32_t) * nv, hipMemcpyHostToDevice, c->stream));
     clear_flags(c);
     if ((rc = tree_depths(c, d, r.depth, 0))) return rc;

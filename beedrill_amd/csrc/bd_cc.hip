@@ -356,13 +356,6 @@ __global__ __launch_bounds__(64) void k_cc_close(const int32_t *__restrict__ com
     __hip_atomic_store(&res->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-__global__ void k_cc_widen(const int32_t *__restrict__ comp, int64_t nv,
-                           int64_t *__restrict__ out) {
-    for (int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; v < nv;
-         v += (int64_t)gridDim.x * blockDim.x)
-        out[v] = comp[v];
-}
-
 }  // namespace
 }  // namespace bd
 
@@ -483,18 +476,7 @@ extern "C" int bd_cc_fetch(bd_ctx *c, int64_t *labels) {
     if (!c || !labels) return BD_EINVAL;
     if (!c->have_cc) return set_err(c, BD_ESTATE, "components have not run");
     BD_HIP(c, hipSetDevice(c->device));
-    int rc;
-    if (!c->d_out && (rc = dev_alloc(c, (void **)&c->d_out,
-                                     (sizeof(int64_t) + sizeof(int32_t)) * c->nv,
-                                     "results in graph ids")))
-        return rc;
-    hipLaunchKernelGGL(k_cc_widen, dim3(grid_for(c, c->nv, 256)), dim3(256), 0, c->stream,
-                       (const int32_t *)c->d_comp, c->nv, c->d_out);
-    BD_HIP(c, hipGetLastError());
-    BD_HIP(c, hipMemcpyAsync(labels, c->d_out, sizeof(int64_t) * c->nv, hipMemcpyDeviceToHost,
-                             c->stream));
-    BD_HIP(c, hipStreamSynchronize(c->stream));
-    return BD_OK;
+    return carry_copy(c, carry::i32_i64, labels, c->d_comp, c->nv);
 }
 
 // components::check (components.cc:152-202) on the host, from downloaded

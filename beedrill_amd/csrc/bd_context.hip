@@ -274,6 +274,7 @@ extern "C" int bd_destroy(bd_ctx *c) {
     if (c->h_flags) (void)hipHostFree(c->h_flags);
     if (c->h_cc) (void)hipHostFree(c->h_cc);
     if (c->h_log) (void)hipHostFree(c->h_log);
+    free_ring(c);
     for (auto &e : c->ev)
         if (e) (void)hipEventDestroy(e);
     for (auto &e : c->ev_pool)
@@ -297,10 +298,9 @@ extern "C" int bd_graph_download(bd_ctx *c, int64_t *off, int32_t *cols) {
     if (!c) return BD_EINVAL;
     if (!c->d_off) return set_err(c, BD_ESTATE, "no graph");
     BD_HIP(c, hipSetDevice(c->device));
-    if (off)
-        BD_HIP(c, hipMemcpy(off, c->d_off, sizeof(int64_t) * (c->nv + 1), hipMemcpyDeviceToHost));
-    if (cols)
-        BD_HIP(c, hipMemcpy(cols, c->d_cols, sizeof(int32_t) * c->nnz, hipMemcpyDeviceToHost));
+    int rc;
+    if (off && (rc = carry_copy(c, carry::i64_i64, off, c->d_off, c->nv + 1))) return rc;
+    if (cols && (rc = carry_copy(c, carry::i32_i32, cols, c->d_cols, c->nnz))) return rc;
     return BD_OK;
 }
 

@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <functional>
 #include <string>
 #include <vector>
 
@@ -115,6 +116,9 @@ struct ctl_block {
 // making a context.)
 constexpr int64_t kHostRecs = 512;
 
+// Chunks of the pinned ring that results are read through (bd_readout.hip).
+constexpr int kRing = 16;
+
 // What a search leaves for the host, in pinned memory that the device writes:
 // the launch that finds the search done fills it and sets seq, last, to the
 // search's number, so the host reads the result without a copy or a
@@ -204,9 +208,12 @@ struct bd_ctx {
     bool depth_valid = false;  // d_depth holds the last search's depths
     // readout workspaces, allocated when first needed and kept with the graph
     uint64_t *d_tree = nullptr;   // ancestors of a deep parent tree
-    int64_t *d_out = nullptr;     // results in graph ids: nv parents, then nv depths
+    int32_t *d_out = nullptr;     // check(): nv parents in graph ids, then nv depths
     uint8_t *d_marks = nullptr;   // check: per range, its spanning list's parent was found
     int32_t *h_flags = nullptr;   // pinned: faults a readout kernel found
+    void *h_ring = nullptr;       // pinned: results on their way to the caller (bd_readout.hip)
+    int64_t ring_bytes = 0;
+    hipEvent_t ring_ev[bd::kRing] = {};
     bool split_off = false;    // profiling: top-down steps never run with remote writes
     bool cand_clean = false;   // d_cand is all -1 (set when a search finishes)
     int chunk_hint = 0;        // first chunk of device-driven launches (0: 16)
@@ -275,6 +282,17 @@ int64_t grid_for(const bd_ctx *c, int64_t work_items, int block);
 // Wait until the device has set *flag (pinned host memory) to value, or every
 // launch queued so far has ended without that.
 int wait_host_flag(bd_ctx *c, const uint32_t *flag, uint32_t value);
+// Narrow form of a result on its way to the host, and the caller's form.
+enum class carry { u8_i32, i32_i32, i32_i64, i64_i64 };
+// Queues, on the context's stream, what writes elements [first, first + count)
+// of the narrow form to out (pinned memory).
+using carry_part = std::function<int(int64_t first, int64_t count, void *out)>;
+// Bring n elements to the caller's dst, in chunks queued by part; dst is
+// complete on return.
+int carry_out(bd_ctx *c, carry kind, void *dst, int64_t n, const carry_part &part);
+// The same from a device array that holds the narrow form (on 16 bytes).
+int carry_copy(bd_ctx *c, carry kind, void *dst, const void *src, int64_t n);
+void free_ring(bd_ctx *c);
 // Entries of a wave's range of the adjacency (walk_range).
 int64_t range_entries(const bd_ctx *c);
 

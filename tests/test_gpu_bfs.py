@@ -922,3 +922,45 @@ def test_check_of_lists_across_ranges(ctx, orc, hub):
                 continue
             bad[v] = p
             assert ctx.check_parents(root, bad) == orc.check(off, adj, root, bad), (root, v, p)
+
+
+@pytest.mark.parametrize("nv", [262143, 262145, 1048576, 1048579, 4194305, 4300001])
+def test_results_on_both_sides_of_the_readout_chunks(ctx, orc, nv):
+    """Depths, parents, labels and the CSR are read in chunks of 1 MB through a
+    ring of 16: sizes at a chunk's ends, and ids past the ring's (4 M)."""
+    ctx.generate_er(nv, 2 * nv + 3, seed=nv & 7)
+    s, d = ctx.edges()
+    off, cols = ctx.csr()
+    deg = np.bincount(s, minlength=nv) + np.bincount(d, minlength=nv)
+    np.testing.assert_array_equal(np.diff(off), deg)
+    assert off[0] == 0 and off[-1] == cols.size
+    # every list's entries, whatever their order
+    a = np.sort(np.repeat(np.arange(nv), deg) * nv + cols)
+    b = np.sort(np.concatenate([s * nv + d, d * nv + s]))
+    np.testing.assert_array_equal(a, b)
+    root = int(ctx.pick_roots(1)[0])
+    st = ctx.bfs(root)
+    depth, parent = ctx.fetch()
+    np.testing.assert_array_equal(depth, orc.bfs_depth(off, cols, root))
+    assert (depth >= 0).sum() == st["reached"]
+    np.testing.assert_array_equal(parent >= 0, depth >= 0)
+    child = (parent >= 0) & (np.arange(nv) != root)
+    np.testing.assert_array_equal(depth[child], depth[parent[child]] + 1)
+    assert orc.check(off, cols, root, parent)
+    ctx.components()
+    labels, _, _ = orc.components(off, cols)
+    np.testing.assert_array_equal(ctx.component_labels(), labels)
+
+
+@pytest.mark.parametrize("length", [249, 250, 251, 252, 300])
+def test_depths_on_both_sides_of_a_byte(ctx, orc, length):
+    """A search of up to 250 levels is read as bytes, a deeper one as ints."""
+    nv = length + 40  # the last vertices are unreached
+    src = np.arange(length - 1)
+    ctx.from_edges(nv, src, src + 1)
+    want = np.where(np.arange(nv) < length, np.arange(nv), -1)
+    ctx.bfs(0)
+    np.testing.assert_array_equal(ctx.fetch()[0], want)
+    rows = ctx.multi_root([0, 3])[0]
+    np.testing.assert_array_equal(rows[0], want)
+    np.testing.assert_array_equal(rows[1], np.where(want < 0, -1, abs(want - 3)))
