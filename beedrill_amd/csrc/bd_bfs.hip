@@ -167,17 +167,21 @@ struct step_close {
     int32_t dir, in_bu_loop, done;
 };
 
-// Per-workgroup LDS state.  The top-down staging and tile arrays and the
-// bottom-up found words, pending lists and first hits share one union, sized
-// by the workgroup.
-template <int BLOCK>
-struct step_smem {
+// What closing a step and choosing the next one's direction works on (LDS).
+struct step_state {
     ctl_block st;  // the search state before this step
     long long s_new, s_new_deg;
     int s_dir;
     int s_split;  // the step closed was a top-down step with remote writes
     float x[8], y[2];  // the network's inputs and outputs
     step_close pre;    // what predict_costs starts from
+};
+
+// Per-workgroup LDS state.  The top-down staging and tile arrays and the
+// bottom-up found words, pending lists and first hits share one union, sized
+// by the workgroup.
+template <int BLOCK>
+struct step_smem : step_state {
     unsigned long long red[4][BLOCK / 64];
     int32_t qn;
     int64_t qpos, qopos;
@@ -1173,8 +1177,7 @@ __device__ __forceinline__ void beamer_next(const step_args &a, ctl_block *c, in
 // Choose the direction of the step described by *c on one wave (no
 // workgroup barrier): lane 0 updates the state; the learned policy evaluates
 // its network on the wave.
-template <int BLOCK>
-__device__ __forceinline__ void choose_dir(const step_args &a, step_smem<BLOCK> &s, ctl_block *c, int32_t last_dir,
+__device__ __forceinline__ void choose_dir(const step_args &a, step_state &s, ctl_block *c, int32_t last_dir,
                            int64_t nnew, int64_t nnew_deg) {
     if (lane_id() == 0) {
         switch (a.policy) {
@@ -1273,6 +1276,65 @@ __device__ __forceinline__ void seg_prefix(int64_t n, int64_t ovf, int64_t seg_c
 constexpr int kCtlWords = (int)(sizeof(ctl_block) / 8);
 static_assert(kCtlWords <= 3 * 64, "ctl_block is copied as three words per lane");
 
+// Launches of the step described by *c.
+__device__ __forceinline__ int32_t step_launches(const ctl_block *c) {
+    return c->dir == kDirTDClaim ? 2 : 1;
+}
+
+// The record of the step described by *c, which found nnew vertices (one
+// lane).
+__device__ __forceinline__ void write_record(const step_args &a, const ctl_block *c, int64_t nnew,
+                                             int64_t nnew_deg, int64_t examined) {
+    const int64_t idx = c->steps;  // records are per level
+    if (idx >= a.log_cap) return;
+    const int32_t sd = step_dir(c->dir);
+    bd_level_rec r;
+    r.level = idx;
+    r.dir = sd;
+    r.frontier = c->frontier;
+    r.frontier_deg = c->frontier_deg;
+    r.unvisited = c->unvisited;
+    r.unvisited_deg = c->unvisited_deg;
+    r.edges_to_check = c->edges_to_check;
+    r.result = sd == BD_DIR_TD ? nnew_deg : nnew;
+    r.next = nnew;
+    r.next_deg = nnew_deg;
+    r.edges_examined = sd == BD_DIR_TD ? c->frontier_deg : examined;
+    r.max_frontier_deg = c->max_frontier_deg;
+    r.tasks = c->tpref[kSeg + 1];
+    r.queued = c->qpref[kSeg + 1];
+    r.ms = -1.0;
+    r.ms_other = -1.0;
+    r.launch = c->launches;
+    r.launches = step_launches(c);
+    (idx < kHostRecs ? a.hlog : a.log)[idx] = r;
+}
+
+// *c becomes the state after that step, its direction not yet chosen.
+__device__ __forceinline__ void close_totals(ctl_block *c, int64_t nnew, int64_t nnew_deg,
+                                             int64_t max_deg) {
+    const int32_t dir = c->dir, sd = step_dir(dir);
+    c->launches += step_launches(c);
+    c->steps += 1;
+    if (sd == BD_DIR_TD)
+        c->td_steps += 1;
+    else
+        c->bu_steps += 1;
+    c->reached += nnew;
+    c->reached_deg += nnew_deg;
+    c->unvisited -= nnew;
+    c->unvisited_deg -= nnew_deg;
+    c->frontier = nnew;
+    c->frontier_deg = nnew_deg;
+    c->max_frontier_deg = max_deg;
+    c->prev_dir = sd;
+    // after a bottom-up step or a claim sweep the frontier is only
+    // in the bitmap
+    c->td_bitmap = (kernel_dir(dir) == BD_DIR_BU || c->td_nolist) ? 1 : 0;
+    c->level = (int32_t)c->steps;
+    if (nnew == 0) c->done = 1;
+}
+
 // Rebuild, in s.st, the state before step L = a.level from the published
 // state before step L-1 and the counters of step L-1: close step L-1
 // (record, totals), describe frontier L (segment prefix sums) and choose
@@ -1281,11 +1343,7 @@ static_assert(kCtlWords <= 3 * 64, "ctl_block is copied as three words per lane"
 // (workgroup 0) also writes the step record.  All global loads are issued
 // before any is used, so the rebuild costs one memory round trip.  Returns
 // true, having changed nothing, when the search ended before this level.
-template <int BLOCK>
-__device__ __forceinline__ void predict_costs(const step_args &a, step_smem<BLOCK> &s);
-
-template <int BLOCK>
-__device__ __forceinline__ bool rebuild_state(const step_args &a, step_smem<BLOCK> &s, bool publish) {
+__device__ __forceinline__ bool rebuild_state(const step_args &a, step_state &s, bool publish) {
     const int L = a.level;
     const int l = lane_id();
     seg_counters *g = a.seg;
@@ -1353,47 +1411,8 @@ __device__ __forceinline__ bool rebuild_state(const step_args &a, step_smem<BLOC
             const int64_t nnew = (int64_t)nn;
             const int64_t nnew_deg = (int64_t)nd;
             const int32_t sd = step_dir(dir);
-            const int64_t idx = c->steps;  // records are per level
-            if (publish && idx < a.log_cap) {
-                bd_level_rec r;
-                r.level = idx;
-                r.dir = sd;
-                r.frontier = c->frontier;
-                r.frontier_deg = c->frontier_deg;
-                r.unvisited = c->unvisited;
-                r.unvisited_deg = c->unvisited_deg;
-                r.edges_to_check = c->edges_to_check;
-                r.result = sd == BD_DIR_TD ? nnew_deg : nnew;
-                r.next = nnew;
-                r.next_deg = nnew_deg;
-                r.edges_examined = sd == BD_DIR_TD ? c->frontier_deg : (int64_t)ex;
-                r.max_frontier_deg = c->max_frontier_deg;
-                r.tasks = c->tpref[kSeg + 1];
-                r.queued = c->qpref[kSeg + 1];
-                r.ms = -1.0;
-                r.ms_other = -1.0;
-                r.launches = dir == kDirTDClaim ? 2 : 1;
-                r.launch = L - r.launches;
-                (idx < kHostRecs ? a.hlog : a.log)[idx] = r;
-            }
-            c->steps += 1;
-            if (sd == BD_DIR_TD)
-                c->td_steps += 1;
-            else
-                c->bu_steps += 1;
-            c->reached += nnew;
-            c->reached_deg += nnew_deg;
-            c->unvisited -= nnew;
-            c->unvisited_deg -= nnew_deg;
-            c->frontier = nnew;
-            c->frontier_deg = nnew_deg;
-            c->max_frontier_deg = (int64_t)mx;
-            c->prev_dir = sd;
-            // after a bottom-up step or a claim sweep the frontier is only
-            // in the bitmap
-            c->td_bitmap = (kernel_dir(dir) == BD_DIR_BU || c->td_nolist) ? 1 : 0;
-            c->level = (int32_t)c->steps;
-            if (nnew == 0) c->done = 1;
+            if (publish) write_record(a, c, nnew, nnew_deg, (int64_t)ex);
+            close_totals(c, nnew, nnew_deg, (int64_t)mx);
             s.s_new = nnew;
             s.s_new_deg = nnew_deg;
             s.s_dir = sd;
@@ -1409,8 +1428,7 @@ __device__ __forceinline__ bool rebuild_state(const step_args &a, step_smem<BLOC
 }
 
 // Second half of the rebuild: the direction of the step.
-template <int BLOCK>
-__device__ __forceinline__ void rebuild_dir(const step_args &a, step_smem<BLOCK> &s) {
+__device__ __forceinline__ void rebuild_dir(const step_args &a, step_state &s) {
     if (s.s_dir != kDirTDWrite) {
         // the remote-write steps of REMOTE_WRITES_HYBRID are its bottom-up
         // phase (hybrid_bfs.cc:262-268)
@@ -1427,8 +1445,7 @@ __device__ __forceinline__ void rebuild_dir(const step_args &a, step_smem<BLOCK>
 // choose_dir may consult it: after a top-down step within the factor mlp_near
 // of the switch, or a bottom-up step that Beamer's rules may leave.  The
 // operands (6 KB a workgroup) are loaded only then.
-template <int BLOCK>
-__device__ __forceinline__ void predict_costs(const step_args &a, step_smem<BLOCK> &s) {
+__device__ __forceinline__ void predict_costs(const step_args &a, step_state &s) {
     const step_close &p = s.pre;
     const int l = lane_id();
     const int64_t nn = p.nnew, nd = p.nnew_deg;
@@ -1469,8 +1486,7 @@ __device__ __forceinline__ void clear_lines(seg_line *ln, int l) {
 // copies once the search is done, so later launches see it), and clear the
 // lines the next step fills, [(L+2)%3], which nobody reads or writes during
 // step L.
-template <int BLOCK>
-__device__ __forceinline__ void publish_state(const step_args &a, step_smem<BLOCK> &s) {
+__device__ __forceinline__ void publish_state(const step_args &a, step_state &s) {
     const int L = a.level;
     const int l = lane_id();
     seg_counters *g = a.seg;
@@ -1499,6 +1515,7 @@ __device__ __forceinline__ void publish_state(const step_args &a, step_smem<BLOC
             a.res->t_start = g->t_start;
             a.res->t_end = g->t_end;
             a.res->task_overflow = g->task_overflow;
+            a.res->launch = L;
         }
         __threadfence_system();
         wave_lds_sync();
@@ -1601,6 +1618,336 @@ __global__ __launch_bounds__(BLOCK) void k_step(step_args a) {
             bu_body<BLOCK>(a, s, cnt, dsum, dmax, exam);
     }
     block_flush_counters<BLOCK>(a, s, cnt, dsum, exam, dmax);
+}
+
+// ---------------------------------------------------------- small frontiers
+
+// Steps of small frontiers, many in one launch: a launch per level costs its
+// start and end, every workgroup's read of the state and counters and a scan
+// of the frontier bitmap, 9.3 us on a 701 x 1024 lattice whatever the
+// frontier, and the lattice has 1300 levels of some 550 vertices.  Here one
+// workgroup keeps the visited bitmap in LDS, and the frontier with a slot for
+// each of its edges; a level is one chain of dependent loads (slot, neighbour,
+// the found vertex's list bounds), a barrier and the closing of the step by
+// the first wave, in registers: 3.9 us, of which two are the loads (that
+// lattice 12.1 -> 4.9 ms, one of 30 x 900 5.9 -> 1.15 ms, a path of 200 k
+// vertices 8.6 -> 1.4 us a level).
+//
+// k_solo goes before the step launch of level L (L > 0) and rewrites what that
+// launch reads -- the state before step L-1, its counters, the depth-L bitmap
+// -- into that of the last step it ran, so k_step needs to know nothing of it;
+// where the step is not one it takes, it changes nothing.  A frontier is taken
+// while it is top-down, fits the LDS arrays, and has no list that one lane
+// would spend long on.
+constexpr int kSoloBlock = 1024;
+constexpr int kSoloItems = 2048;  // frontier vertices
+constexpr int kSoloEdges = 6144;  // their edges
+constexpr int kSoloDeg = 64;      // entries of the longest list
+constexpr int kSoloRounds = 3;    // edges a lane has in flight
+// Words of a graph that runs k_solo: its visited bitmap has to fit in LDS
+// beside the frontiers.  Claims by global atomics, 64 requests to L2 from one
+// compute unit a wave, left a level at 9.2 us and a lattice of 1.5 M vertices
+// where it was.
+constexpr int kSoloWords = 12800;
+constexpr int kSoloSteps = 1 << 14;  // steps of one launch
+constexpr int kRecWords = (int)(sizeof(bd_level_rec) / 8);
+
+struct solo_smem : step_state {
+    uint64_t vis[kSoloWords];
+    int32_t v[2][kSoloItems];
+    uint32_t rel[2][kSoloItems];     // list's start less the vertex's first slot
+    uint16_t owner[2][kSoloEdges];   // a slot's vertex
+    unsigned long long fill[3];      // of frontier i % 3: vertices << 32 | edges
+    uint32_t max_deg[3];
+    bd_level_rec rec;  // of the step just closed
+    int32_t go;
+};
+static_assert(sizeof(solo_smem) <= 160 * 1024, "LDS of a workgroup");
+
+__host__ __device__ __forceinline__ bool solo_fits(int64_t n, int64_t deg, int64_t max_deg) {
+    return n <= kSoloItems && deg <= kSoloEdges && max_deg <= kSoloDeg;
+}
+
+__host__ __device__ __forceinline__ bool solo_takes(const ctl_block *c) {
+    return c->dir == BD_DIR_TD && solo_fits(c->frontier, c->frontier_deg, c->max_frontier_deg);
+}
+
+// The lanes' newly found vertices (R a lane: list [b, b + d), d = 0 where not
+// won) join the frontier in buffer buf, counted in slot k; those the arrays
+// cannot hold go to the bitmap, and the counts then end the run.  (nnz < 2^32:
+// the degrees of a frontier sum to less.)  Wave-collective.
+template <int R>
+__device__ __forceinline__ void solo_push(const step_args &a, solo_smem &s, int buf, int k,
+                                          const bool (&won)[R], const int32_t (&u)[R],
+                                          const int64_t (&b)[R], const uint32_t (&d)[R]) {
+    const int lane = lane_id();
+    uint64_t mine = 0;  // vertices << 32 | edges
+    uint32_t mx = 0;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        mine += ((uint64_t)won[r] << 32) + d[r];
+        mx = d[r] > mx ? d[r] : mx;
+    }
+    if (!__ballot(mine != 0)) return;
+    const uint64_t incl = wave_scan64(mine, [](uint64_t p, uint64_t q) { return p + q; });
+    const uint64_t total = lane63(incl);
+    mx = wave_max32(mx);
+    unsigned long long at = 0;
+    if (lane == 0) {
+        at = atomicAdd(&s.fill[k], (unsigned long long)total);
+        atomicMax(&s.max_deg[k], mx);
+    }
+    at = (unsigned long long)lane_bcast((int64_t)at, 0) + incl - mine;
+    uint32_t i = (uint32_t)(at >> 32), slot = (uint32_t)at;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        if (!won[r]) continue;
+        if (i >= kSoloItems) {
+            atomicOr((unsigned long long *)a.front + (u[r] >> 6), 1ULL << (u[r] & 63));
+        } else {
+            s.v[buf][i] = u[r];
+            s.rel[buf][i] = (uint32_t)b[r] - slot;
+            if (d[r] <= kSoloDeg && slot + d[r] <= kSoloEdges)
+                for (uint32_t j = 0; j < d[r]; ++j) s.owner[buf][slot + j] = (uint16_t)i;
+        }
+        ++i;
+        slot += d[r];
+    }
+}
+
+// Visit R edges a lane, slots e0 + lane + 1024 r of the frontier in buffer cur;
+// what they find is the next frontier, counted in slot kn.  Lanes past the
+// last slot read its edge again, so that no load waits behind a branch.
+template <int R>
+__device__ __forceinline__ void solo_visit(const step_args &a, solo_smem &s, int cur, int kn,
+                                           uint32_t e0, uint32_t edges) {
+    typedef int64_t bounds __attribute__((ext_vector_type(2), aligned(8)));
+    bool won[R];
+    int32_t u[R], src[R];
+    uint32_t d[R];
+    int64_t b[R];
+    bounds be[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const uint32_t i = e0 + r * kSoloBlock + lane_id();
+        won[r] = i < edges;
+        d[r] = won[r] ? i : edges - 1;
+        src[r] = s.owner[cur][d[r]];
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        d[r] += s.rel[cur][src[r]];
+        src[r] = s.v[cur][src[r]];
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) u[r] = a.cols[d[r]];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        if (!won[r]) continue;
+        const uint32_t bit = 1u << (u[r] & 31);
+        won[r] = !(atomicOr((unsigned int *)s.vis + (u[r] >> 5), bit) & bit);
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+        if (won[r]) be[r] = *(const bounds *)(a.off + u[r]);
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        b[r] = 0;
+        d[r] = 0;
+        if (won[r]) {
+            a.parent[u[r]] = src[r];
+            b[r] = be[r].x;
+            d[r] = (uint32_t)(be[r].y - be[r].x);
+        }
+    }
+    solo_push(a, s, cur ^ 1, kn, won, u, b, d);
+}
+
+// What top-down steps change of the search state, in scalar registers of the
+// first wave.
+struct solo_state {
+    int64_t edges_to_check, scout, frontier, frontier_deg, max_deg, unvisited, unvisited_deg,
+        reached, reached_deg, steps;
+};
+
+__global__ __launch_bounds__(kSoloBlock) void k_solo(step_args a) {
+    __shared__ solo_smem s;
+    const int L = a.level, tid = threadIdx.x, lane = tid & 63;
+    const int wid = lane_bcast(tid >> 6, 0);
+    if (wid == 0) {
+        const bool was_done = rebuild_state(a, s, true);
+        if (!was_done) rebuild_dir(a, s);
+        if (lane == 0) s.go = !was_done && !s.st.done && solo_takes(&s.st);
+    }
+    if (tid < 3) {
+        s.fill[tid] = 0;
+        s.max_deg[tid] = 0;
+    }
+    __syncthreads();
+    if (!s.go) return;
+    // the frontier, out of its bitmap
+    uint64_t *front = (uint64_t *)a.front;
+    for (int64_t w0 = wid * 64; w0 < a.live_nwords; w0 += 4 * kSoloBlock) {
+        uint64_t x[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int64_t w = w0 + r * kSoloBlock + lane;
+            x[r] = w < a.live_nwords ? front[w] : 0;
+            if (w < a.live_nwords) s.vis[w] = a.vis[w];
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int64_t w = w0 + r * kSoloBlock + lane;
+            if (x[r]) front[w] = 0;
+            while (__ballot(x[r] != 0)) {
+                const bool won[1] = {x[r] != 0};
+                const int32_t u[1] = {
+                    won[0] ? (int32_t)(w * 64 + __ffsll((unsigned long long)x[r]) - 1) : 0};
+                const int64_t b[1] = {a.off[u[0]]};
+                const uint32_t d[1] = {won[0] ? (uint32_t)(a.off[u[0] + 1] - b[0]) : 0};
+                solo_push(a, s, 0, 0, won, u, b, d);
+                x[r] &= x[r] - 1;
+            }
+        }
+    }
+    __threadfence();  // the cleared words, before bits are set in them again
+    __syncthreads();
+    // the state before the step being run
+    const ctl_block *c = &s.st;
+    solo_state st = {lane_bcast(c->edges_to_check, 0), lane_bcast(c->scout, 0),
+                     lane_bcast(c->frontier, 0),       lane_bcast(c->frontier_deg, 0),
+                     lane_bcast(c->max_frontier_deg, 0), lane_bcast(c->unvisited, 0),
+                     lane_bcast(c->unvisited_deg, 0),  lane_bcast(c->reached, 0),
+                     lane_bcast(c->reached_deg, 0),    lane_bcast(c->steps, 0)};
+    const int64_t alpha = lane_bcast(c->alpha, 0);
+    const int64_t split = a.policy != BD_POLICY_TD_ONLY && a.td_split > 0 ? a.td_split : 1LL << 62;
+    int cur = 0, k = 0, closed = 0;  // steps closed
+    // the first wave has the least of the edges, as it closes the step
+    const int ew = wid == 0 ? kSoloBlock / 64 - 1 : wid - 1;
+    for (;;) {
+        const uint32_t edges = (uint32_t)lane_bcast((int32_t)(uint32_t)s.fill[k], 0);
+        const int kn = k == 2 ? 0 : k + 1;
+        // rounds of 1024 edges together, as many as this wave has (a round
+        // past the end costs the loads' issue all the same)
+        for (uint32_t e0 = ew * 64; e0 < edges; e0 += kSoloRounds * kSoloBlock) {
+            if (e0 + 2 * kSoloBlock < edges)
+                solo_visit<kSoloRounds>(a, s, cur, kn, e0, edges);
+            else if (e0 + kSoloBlock < edges)
+                solo_visit<2>(a, s, cur, kn, e0, edges);
+            else
+                solo_visit<1>(a, s, cur, kn, e0, edges);
+        }
+        __syncthreads();
+        if (wid == 0) {
+            const uint64_t f = (uint64_t)lane_bcast((int64_t)s.fill[kn], 0);
+            const int64_t nn = (int64_t)(f >> 32), nd = (int64_t)(uint32_t)f;
+            const int64_t mx = lane_bcast((int32_t)s.max_deg[kn], 0);
+            // close the step if the next is one to take as well
+            ctl_block t;
+            t.alpha = alpha;
+            t.edges_to_check = st.edges_to_check;
+            t.scout = st.scout;
+            t.frontier = nn;
+            t.in_bu_loop = 0;
+            t.dir = BD_DIR_TD;
+            if (a.policy != BD_POLICY_TD_ONLY) beamer_next(a, &t, BD_DIR_TD, nn, nd);
+            const bool go = nn > 0 && solo_fits(nn, nd, mx) && t.dir == BD_DIR_TD && nd < split &&
+                            closed < kSoloSteps;
+            if (lane == 0) {
+                s.go = go;
+                const int kc = kn == 2 ? 0 : kn + 1;
+                s.fill[kc] = 0;
+                s.max_deg[kc] = 0;
+                bd_level_rec r;
+                r.level = st.steps;
+                r.dir = BD_DIR_TD;
+                r.frontier = st.frontier;
+                r.frontier_deg = st.frontier_deg;
+                r.unvisited = st.unvisited;
+                r.unvisited_deg = st.unvisited_deg;
+                r.edges_to_check = st.edges_to_check;
+                r.result = nd;
+                r.next = nn;
+                r.next_deg = nd;
+                r.edges_examined = st.frontier_deg;
+                r.max_frontier_deg = st.max_deg;
+                r.tasks = closed ? 0 : c->tpref[kSeg + 1];
+                r.queued = closed ? 0 : c->qpref[kSeg + 1];
+                r.ms = -1.0;
+                r.ms_other = -1.0;
+                r.launch = c->launches + closed;
+                r.launches = 1;
+                s.rec = r;
+            }
+            if (go) {
+                ++closed;
+                st.edges_to_check = t.edges_to_check;
+                st.scout = t.scout;
+                st.frontier = nn;
+                st.frontier_deg = nd;
+                st.max_deg = mx;
+                st.unvisited -= nn;
+                st.unvisited_deg -= nd;
+                st.reached += nn;
+                st.reached_deg += nd;
+                ++st.steps;
+            }
+        }
+        __syncthreads();
+        k = kn;
+        cur ^= 1;
+        if (!s.go) break;
+        // the record leaves from another wave, a word a lane
+        if (wid == kSoloBlock / 64 - 1 && lane < kRecWords && s.rec.level < a.log_cap) {
+            bd_level_rec *log = s.rec.level < kHostRecs ? a.hlog : a.log;
+            ((uint64_t *)(log + s.rec.level))[lane] = ((const uint64_t *)&s.rec)[lane];
+        }
+    }
+    // hand the last step over: its frontier in the bitmap, the state before
+    // it, its counts
+    const int n = (int)(s.fill[k] >> 32) < kSoloItems ? (int)(s.fill[k] >> 32) : kSoloItems;
+    for (int i = tid; i < n; i += kSoloBlock) {
+        const int32_t u = s.v[cur][i];
+        atomicOr((unsigned long long *)front + (u >> 6), 1ULL << (u & 63));
+    }
+    for (int64_t w = tid; w < a.live_nwords; w += kSoloBlock) a.vis[w] = s.vis[w];
+    if (wid == 0) {
+        if (lane == 0) {
+            ctl_block *h = &s.st;
+            h->td_nolist = 1;
+            if (closed) {
+                h->edges_to_check = st.edges_to_check;
+                h->scout = st.scout;
+                h->frontier = st.frontier;
+                h->frontier_deg = st.frontier_deg;
+                h->max_frontier_deg = st.max_deg;
+                h->unvisited = st.unvisited;
+                h->unvisited_deg = st.unvisited_deg;
+                h->reached = st.reached;
+                h->reached_deg = st.reached_deg;
+                h->steps = st.steps;
+                h->level = (int32_t)st.steps;
+                h->td_steps += closed;
+                h->launches += closed;
+                h->prev_dir = BD_DIR_TD;
+                h->td_bitmap = 1;
+                h->qpref[kSeg + 1] = 0;
+                h->tpref[kSeg + 1] = 0;
+            }
+        }
+        wave_lds_sync();
+        const uint64_t *src = (const uint64_t *)&s.st;
+        uint64_t *dst = (uint64_t *)&a.c[(L - 1) & 1];
+        for (int i = lane; i < kCtlWords; i += 64) dst[i] = src[i];
+        seg_line *ln = a.seg->line[L % 3];
+        clear_lines(ln, lane);
+        wave_lds_sync();
+        if (lane == 0) {
+            ln[0].acc[0] = s.fill[k] >> 32;
+            ln[0].acc[1] = (uint32_t)s.fill[k];
+            ln[0].acc[3] = s.max_deg[k];
+        }
+    }
 }
 
 // Start a search: clear() (hybrid_bfs.cc:433-443) has been done by k_clear;
@@ -2193,6 +2540,21 @@ int close_level(bd_ctx *c, const step_args &a) {
     return read_ctl(c);
 }
 
+// k_solo before the step launches of a device-driven search: plain searches
+// that are not timed launch by launch.
+bool solo_allowed(const bd_ctx *c, const step_args &a) {
+    return c->tune.time_steps == 2 && c->tune.step_kernels == 2 && c->nnz < (1LL << 32) &&
+           a.live_nwords <= kSoloWords &&
+           (a.policy == BD_POLICY_BEAMER || a.policy == BD_POLICY_TD_ONLY ||
+            (a.policy == BD_POLICY_LEARNED && !a.has_mlp));
+}
+
+int launch_solo(bd_ctx *c, const step_args &a) {
+    hipLaunchKernelGGL(k_solo, dim3(1), dim3(kSoloBlock), 0, c->stream, a);
+    BD_HIP(c, hipGetLastError());
+    return BD_OK;
+}
+
 int launch_init(bd_ctx *c, const step_args &a, int64_t source, const int64_t *srcs,
                 int64_t nsrc, hipEvent_t stop = nullptr) {
     if (stop)  // stamped when k_init ends, i.e. when the first step starts
@@ -2336,9 +2698,16 @@ int run_search(bd_ctx *c, int64_t source, int64_t alpha, int64_t beta, int polic
         // graph took, and a few more (16 for the first search); launches
         // past the end return at once but still occupy the device
         int chunk = c->chunk_hint > 0 ? c->chunk_hint : 16;
+        // A graph without long lists may be one of many small levels (a
+        // lattice, a path): k_solo after its first.  Later it goes before
+        // every step of a chunk that starts from a frontier it takes.
+        const bool solo_ok = solo_allowed(c, make_args(c, 0, alpha, beta, policy));
+        bool every = false;
         for (;;) {
             for (int k = 0; k < chunk; ++k, ++L) {
                 const step_args a = make_args(c, L, alpha, beta, policy);
+                if (every || (solo_ok && L == 1 && c->max_deg <= kSoloDeg))
+                    if ((rc = launch_solo(c, a))) return rc;
                 hipEvent_t e0 = nullptr, e1 = nullptr;
                 if (per_launch) {
                     e0 = c->ev_pool[2 * k];
@@ -2366,6 +2735,12 @@ int run_search(bd_ctx *c, int64_t source, int64_t alpha, int64_t beta, int polic
             if (search_done(c)) break;
             if (L > max_levels) return set_err(c, BD_EHIP, "search did not terminate");
             chunk = std::min(chunk * 2, kMaxLevelsPerSync);
+            if (solo_ok) {
+                if ((rc = read_ctl(c))) return rc;
+                const ctl_block &h = c->h_ctl[c->h_ctl[1].steps > c->h_ctl[0].steps];
+                every = solo_takes(&h);
+                if (every) chunk = 8;
+            }
         }
     }
     const double host_ms = std::chrono::duration<double, std::milli>(
@@ -2373,9 +2748,8 @@ int run_search(bd_ctx *c, int64_t source, int64_t alpha, int64_t beta, int polic
                                .count();
     if ((rc = finish_search(c, source, out, host_ms))) return rc;
     if (!c->last_log.empty() && (int64_t)c->last_log.size() == c->last_steps) {
-        const bd_level_rec &r = c->last_log.back();
         // its level launches and the launch that found the frontier empty
-        const int64_t used = r.launch + r.launches + 1;
+        const int64_t used = (int64_t)c->h_res->launch + 1;
         c->chunk_hint = (int)std::min<int64_t>(std::max<int64_t>(used + 3, 4), kMaxLevelsPerSync);
     }
     if (c->tune.time_steps == 3) step_ms = c->last_launch_ms;  // per-launch times only

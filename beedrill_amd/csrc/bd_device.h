@@ -71,6 +71,17 @@ __device__ __forceinline__ unsigned long long wave_max(unsigned long long x) {
     return lane63(wave_scan64(x, [](uint64_t p, uint64_t q) { return p > q ? p : q; }));
 }
 
+__device__ __forceinline__ uint32_t wave_max32(uint32_t x) {
+    const auto up = [](uint32_t p, uint32_t q) { return p > q ? p : q; };
+    x = up(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xf, 0xf, true));
+    x = up(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xf, 0xf, true));
+    x = up(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xf, 0xf, true));
+    x = up(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xf, 0xf, true));
+    x = up(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xa, 0xf, true));
+    x = up(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xc, 0xf, true));
+    return (uint32_t)__builtin_amdgcn_readlane((int)x, 63);
+}
+
 __device__ __forceinline__ unsigned long long wave_min(unsigned long long x) {
     return lane63(wave_scan64(x, [](uint64_t p, uint64_t q) { return p < q ? p : q; }));
 }

@@ -109,6 +109,7 @@ struct ctl_block {
     int64_t bu_steps;
     int64_t reached;
     int64_t reached_deg;
+    int64_t launches;  // step launches so far (a step run by k_solo counts as one)
 };
 
 // Step records the device writes straight to host memory; a deeper search's
@@ -127,6 +128,7 @@ struct search_result {
     ctl_block ctl;
     unsigned long long task_overflow;
     uint64_t t_start, t_end;
+    int32_t launch;  // the launch that found the search done
     uint32_t seq;
 };
 

@@ -87,7 +87,8 @@ typedef struct {
     int64_t queued;           /* F's other vertices, read from the queue   */
     double ms;                /* device time of the step (timed runs only) */
     double ms_other;          /* profile runs: time of the other direction */
-    int64_t launch;           /* index of the step's first kernel launch   */
+    int64_t launch;           /* index of the step's first kernel launch (a
+                                 step that shares one counts as one)       */
     int64_t launches;         /* its launches: 1, or 2 for a top-down step
                                  run with remote writes                    */
 } bd_level_rec;

@@ -964,3 +964,77 @@ def test_depths_on_both_sides_of_a_byte(ctx, orc, length):
     rows = ctx.multi_root([0, 3])[0]
     np.testing.assert_array_equal(rows[0], want)
     np.testing.assert_array_equal(rows[1], np.where(want < 0, -1, abs(want - 3)))
+
+
+def bundle_graph(paths, length, fan=16):
+    """A tree of fan-out `fan` whose `paths` last-level vertices each start a
+    path of `length` vertices: frontiers of exactly `paths` from there on."""
+    src, dst, row, nv = [], [], [0], 1
+    while len(row) < paths:
+        want = min(paths, fan * len(row))
+        kids = np.arange(nv, nv + want)
+        src.append(np.asarray(row)[np.arange(want) * len(row) // want])
+        dst.append(kids)
+        nv += want
+        row = kids
+    for _ in range(length):
+        kids = np.arange(nv, nv + paths)
+        src.append(np.asarray(row))
+        dst.append(kids)
+        nv += paths
+        row = kids
+    return nv, np.concatenate(src), np.concatenate(dst)
+
+
+@pytest.mark.parametrize("policy,alpha", [("beamer", 15), ("beamer", 1 << 40), ("td_only", 15),
+                                          ("learned", 3)])
+@pytest.mark.parametrize("paths", [1, 63, 64, 65, 1025, 2047, 2048, 2049, 3100])
+def test_small_frontiers_on_both_sides_of_the_solo_rule(ctx, orc, paths, policy, alpha):
+    """Steps run many to a launch (up to 2048 vertices and 6144 edges), and
+    handed over where the frontier outgrows that or turns bottom-up: depths,
+    parents and step records are the oracle's."""
+    nv, s, d = bundle_graph(paths, 40)
+    off, adj, m = oracle_csr(orc, nv, s, d)
+    ctx.upload_csr(off, adj, m)
+    for root in (0, nv - 1, nv // 2):
+        for _ in range(2):  # the second search queues as many launches as the first needed
+            run_and_compare(ctx, orc, off, adj, m, root, policy=policy, alpha=alpha)
+            if policy == "td_only":
+                _, ref = orc.td_only(off, adj, m, root)
+                np.testing.assert_array_equal(ctx.fetch()[0], ref)
+            assert _launches_follow(ctx.levels())
+
+
+@pytest.mark.parametrize("leaves", [0, 60, 61, 62, 63, 64, 300, 9000])
+def test_small_frontiers_with_long_lists(ctx, orc, leaves):
+    """A path of 700 with a vertex of `leaves` leaves at 90 and at 500: lists
+    of up to 64 entries are walked within the launch, longer ones are not."""
+    n = 700
+    s = [np.arange(n - 1)]
+    d = [np.arange(1, n)]
+    for k, at in enumerate((90, 500)):
+        s.append(np.full(leaves, at))
+        d.append(np.arange(n + k * leaves, n + (k + 1) * leaves))
+    nv = n + 2 * leaves + 5
+    off, adj, m = oracle_csr(orc, nv, np.concatenate(s), np.concatenate(d))
+    ctx.upload_csr(off, adj, m)
+    for root in (0, 300, n - 1):
+        for alpha in (15, 1 << 40):
+            run_and_compare(ctx, orc, off, adj, m, root, alpha=alpha)
+            assert _launches_follow(ctx.levels())
+
+
+@pytest.mark.parametrize("rows,cols", [(799, 1024), (800, 1024), (801, 1024), (1024, 900)])
+def test_lattices_on_both_sides_of_the_solo_bitmap(ctx, orc, rows, cols):
+    """A visited bitmap of up to 12800 words is kept in LDS."""
+    ctx.generate_lattice(rows, cols)
+    off, adj = ctx.csr()
+    for root in (0, rows * cols // 2 + 7):
+        st = ctx.bfs(root)
+        depth, parent = ctx.fetch()
+        np.testing.assert_array_equal(depth, orc.bfs_depth(off, adj, root))
+        assert orc.check(off, adj, root, parent)
+        lv = ctx.levels()
+        np.testing.assert_array_equal([r["frontier"] for r in lv], np.bincount(depth[depth >= 0]))
+        assert st["steps"] == len(lv) and st["reached"] == (depth >= 0).sum()
+        assert [r["level"] for r in lv] == list(range(len(lv)))
