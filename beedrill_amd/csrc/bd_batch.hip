@@ -653,8 +653,8 @@ int ms_buffers(bd_ctx *c, int nrows) {
     }
     if (!c->d_ms_hubs || c->ms_hub_order != c->s_order) {
         // the hubs of the search layout, once per graph and layout
-        dev_free(c->d_ms_hubs);
-        dev_free(c->d_ms_hub_slices);
+        dev_free(c, c->d_ms_hubs);
+        dev_free(c, c->d_ms_hub_slices);
         c->d_ms_hubs = nullptr;
         c->d_ms_hub_slices = nullptr;
         const int64_t max_hubs = c->nnz / kMsHubDeg + 1;
@@ -676,7 +676,7 @@ int ms_buffers(bd_ctx *c, int nrows) {
         c->ms_hub_order = c->s_order;
     }
     if (nrows > c->ms_depth_rows) {
-        dev_free(c->d_ms_depth);
+        dev_free(c, c->d_ms_depth);
         c->d_ms_depth = nullptr;
         c->ms_depth_rows = 0;
         if ((rc = dev_alloc(c, (void **)&c->d_ms_depth, sizeof(int32_t) * c->nv * nrows,
@@ -724,9 +724,10 @@ int run_multi_root(bd_ctx *c, const int64_t *roots, int n, int32_t *depths, doub
     int64_t *d_roots = nullptr;
     if ((rc = dev_alloc(c, (void **)&d_roots, sizeof(int64_t) * n, "roots"))) return rc;
     struct guard {
+        bd_ctx *c;
         void *p;
-        ~guard() { dev_free(p); }
-    } g{d_roots};
+        ~guard() { dev_free(c, p); }
+    } g{c, d_roots};
     const int64_t nv = c->nv;
     ms_args a;
     a.off = c->d_soff;

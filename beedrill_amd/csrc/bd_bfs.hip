@@ -2774,7 +2774,7 @@ extern "C" int bd_bfs_run(bd_ctx *c, int64_t source, int64_t alpha, int64_t beta
 extern "C" int bd_bfs_set_script(bd_ctx *c, const int32_t *dirs, int64_t n) {
     if (!c || n < 0 || (n > 0 && !dirs)) return BD_EINVAL;
     BD_HIP(c, hipSetDevice(c->device));
-    dev_free(c->d_script);
+    dev_free(c, c->d_script);
     c->d_script = nullptr;
     c->script_len = 0;
     if (n == 0) return BD_OK;
@@ -2968,7 +2968,7 @@ extern "C" int bd_bfs_count_traversed(bd_ctx *c, int64_t *out) {
     }
     if (e == hipSuccess) e = hipMemcpyAsync(h.data(), d, bytes, hipMemcpyDeviceToHost, c->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-    dev_free(d);
+    dev_free(c, d);
     if (e != hipSuccess) return hip_err(c, e, "count_traversed");
     unsigned long long sum = 0;
     for (int s = 0; s < kSlots; ++s) sum += h[s * kLine];
@@ -3050,9 +3050,10 @@ extern "C" int bd_bfs_profile(bd_ctx *c, int64_t source, int64_t alpha, int64_t 
     uint4 *scrub = nullptr;
     if ((rc = dev_alloc(c, (void **)&scrub, sizeof(uint4) * (scrub_n + 1), "scrub"))) return rc;
     struct guard {
+        bd_ctx *c;
         uint4 *p;
-        ~guard() { dev_free(p); }
-    } g{scrub};
+        ~guard() { dev_free(c, p); }
+    } g{c, scrub};
     BD_HIP(c, hipMemsetAsync(scrub, 0, sizeof(uint4) * (scrub_n + 1), c->stream));
     if ((rc = start_search(c, source, alpha, beta, policy))) return rc;
     if ((rc = read_ctl(c))) return rc;
@@ -3183,9 +3184,10 @@ extern "C" int bd_bfs_multi_graph(bd_ctx *c, int ngraphs, const int64_t *vbase,
                         "batch sources")))
         return rc;
     struct guard {
+        bd_ctx *c;
         void *p;
-        ~guard() { dev_free(p); }
-    } gd{d};
+        ~guard() { dev_free(c, p); }
+    } gd{c, d};
     int64_t *d_src = d, *d_vbase = d + ngraphs;
     int *d_bad = (int *)(d + 2 * ngraphs + 1);
     BD_HIP(c, hipMemcpy(d_src, src.data(), sizeof(int64_t) * ngraphs, hipMemcpyHostToDevice));

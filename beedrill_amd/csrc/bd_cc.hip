@@ -394,7 +394,7 @@ extern "C" int bd_cc_run(bd_ctx *c, bd_cc_stats *out) {
         // indexes, outside the timed run; its time and memory are reported)
         BD_HIP(c, hipEventRecord(c->ev[0], c->stream));
         const int64_t cap = c->nnz / kCcSlice + c->nnz / kCcHeavy + 1;
-        dev_free(c->d_cc_tasks);  // left by a build that failed part-way
+        dev_free(c, c->d_cc_tasks);  // left by a build that failed part-way
         c->d_cc_tasks = nullptr;
         if ((rc = dev_alloc(c, (void **)&c->d_cc_tasks, sizeof(td_task) * cap, "component slices")))
             return rc;

@@ -238,8 +238,9 @@ __global__ void k_unpack(const uint64_t *__restrict__ el, int64_t m, int64_t *__
 }
 
 struct dev_buf {
+    bd_ctx *c;
     void *p = nullptr;
-    ~dev_buf() { dev_free(p); }
+    ~dev_buf() { dev_free(c, p); }
     template <class T>
     T *as() const {
         return (T *)p;
@@ -255,7 +256,7 @@ int sort_keys_u64(bd_ctx *c, const uint64_t *in, uint64_t *out, int64_t n, int b
     size_t tmp = 0;
     BD_HIP(c, rocprim::radix_sort_keys(nullptr, tmp, in, out, (size_t)n, 0, (unsigned)bits,
                                        c->stream));
-    dev_buf t;
+    dev_buf t{c};
     int rc = dev_alloc(c, &t.p, tmp, "sort temp");
     if (rc) return rc;
     BD_HIP(c, rocprim::radix_sort_keys(t.p, tmp, in, out, (size_t)n, 0, (unsigned)bits, c->stream));
@@ -268,7 +269,7 @@ int sort_pairs(bd_ctx *c, const K *kin, K *kout, const V *vin, V *vout, int64_t 
     size_t tmp = 0;
     BD_HIP(c, rocprim::radix_sort_pairs(nullptr, tmp, kin, kout, vin, vout, (size_t)n, 0,
                                         (unsigned)bits, c->stream));
-    dev_buf t;
+    dev_buf t{c};
     int rc = dev_alloc(c, &t.p, tmp, "sort temp");
     if (rc) return rc;
     BD_HIP(c, rocprim::radix_sort_pairs(t.p, tmp, kin, kout, vin, vout, (size_t)n, 0,
@@ -278,13 +279,13 @@ int sort_pairs(bd_ctx *c, const K *kin, K *kout, const V *vin, V *vout, int64_t 
 }
 
 int unique_u64(bd_ctx *c, const uint64_t *in, uint64_t *out, int64_t n, int64_t *m) {
-    dev_buf cnt;
+    dev_buf cnt{c};
     int rc = dev_alloc(c, &cnt.p, sizeof(size_t), "unique count");
     if (rc) return rc;
     size_t tmp = 0;
     BD_HIP(c, rocprim::unique(nullptr, tmp, in, out, cnt.as<size_t>(), (size_t)n,
                               rocprim::equal_to<uint64_t>(), c->stream));
-    dev_buf t;
+    dev_buf t{c};
     if ((rc = dev_alloc(c, &t.p, tmp, "unique temp"))) return rc;
     BD_HIP(c, rocprim::unique(t.p, tmp, in, out, cnt.as<size_t>(), (size_t)n,
                               rocprim::equal_to<uint64_t>(), c->stream));
@@ -307,7 +308,7 @@ __global__ void k_shuffle_keys(int64_t m, uint64_t seed, uint64_t *__restrict__ 
 // buffer is caller-owned and is reused as scratch.
 int finish_edges(bd_ctx *c, uint64_t *in, int64_t m, int s, int64_t nv, bool relabel,
                  uint64_t seed, bool packed_input) {
-    dev_buf skeys, packed;
+    dev_buf skeys{c}, packed{c};
     int rc;
     if ((rc = dev_alloc(c, &skeys.p, sizeof(uint64_t) * m, "shuffle keys"))) return rc;
     if ((rc = dev_alloc(c, &packed.p, sizeof(uint64_t) * m, "packed edges"))) return rc;
@@ -324,7 +325,7 @@ int finish_edges(bd_ctx *c, uint64_t *in, int64_t m, int s, int64_t nv, bool rel
                            packed.as<uint64_t>());
     }
     BD_HIP(c, hipGetLastError());
-    dev_free(c->d_el);
+    dev_free(c, c->d_el);
     c->d_el = nullptr;
     if ((rc = dev_alloc(c, (void **)&c->d_el, sizeof(uint64_t) * m, "edge list"))) return rc;
     // `in` is no longer needed: it receives the sorted shuffle keys
@@ -337,13 +338,13 @@ int finish_edges(bd_ctx *c, uint64_t *in, int64_t m, int s, int64_t nv, bool rel
 int build_csr_from_el(bd_ctx *c, int64_t nv, int64_t m) {
     // c->d_el holds m packed edges in el64 order.
     const int64_t n2 = 2 * m;
-    dev_buf keys, vals, skeys;
+    dev_buf keys{c}, vals{c}, skeys{c};
     int rc;
     free_search_layout(c);
-    dev_free(c->d_off);
-    dev_free(c->d_cols);
-    dev_free(c->d_dead);
-    dev_free(c->d_head);
+    dev_free(c, c->d_off);
+    dev_free(c, c->d_cols);
+    dev_free(c, c->d_dead);
+    dev_free(c, c->d_head);
     c->d_off = nullptr;
     c->d_cols = nullptr;
     c->d_dead = nullptr;
@@ -595,16 +596,16 @@ __global__ void k_heads_across(const int64_t *__restrict__ off, const int32_t *_
 
 void free_search_layout(bd_ctx *c) {
     if (c->d_perm) {  // renumbered: the layout owns its arrays
-        dev_free(c->d_soff);
-        dev_free(c->d_scols);
-        dev_free(c->d_sdead);
+        dev_free(c, c->d_soff);
+        dev_free(c, c->d_scols);
+        dev_free(c, c->d_sdead);
     }
-    dev_free(c->d_perm);
-    dev_free(c->d_inv);
-    dev_free(c->d_head);
-    dev_free(c->d_hub_bm);
-    dev_free(c->d_hub_med);
-    dev_free(c->d_hub_big);
+    dev_free(c, c->d_perm);
+    dev_free(c, c->d_inv);
+    dev_free(c, c->d_head);
+    dev_free(c, c->d_hub_bm);
+    dev_free(c, c->d_hub_med);
+    dev_free(c, c->d_hub_big);
     c->d_hub_bm = nullptr;
     c->d_hub_med = nullptr;
     c->d_hub_big = nullptr;
@@ -623,7 +624,7 @@ void free_search_layout(bd_ctx *c) {
 static int build_hubs(bd_ctx *c) {
     const int64_t nnz = c->nnz;
     int rc;
-    dev_buf cnt;
+    dev_buf cnt{c};
     if ((rc = dev_alloc(c, &cnt.p, 2 * sizeof(unsigned long long), "hub counts"))) return rc;
     if ((rc = dev_alloc(c, (void **)&c->d_hub_bm, sizeof(uint64_t) * c->nwords, "hub bitmap")))
         return rc;
@@ -679,7 +680,7 @@ int build_search_layout(bd_ctx *c) {
     free_search_layout(c);
     const int64_t nv = c->nv, nnz = c->nnz;
     int rc;
-    dev_buf keys, skeys, sdeg, cnt, tmp, rec;
+    dev_buf keys{c}, skeys{c}, sdeg{c}, cnt{c}, tmp{c}, rec{c};
     if ((rc = dev_alloc(c, &cnt.p, 2 * sizeof(unsigned long long), "degree counts"))) return rc;
     BD_HIP(c, hipMemsetAsync(cnt.p, 0, 2 * sizeof(unsigned long long), c->stream));
     hipLaunchKernelGGL(k_degree_stats, dim3(std::min<int64_t>(grid1d(c, nv), c->cu_count)),
@@ -770,7 +771,7 @@ extern "C" int bd_graph_upload(bd_ctx *c, const int64_t *off, const int32_t *col
         return rc;
     BD_HIP(c, hipMemcpy(c->d_off, off, sizeof(int64_t) * (nv + 1), hipMemcpyHostToDevice));
     if (nnz) BD_HIP(c, hipMemcpy(c->d_cols, cols, sizeof(int32_t) * nnz, hipMemcpyHostToDevice));
-    dev_buf err;
+    dev_buf err{c};
     if ((rc = dev_alloc(c, &err.p, sizeof(int), "flag"))) return rc;
     BD_HIP(c, hipMemsetAsync(err.p, 0, sizeof(int), c->stream));
     hipLaunchKernelGGL(k_validate_csr, dim3(grid1d(c, std::max(nv, nnz))), dim3(kBlock), 0,
@@ -815,7 +816,7 @@ extern "C" int bd_graph_from_edges(bd_ctx *c, const int64_t *src, const int64_t 
     free_graph(c);
     if ((rc = dev_alloc(c, (void **)&c->d_el, sizeof(uint64_t) * m, "edge list"))) return rc;
     const int64_t chunk = std::min<int64_t>(std::max<int64_t>(m, 1), (int64_t)1 << 24);
-    dev_buf stage, err;
+    dev_buf stage{c}, err{c};
     if ((rc = dev_alloc(c, &stage.p, sizeof(int64_t) * 2 * chunk, "staging"))) return rc;
     if ((rc = dev_alloc(c, &err.p, sizeof(int), "flag"))) return rc;
     BD_HIP(c, hipMemsetAsync(err.p, 0, sizeof(int), c->stream));
@@ -968,7 +969,7 @@ extern "C" int bd_graph_load_el64(bd_ctx *c, const char *path) {
     }
     const int64_t chunk = std::min<int64_t>(h.m, (int64_t)1 << 22);
     std::vector<int64_t> buf(2 * chunk), s(chunk), d(chunk);
-    dev_buf stage, err;
+    dev_buf stage{c}, err{c};
     if ((rc = dev_alloc(c, &stage.p, sizeof(int64_t) * 2 * chunk, "staging")) ||
         (rc = dev_alloc(c, &err.p, sizeof(int), "flag"))) {
         fclose(fp);
@@ -1019,7 +1020,7 @@ extern "C" int bd_graph_generate(bd_ctx *c, int kind, int64_t nv, int64_t num_ed
         if (cols <= 0 || nv % cols) return set_err(c, BD_EINVAL, "lattice: nv must be rows*cols");
         const int64_t rows = nv / cols;
         const int64_t m = rows * (cols - 1) + (rows - 1) * cols;
-        dev_buf el;
+        dev_buf el{c};
         if ((rc = dev_alloc(c, &el.p, sizeof(uint64_t) * std::max<int64_t>(m, 1), "lattice")))
             return rc;
         hipLaunchKernelGGL(k_lattice, dim3(grid1d(c, nv)), dim3(kBlock), 0, c->stream, rows, cols,
@@ -1033,7 +1034,7 @@ extern "C" int bd_graph_generate(bd_ctx *c, int kind, int64_t nv, int64_t num_ed
     if (kind == BD_GEN_RMAT && (nv & (nv - 1)))
         return set_err(c, BD_EINVAL, "RMAT needs a power-of-two vertex count");
     const int64_t ne = num_edges;
-    dev_buf A, B;
+    dev_buf A{c}, B{c};
     if ((rc = dev_alloc(c, &A.p, sizeof(uint64_t) * std::max<int64_t>(ne, 1), "raw edges")))
         return rc;
     if ((rc = dev_alloc(c, &B.p, sizeof(uint64_t) * std::max<int64_t>(ne, 1), "sorted edges")))
@@ -1042,7 +1043,7 @@ extern "C" int bd_graph_generate(bd_ctx *c, int kind, int64_t nv, int64_t num_ed
         const int scale = s;
         if (scale < 1) return set_err(c, BD_EINVAL, "RMAT needs nv >= 2");
         const int64_t self_cap = (int64_t)1 << 20;
-        dev_buf nself, sidx;
+        dev_buf nself{c}, sidx{c};
         if ((rc = dev_alloc(c, &nself.p, sizeof(unsigned long long), "self count")) ||
             (rc = dev_alloc(c, &sidx.p, sizeof(int64_t) * self_cap, "self index")))
             return rc;
@@ -1071,7 +1072,7 @@ extern "C" int bd_graph_generate(bd_ctx *c, int kind, int64_t nv, int64_t num_ed
                 } while (x == y);
                 val[k] = ((uint64_t)x << 32) | (uint64_t)y;
             }
-            dev_buf pv;
+            dev_buf pv{c};
             if ((rc = dev_alloc(c, &pv.p, sizeof(uint64_t) * hn, "patch"))) return rc;
             BD_HIP(c, hipMemcpy(sidx.p, idx.data(), sizeof(int64_t) * hn, hipMemcpyHostToDevice));
             BD_HIP(c, hipMemcpy(pv.p, val.data(), sizeof(uint64_t) * hn, hipMemcpyHostToDevice));
@@ -1108,7 +1109,7 @@ extern "C" int bd_graph_edges_download(bd_ctx *c, int64_t *src, int64_t *dst) {
     if (!c->d_el) return set_err(c, BD_ESTATE, "no edge list resident (graph was uploaded as CSR)");
     BD_HIP(c, hipSetDevice(c->device));
     const int64_t m = c->el_m;
-    dev_buf s, d;
+    dev_buf s{c}, d{c};
     int rc;
     if ((rc = dev_alloc(c, &s.p, sizeof(int64_t) * m, "unpack")) ||
         (rc = dev_alloc(c, &d.p, sizeof(int64_t) * m, "unpack")))

@@ -7,6 +7,7 @@
 
 #include <functional>
 #include <string>
+#include <unordered_map>
 #include <vector>
 
 #include "../../include/beedrill_amd.h"
@@ -132,6 +133,12 @@ struct search_result {
     uint32_t seq;
 };
 
+// Device memory a context has, or keeps for its next allocations.
+struct dev_block {
+    void *p;
+    size_t bytes;
+};
+
 }  // namespace bd
 
 struct bd_ctx {
@@ -140,6 +147,9 @@ struct bd_ctx {
     int64_t wall_khz = 100000;
     hipStream_t stream = nullptr;
     std::string err;
+    std::unordered_map<void *, size_t> live;  // dev_alloc's blocks
+    std::vector<bd::dev_block> pool;          // freed ones kept (dev_free)
+    size_t pool_bytes = 0;
 
     // graph (flat device CSR)
     int64_t nv = 0, nnz = 0, m = 0, nwords = 0;
@@ -260,7 +270,7 @@ int set_err(bd_ctx *c, int code, const std::string &msg);
 int hip_err(bd_ctx *c, hipError_t e, const char *what);
 // Allocate n bytes of device memory (zero-size requests allocate 256 B).
 int dev_alloc(bd_ctx *c, void **p, size_t bytes, const char *what);
-void dev_free(void *p);
+void dev_free(bd_ctx *c, void *p);
 // Release all graph-dependent buffers.
 void free_graph(bd_ctx *c);
 // (Re)allocate search buffers for the resident graph (and build its search

@@ -395,7 +395,7 @@ int check_mlp(bd_ctx *c) {
 // (a training run of 100 k samples) so that repeated calls allocate nothing.
 int mlp_ws(bd_ctx *c, size_t bytes, float **p) {
     if (c->mlp_ws_bytes < bytes) {
-        dev_free(c->d_mlp_ws);
+        dev_free(c, c->d_mlp_ws);
         c->d_mlp_ws = nullptr;
         c->mlp_ws_bytes = 0;
         int rc = dev_alloc(c, (void **)&c->d_mlp_ws, bytes, "network workspace");
@@ -410,7 +410,7 @@ struct mlp_ws_guard {
     bd_ctx *c;
     ~mlp_ws_guard() {
         if (c->mlp_ws_bytes <= ((size_t)16 << 20)) return;
-        dev_free(c->d_mlp_ws);
+        dev_free(c, c->d_mlp_ws);
         c->d_mlp_ws = nullptr;
         c->mlp_ws_bytes = 0;
     }
