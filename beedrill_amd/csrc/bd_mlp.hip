@@ -11,6 +11,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <type_traits>
 #include <vector>
 
 #include "bd_internal.h"
@@ -35,6 +36,7 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int kTrainWaves = 4;               // waves per workgroup, each with its own samples
 constexpr int kTrainBlock = 64 * kTrainWaves;
+constexpr int kTrainParams = kMaxParams / kTrainBlock + 1;  // a thread's (and the loss)
 constexpr int kTrainMaxGrid = 64;            // workgroups, i.e. partial gradients, of one pass
 constexpr int kPartStride = kMaxParams + 2;  // a workgroup's gradients, then its loss
 constexpr int kRow = 33;                     // LDS row stride: rows land on different banks
@@ -211,48 +213,90 @@ struct train_args {
 
 // Measured, 3038 samples: 1750 us a pass with a thread per sample and an LDS
 // atomic per sample and parameter (all lanes of a wave on one address); now
-// a launch's latency, the parameter update and ~110 MFMAs per wave.
+// a launch's latency, the parameter update and ~110 MFMAs per wave, 16.0 us
+// (27.4 with one parameter's partials loaded after another's and the waves'
+// gradients added up in turn).  All of a thread's parameters are loaded
+// together, up to 24 partials of each, and the first tile's samples before
+// them.  The update is still 6 us of it; twice the threads for it alone leave
+// the others half the registers, which spilled (21 us).
 __global__ __launch_bounds__(kTrainBlock) void k_mlp_train(train_args a) {
     __shared__ mlp_lds s;
     // per wave: activations and gradients of its samples, [sample][unit]
     __shared__ float A1[kTrainWaves][32 * kRow], A2[kTrainWaves][32 * kRow];
     __shared__ float D1[kTrainWaves][32 * kRow], D2[kTrainWaves][32 * kRow];
     __shared__ float X[kTrainWaves][32 * kMlpIn], DY[kTrainWaves][32 * 2];
-    __shared__ float red[kPartStride];
     const int tid = threadIdx.x, l = tid & 63, wid = tid >> 6;
     const int i = l & 31, q = l >> 5;
     const int np = (int)mlp_nparams(a.h1, a.h2);
     s.clear(tid, kTrainBlock);
-    for (int k = tid; k < kPartStride; k += kTrainBlock) red[k] = 0.f;
     __syncthreads();
-    for (int k = tid; k < np; k += kTrainBlock) {
-        float p = a.st_in[k], mo = 0.f, ve = 0.f;
-        if (a.step > 0) {
-            float g = 0.f;
-            int b = 0;
-            for (; b + 8 <= a.nparts; b += 8) {
-                float v[8];
+    const int64_t ntiles = (a.n + 31) / 32;
+    const int64_t tile0 = (int64_t)blockIdx.x * kTrainWaves + wid;
+    float xn[4], tn = 0.f, mn = 0.f;  // the next tile's inputs, target and mask
+    const auto fetch = [&](int64_t tile) {
+        const int64_t at = tile * 32 + i;
+        const bool valid = at < a.n;
 #pragma unroll
-                for (int r = 0; r < 8; ++r) v[r] = a.part_in[(b + r) * kPartStride + k];
-                g += ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
-            }
-            for (; b < a.nparts; ++b) g += a.part_in[b * kPartStride + k];
-            const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
-            mo = a.step > 1 ? a.st_in[kMaxParams + k] : 0.f;
-            ve = a.step > 1 ? a.st_in[2 * kMaxParams + k] : 0.f;
-            mo = b1 * mo + (1.f - b1) * g;
-            ve = b2 * ve + (1.f - b2) * g * g;
-            const float mh = mo / a.c1, vh = ve / a.c2;
-            p -= a.lr * mh / (sqrtf(vh) + eps);
+        for (int k = 0; k < 4; ++k) xn[k] = valid ? a.x[at * kMlpIn + 2 * k + q] : 0.f;
+        tn = valid ? a.t[at * 2 + q] : 0.f;
+        mn = valid ? (a.mask ? a.mask[at * 2 + q] : 1.f) : 0.f;
+    };
+    fetch(tile0);
+    {
+        float p[kTrainParams], mo[kTrainParams], ve[kTrainParams], g[kTrainParams];
+#pragma unroll
+        for (int r = 0; r < kTrainParams; ++r) {
+            const int k = tid + r * kTrainBlock;
+            p[r] = k < np ? a.st_in[k] : 0.f;
+            mo[r] = k < np && a.step > 1 ? a.st_in[kMaxParams + k] : 0.f;
+            ve[r] = k < np && a.step > 1 ? a.st_in[2 * kMaxParams + k] : 0.f;
+            g[r] = 0.f;
         }
-        s.put(k, a.h1, a.h2, p);
-        if (blockIdx.x == 0) {
-            if (a.st_out) {
-                a.st_out[k] = p;
-                a.st_out[kMaxParams + k] = mo;
-                a.st_out[2 * kMaxParams + k] = ve;
+        if (a.step > 0) {
+            int b = 0;
+            const auto add = [&](auto count) {
+                constexpr int N = decltype(count)::value;
+                float v[kTrainParams][N];
+#pragma unroll
+                for (int r = 0; r < kTrainParams; ++r) {
+                    const int k = tid + r * kTrainBlock < np ? tid + r * kTrainBlock : 0;
+#pragma unroll
+                    for (int j = 0; j < N; ++j) v[r][j] = a.part_in[(b + j) * kPartStride + k];
+                }
+#pragma unroll
+                for (int r = 0; r < kTrainParams; ++r) {
+                    if (N == 1) g[r] += v[r][0];
+#pragma unroll
+                    for (int j = 0; j + 8 <= N; j += 8)
+                        g[r] += ((v[r][j] + v[r][j + 1]) + (v[r][j + 2] + v[r][j + 3])) +
+                                ((v[r][j + 4] + v[r][j + 5]) + (v[r][j + 6] + v[r][j + 7]));
+                }
+                b += N;
+            };
+            while (b + 24 <= a.nparts) add(std::integral_constant<int, 24>{});
+            while (b + 8 <= a.nparts) add(std::integral_constant<int, 8>{});
+            while (b < a.nparts) add(std::integral_constant<int, 1>{});
+        }
+#pragma unroll
+        for (int r = 0; r < kTrainParams; ++r) {
+            const int k = tid + r * kTrainBlock;
+            if (k >= np) continue;
+            if (a.step > 0) {
+                const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
+                mo[r] = fmaf(1.f - b1, g[r], b1 * mo[r]);
+                ve[r] = fmaf((1.f - b2) * g[r], g[r], b2 * ve[r]);
+                const float mh = mo[r] / a.c1, vh = ve[r] / a.c2;
+                p[r] -= a.lr * mh / (sqrtf(vh) + eps);
             }
-            if (a.p_out) a.p_out[k] = p;
+            s.put(k, a.h1, a.h2, p[r]);
+            if (blockIdx.x == 0) {
+                if (a.st_out) {
+                    a.st_out[k] = p[r];
+                    a.st_out[kMaxParams + k] = mo[r];
+                    a.st_out[2 * kMaxParams + k] = ve[r];
+                }
+                if (a.p_out) a.p_out[k] = p[r];
+            }
         }
     }
     __syncthreads();
@@ -267,19 +311,18 @@ __global__ __launch_bounds__(kTrainBlock) void k_mlp_train(train_args a) {
     const f32x16 z = {};
     f32x16 g1 = z, g2 = z, g3 = z;  // rows: unit of the layer's output, columns: of its input
     float gb1 = 0.f, gb2 = 0.f, gb3 = 0.f, loss = 0.f;
-    const int64_t ntiles = (a.n + 31) / 32;
-    for (int64_t tile = (int64_t)blockIdx.x * kTrainWaves + wid; tile < ntiles;
-         tile += (int64_t)gridDim.x * kTrainWaves) {
-        const int64_t at = tile * 32 + i;
-        const bool valid = at < a.n;
+    for (int64_t tile = tile0; tile < ntiles; tile += (int64_t)gridDim.x * kTrainWaves) {
+        const bool valid = tile * 32 + i < a.n;
+        const float tv = tn, mk = mn;
         float x[4], y[2];
-        bool odd = false;  // an infinity or NaN among the inputs or activations
+        float odd = 0.f;  // NaN: an infinity or NaN among the inputs or activations
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
-            x[k] = valid ? a.x[at * kMlpIn + 2 * k + q] : 0.f;
-            odd |= !(fabsf(x[k]) <= 3.4e38f);
+            x[k] = xn[k];
+            odd = fmaf(x[k], 0.f, odd);
             xs[i * kMlpIn + 2 * k + q] = x[k];
         }
+        fetch(tile + (int64_t)gridDim.x * kTrainWaves);
         f32x16 a1, a2;
         mlp_fwd32(w, x, a1, a2, y);
         float dyv = 0.f;
@@ -288,8 +331,7 @@ __global__ __launch_bounds__(kTrainBlock) void k_mlp_train(train_args a) {
             const float yo = __shfl(y[1], i);
             const float yv = q ? yo : y[0];
             if (valid) {
-                const float mk = a.mask ? a.mask[at * 2 + q] : 1.f;
-                const float e = yv - a.t[at * 2 + q];
+                const float e = yv - tv;
                 loss += mk * e * e;
                 dyv = 2.f * mk * e * a.inv_count;
             }
@@ -299,7 +341,7 @@ __global__ __launch_bounds__(kTrainBlock) void k_mlp_train(train_args a) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
             d2[r] = valid && a2[r] > 0.f ? d2[r] : 0.f;
-            odd |= !(a1[r] <= 3.4e38f);
+            odd = fmaf(a1[r], 0.f, odd);
             a1s[i * kRow + mrow(r, l)] = valid ? a1[r] : 0.f;
             a2s[i * kRow + mrow(r, l)] = valid ? a2[r] : 0.f;
             d2s[i * kRow + mrow(r, l)] = d2[r];
@@ -311,7 +353,7 @@ __global__ __launch_bounds__(kTrainBlock) void k_mlp_train(train_args a) {
         for (int r = 0; r < 16; ++r) d1s[i * kRow + mrow(r, l)] = valid && a1[r] > 0.f ? d1[r] : 0.f;
         wave_lds_sync();
         // weight gradients: contractions over the samples, two per step
-        if (!__ballot(odd)) {
+        if (!__ballot(odd != 0.f)) {
 #pragma unroll
             for (int k = 0; k < 16; ++k) {
                 const int sm = 2 * k + q;
@@ -353,27 +395,54 @@ __global__ __launch_bounds__(kTrainBlock) void k_mlp_train(train_args a) {
     gb3 += __shfl_xor(gb3, 32);
 #pragma unroll
     for (int d = 32; d; d >>= 1) loss += __shfl_xor(loss, d);
-    // the waves add theirs in turn: the sum's order is fixed
+    // The waves' gradients go to their own arrays, which no sample needs any
+    // more, and every thread adds up some parameters' in the waves' order.
+    // (Waves adding theirs to one array in turn took 14.5 k of 45 k cycles.)
+    enum { kG3 = 32 * kMlpIn, kB1 = kG3 + 64, kB2 = kB1 + 32, kB3 = kB2 + 32, kLoss = kB3 + 2 };
+    static_assert(kLoss < 32 * kRow, "fits a sample array");
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const int k = mrow(r, l);
+        a1s[k * kRow + i] = g2[r];
+        if (i < kMlpIn) a2s[k * kMlpIn + i] = g1[r];
+        if (k < kMlpOut) a2s[kG3 + k * 32 + i] = g3[r];
+    }
+    if (l < 32) {
+        a2s[kB1 + l] = gb1;
+        a2s[kB2 + l] = gb2;
+    }
+    if (l < kMlpOut) a2s[kB3 + l] = gb3;
+    if (l == 0) a2s[kLoss] = loss;
+    __syncthreads();
     const int o_b1 = a.h1 * kMlpIn, o_w2 = o_b1 + a.h1, o_b2 = o_w2 + a.h2 * a.h1,
               o_w3 = o_b2 + a.h2, o_b3 = o_w3 + kMlpOut * a.h2;
-    for (int wv = 0; wv < kTrainWaves; ++wv) {
-        if (wv == wid) {
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int k = mrow(r, l);
-                if (k < a.h1 && i < kMlpIn) red[k * kMlpIn + i] += g1[r];
-                if (k < a.h2 && i < a.h1) red[o_w2 + k * a.h1 + i] += g2[r];
-                if (k < kMlpOut && i < a.h2) red[o_w3 + k * a.h2 + i] += g3[r];
-            }
-            if (l < a.h1) red[o_b1 + l] += gb1;
-            if (l < a.h2) red[o_b2 + l] += gb2;
-            if (l < kMlpOut) red[o_b3 + l] += gb3;
-            if (l == 0) red[np] += loss;
+    for (int r = 0; r < kTrainParams; ++r) {
+        const int k = tid + r * kTrainBlock;  // np < kTrainParams * kTrainBlock
+        if (k > np) continue;
+        const bool in_w2 = k >= o_w2 && k < o_b2;
+        int at;
+        if (in_w2) {
+            const int row = (k - o_w2) / a.h1;
+            at = row * kRow + (k - o_w2 - row * a.h1);
+        } else if (k < o_b1) {
+            at = k;
+        } else if (k < o_w2) {
+            at = kB1 + k - o_b1;
+        } else if (k < o_w3) {
+            at = kB2 + k - o_b2;
+        } else if (k < o_b3) {
+            const int o = k - o_w3 >= a.h2;
+            at = kG3 + o * 32 + (k - o_w3 - o * a.h2);
+        } else {
+            at = kB3 + k - o_b3;  // b3, then the loss
         }
-        __syncthreads();
+        const float *from = (in_w2 ? &A1[0][0] : &A2[0][0]) + at;
+        float sum = 0.f;
+#pragma unroll
+        for (int wv = 0; wv < kTrainWaves; ++wv) sum += from[wv * 32 * kRow];
+        a.part_out[(int64_t)blockIdx.x * kPartStride + k] = sum;
     }
-    for (int k = tid; k <= np; k += kTrainBlock)
-        a.part_out[(int64_t)blockIdx.x * kPartStride + k] = red[k];
 }
 
 // The sum of a pass's partial gradients; entry np is the loss.
