@@ -78,6 +78,11 @@ constexpr int kTdRounds = 2;
 // Largest bottom-up chunk (visited words per wave): a chunk's unvisited
 // vertices are listed in LDS, 2 bytes each.
 constexpr int kBuChunkWords = 32;
+// Entries of a pending list looked at before the others', and rounds of 64 of
+// them whose loads are issued together (bu_pending).
+constexpr int kBuFirst = 8;
+static_assert(kBuFirst <= kColsPad, "read past a list's end");
+constexpr int kBuRounds = 2;
 // Rounds of 64 bottom-up vertices whose head loads are issued together
 // (bu_batch > 1).
 constexpr int kBuBatch = 4;
@@ -754,14 +759,73 @@ __device__ __forceinline__ void td_bitmap_body(const step_args &a, step_smem<BLO
 
 // --------------------------------------------------------------- bottom-up
 
+// R rounds of 64 entries from entry k0 of the lanes' concatenated list pieces
+// (bu_scan), total entries in all.  The rounds' loads are issued together;
+// lanes past the end read the last entry again.
+template <int R>
+__device__ __forceinline__ void bu_rounds(const step_args &a, unsigned long long *hit, int32_t k0,
+                                          int32_t total, int64_t first, int32_t excl) {
+    const int lane = lane_id();
+    int own[R];
+    int32_t pos[R], u[R];
+    uint32_t fw[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        int32_t idx = k0 + 64 * r + lane;
+        idx = idx < total ? idx : total - 1;
+        // owner: the largest lane i with excl_i <= idx
+        int i = 0;
+#pragma unroll
+        for (int st = 32; st > 0; st >>= 1) {
+            const int mid = i + st;
+            const int32_t em = __shfl(excl, mid < 64 ? mid : 63);
+            if (mid < 64 && em <= idx) i = mid;
+        }
+        own[r] = i;
+        pos[r] = idx - __shfl(excl, i);
+        u[r] = __builtin_nontemporal_load(a.cols + (__shfl(first, i) + pos[r]));
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) fw[r] = ((const uint32_t *)a.front)[u[r] >> 5];
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+        if (((fw[r] >> (u[r] & 31)) & 1) && k0 + 64 * r + lane < total)
+            atomicMin(&hit[own[r]], ((unsigned long long)(uint32_t)pos[r] << 32) | (uint32_t)u[r]);
+}
+
+// The n entries from `first` of each lane's list, laid end to end and taken 64
+// at a time; a hit lowers the owner's hit[] to its position from there.
+// Wave-collective.
+__device__ __forceinline__ void bu_scan(const step_args &a, unsigned long long *hit, int64_t first,
+                                        int32_t n) {
+    int32_t excl = wave_incl_scan32(n);
+    const int32_t total = lane_bcast(excl, 63);
+    excl -= n;
+    for (int32_t k0 = 0; k0 < total; k0 += 64 * kBuRounds) {
+        if (k0 + 64 < total)
+            bu_rounds<kBuRounds>(a, hit, k0, total, first, excl);
+        else
+            bu_rounds<1>(a, hit, k0, total, first, excl);
+    }
+}
+
 // Scan the lists of the wave's pending vertices (those whose head index is
-// not in the frontier), pend[i] for i < n.  The first bu_cap neighbours of
-// all n lists are laid end to end and taken 64 at a time, one per lane;
-// a hit records (position << 32 | neighbour) with an LDS atomic minimum, so
-// each vertex keeps its first hit in CSR order, as a sequential scan would.
+// not in the frontier), pend[i] for i < n.  Each lane takes its own list's
+// first kBuFirst neighbours, all their loads in flight; the rest of the first
+// bu_cap of the lists without a hit there are laid end to end and taken 64 at
+// a time, one per lane, where a hit records (position << 32 | neighbour) with
+// an LDS atomic minimum, so each vertex keeps its first hit in CSR order, as a
+// sequential scan would.
 // Lists that hold no hit in their first bu_cap neighbours are finished by
 // the whole wave.  Found vertices get their parent and their bit in the
 // wave's found words (chunk word (v >> 6) - w0).
+// Bound by the latency of a round (owner, entry, frontier word: 1.6 us).  An
+// Erdos-Renyi graph of 3 M vertices and mean degree 27, a sixth of them in the
+// frontier, took 200 rounds a wave and 370 us with whole lists a round at a
+// time; 236 us with eight entries first and two rounds in flight, 230 with the
+// eight a lane's own.  RMAT scale 24, level 2: 93 us, 87, 82.  (Four or twelve
+// entries first: ER 274 and 239; three rounds or more in flight leave four
+// waves per SIMD, and every level 1 us slower.)
 template <int BLOCK>
 __device__ __forceinline__ void bu_pending(const step_args &a, step_smem<BLOCK> &s, const int32_t *pend, int n,
                            int64_t w0, unsigned long long &cnt, unsigned long long &dsum,
@@ -775,41 +839,40 @@ __device__ __forceinline__ void bu_pending(const step_args &a, step_smem<BLOCK> 
         e = a.off[v + 1];
     }
     const int32_t len = (int32_t)(e - b < a.bu_cap ? e - b : a.bu_cap);
-    int32_t excl = wave_incl_scan32(len);
-    const int32_t total = lane_bcast(excl, 63);
-    excl -= len;
-    unsigned long long *hit = s.b_hit[wid];
-    hit[lane] = ~0ULL;
-    wave_lds_sync();
-    for (int32_t k0 = 0; k0 < total; k0 += 64) {
-        const int32_t idx = k0 + lane;
-        // owner: the largest lane i with excl_i <= idx
-        int i = 0;
+    const int32_t len1 = len < kBuFirst ? len : kBuFirst;
+    typedef int32_t quad __attribute__((ext_vector_type(4), aligned(4)));
+    const bool more = __ballot(len1 > 4) != 0;
+    quad q[2];
+    uint32_t fw[kBuFirst];
+    q[0] = __builtin_nontemporal_load((const quad *)(a.cols + b));
+    if (more) q[1] = __builtin_nontemporal_load((const quad *)(a.cols + b + 4));
 #pragma unroll
-        for (int st = 32; st > 0; st >>= 1) {
-            const int mid = i + st;
-            const int32_t em = __shfl(excl, mid < 64 ? mid : 63);
-            if (mid < 64 && em <= idx) i = mid;
-        }
-        const int32_t pos = idx - __shfl(excl, i);
-        const int64_t bi = __shfl(b, i);
-        if (idx < total) {
-            const int32_t u = __builtin_nontemporal_load(a.cols + bi + pos);
-            if ((a.front[u >> 6] >> (u & 63)) & 1)
-                atomicMin(&hit[i], ((unsigned long long)(uint32_t)pos << 32) | (uint32_t)u);
+    for (int k = 0; k < kBuFirst; ++k)
+        if (k < 4 || more)
+            fw[k] = ((const uint32_t *)a.front)[k < len1 ? q[k / 4][k % 4] >> 5 : 0];
+    int32_t par = -1, pos = 0;
+#pragma unroll
+    for (int k = kBuFirst - 1; k >= 0; --k) {
+        if (k >= 4 && !more) continue;
+        if (k < len1 && ((fw[k] >> (q[k / 4][k % 4] & 31)) & 1)) {
+            par = q[k / 4][k % 4];
+            pos = k + 1;
         }
     }
-    wave_lds_sync();
-    const unsigned long long hk = hit[lane];
-    int32_t par = -1;
-    if (valid) {
+    const int32_t len2 = par < 0 ? len - len1 : 0;
+    if (__ballot(len2 > 0)) {
+        unsigned long long *hit = s.b_hit[wid];
+        hit[lane] = ~0ULL;
+        wave_lds_sync();
+        bu_scan(a, hit, b + len1, len2);
+        wave_lds_sync();
+        const unsigned long long hk = hit[lane];
         if (hk != ~0ULL) {
             par = (int32_t)(uint32_t)hk;
-            exam += (hk >> 32) + 1;
-        } else {
-            exam += (unsigned long long)len;
+            pos = len1 + (int32_t)(hk >> 32) + 1;
         }
     }
+    if (valid) exam += (unsigned long long)(par >= 0 ? pos : len);
     // lists with no hit in their first bu_cap neighbours: the whole wave
     uint64_t lm = __ballot(valid && par < 0 && e - b > len);
     while (lm) {

@@ -352,7 +352,7 @@ int build_csr_from_el(bd_ctx *c, int64_t nv, int64_t m) {
     if ((rc = dev_alloc(c, &keys.p, sizeof(uint32_t) * n2, "directed keys"))) return rc;
     if ((rc = dev_alloc(c, &vals.p, sizeof(uint32_t) * n2, "directed values"))) return rc;
     if ((rc = dev_alloc(c, &skeys.p, sizeof(uint32_t) * n2, "sorted keys"))) return rc;
-    if ((rc = dev_alloc(c, (void **)&c->d_cols, sizeof(int32_t) * n2, "cols"))) return rc;
+    if ((rc = dev_alloc(c, (void **)&c->d_cols, sizeof(int32_t) * (n2 + kColsPad), "cols"))) return rc;
     if ((rc = dev_alloc(c, (void **)&c->d_off, sizeof(int64_t) * (nv + 1), "offsets"))) return rc;
     const int64_t nwords = (nv + 63) / 64;
     if ((rc = dev_alloc(c, (void **)&c->d_dead, sizeof(uint64_t) * nwords, "dead bitmap")))
@@ -719,7 +719,8 @@ int build_search_layout(bd_ctx *c) {
     if ((rc = dev_alloc(c, (void **)&c->d_inv, sizeof(int32_t) * nv, "search ids"))) return rc;
     if ((rc = dev_alloc(c, (void **)&c->d_soff, sizeof(int64_t) * (nv + 1), "search offsets")))
         return rc;
-    if ((rc = dev_alloc(c, (void **)&c->d_scols, sizeof(int32_t) * nnz, "search cols")))
+    if ((rc = dev_alloc(c, (void **)&c->d_scols, sizeof(int32_t) * (nnz + kColsPad),
+                        "search cols")))
         return rc;
     if ((rc = dev_alloc(c, (void **)&c->d_sdead, sizeof(uint64_t) * c->nwords,
                         "search dead bitmap")))
@@ -766,7 +767,7 @@ extern "C" int bd_graph_upload(bd_ctx *c, const int64_t *off, const int32_t *col
     free_graph(c);
     const int64_t nwords = (nv + 63) / 64;
     if ((rc = dev_alloc(c, (void **)&c->d_off, sizeof(int64_t) * (nv + 1), "offsets"))) return rc;
-    if ((rc = dev_alloc(c, (void **)&c->d_cols, sizeof(int32_t) * nnz, "cols"))) return rc;
+    if ((rc = dev_alloc(c, (void **)&c->d_cols, sizeof(int32_t) * (nnz + kColsPad), "cols"))) return rc;
     if ((rc = dev_alloc(c, (void **)&c->d_dead, sizeof(uint64_t) * nwords, "dead bitmap")))
         return rc;
     BD_HIP(c, hipMemcpy(c->d_off, off, sizeof(int64_t) * (nv + 1), hipMemcpyHostToDevice));

@@ -34,6 +34,10 @@ constexpr int64_t kHubSlice = 4096;
 // when the frontier has this many edges (below it, the hubs it holds are few).
 constexpr int64_t kHubPassEdges = 1 << 20;
 
+// Entries the arrays of neighbours are longer than their lists, so that a read
+// of a few entries from a list's start stays inside.
+constexpr int64_t kColsPad = 8;
+
 // Frontier lists (queue of ordinary vertices, task slices of high-degree
 // vertices) are segmented: workgroup b appends to segment b % kSeg, so no
 // address is shared by more than a few dozen workgroups -- on MI355X a

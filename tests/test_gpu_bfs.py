@@ -1038,3 +1038,31 @@ def test_lattices_on_both_sides_of_the_solo_bitmap(ctx, orc, rows, cols):
         np.testing.assert_array_equal([r["frontier"] for r in lv], np.bincount(depth[depth >= 0]))
         assert st["steps"] == len(lv) and st["reached"] == (depth >= 0).sum()
         assert [r["level"] for r in lv] == list(range(len(lv)))
+
+
+@pytest.mark.parametrize("head", [1, 2])
+@pytest.mark.parametrize("order", [2, 4])
+@pytest.mark.parametrize("seed", [1, 2, 3])
+def test_bottom_up_lists_at_every_piece(ctx, orc, seed, order, head):
+    """Bottom-up steps over lists of 0 to 80 entries whose first hit lies
+    anywhere: the four and eight entries a lane reads of its own list, the
+    rest up to bu_cap, and what the wave finishes; edges examined included.
+    The graph's last list ends where the array of neighbours does."""
+    r = np.random.default_rng(seed)
+    nv = 6000
+    deg = np.concatenate([r.integers(0, 13, nv // 2), r.integers(28, 40, nv // 4),
+                          r.integers(60, 81, nv // 4)])
+    s = np.repeat(np.arange(nv), r.permutation(deg) // 2)
+    d = r.integers(0, nv, s.size)
+    s, d = np.append(s, nv - 1), np.append(d, 0)
+    off, adj, m = oracle_csr(orc, nv, s, d)
+    t0 = ctx.get_tuning()
+    try:
+        ctx.set_tuning(vertex_order=order, bu_head=head)
+        ctx.upload_csr(off, adj, m)
+        for root in ctx.pick_roots(3):
+            for cap in (1, 7, 8, 9, 32):
+                ctx.set_tuning(bu_cap=cap)
+                run_and_compare(ctx, orc, off, adj, m, int(root), alpha=1 << 40, beta=1 << 40)
+    finally:
+        ctx.set_tuning(**t0)
