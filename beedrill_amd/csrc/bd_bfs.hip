@@ -2233,8 +2233,12 @@ __device__ __forceinline__ int32_t result_parent(const tree_args &a, int32_t i) 
     return p < 0 ? -1 : (a.perm ? a.perm[p] : p);
 }
 
-// Both, of every vertex, for check().
-__global__ void k_result(tree_args a, int32_t *__restrict__ parent, int32_t *__restrict__ depth) {
+// Both, of every vertex, for check(), whose marks are cleared on the way.
+__global__ void k_result(tree_args a, int32_t *__restrict__ parent, int32_t *__restrict__ depth,
+                         uint8_t *__restrict__ marks, int64_t nmarks) {
+    for (int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; k < nmarks;
+         k += (int64_t)gridDim.x * blockDim.x)
+        marks[k] = 0;
     for (int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; v < a.nv;
          v += (int64_t)gridDim.x * blockDim.x) {
         const int32_t i = a.inv ? a.inv[v] : (int32_t)v;
@@ -2942,15 +2946,23 @@ int result_args(bd_ctx *c, bool depth, tree_args *a) {
     return BD_OK;
 }
 
+// check()'s ranges of the adjacency, and its marks (one a range, and two).
+int64_t check_ranges(const bd_ctx *c) {
+    const int64_t chunk = range_entries(c);
+    return (c->nnz + chunk - 1) / chunk;
+}
+
+int ensure_marks(bd_ctx *c) {
+    return c->d_marks ? BD_OK
+                      : dev_alloc(c, (void **)&c->d_marks, check_ranges(c) + 2, "check marks");
+}
+
 // check() of a tree in graph ids whose parents and depths are on the device
-// (or being written on the stream), against the resident graph.  *ok = 1 PASS,
+// (or being written on the stream, as the cleared marks), against the resident graph.  *ok = 1 PASS,
 // 0 FAIL; a fault already in h_flags is a FAIL.
 int check_tree(bd_ctx *c, const int32_t *parent, const int32_t *depth, int64_t source, int *ok) {
-    int rc;
     const int64_t chunk = range_entries(c);
-    const int64_t n = (c->nnz + chunk - 1) / chunk;
-    if (!c->d_marks && (rc = dev_alloc(c, (void **)&c->d_marks, n + 2, "check marks"))) return rc;
-    BD_HIP(c, hipMemsetAsync(c->d_marks, 0, n + 2, c->stream));
+    const int64_t n = check_ranges(c);
     if (n > 0)
         hipLaunchKernelGGL(k_check_edges, dim3((unsigned)((n * 64 + 255) / 256)), dim3(256), 0,
                            c->stream, (const int64_t *)c->d_off, (const int32_t *)c->d_cols, parent,
@@ -3054,9 +3066,9 @@ extern "C" int bd_bfs_check(bd_ctx *c, int64_t source, int *ok) {
     if (rc) return rc;
     clear_flags(c);
     tree_args a;
-    if ((rc = result_args(c, true, &a))) return rc;
+    if ((rc = result_args(c, true, &a)) || (rc = ensure_marks(c))) return rc;
     hipLaunchKernelGGL(k_result, dim3(grid_for(c, c->nv, 256)), dim3(256), 0, c->stream, a,
-                       r.parent, r.depth);
+                       r.parent, r.depth, c->d_marks, check_ranges(c) + 2);
     BD_HIP(c, hipGetLastError());
     return check_tree(c, r.parent, r.depth, source, ok);
 }
@@ -3086,6 +3098,8 @@ extern "C" int bd_bfs_check_parents(bd_ctx *c, int64_t source, const int64_t *pa
         *ok = 0;
         return BD_OK;
     }
+    if ((rc = ensure_marks(c))) return rc;
+    BD_HIP(c, hipMemsetAsync(c->d_marks, 0, check_ranges(c) + 2, c->stream));
     return check_tree(c, d, r.depth, source, ok);
 }
 
@@ -3243,8 +3257,7 @@ extern "C" int bd_bfs_multi_graph(bd_ctx *c, int ngraphs, const int64_t *vbase,
     BD_HIP(c, hipSetDevice(c->device));
     int rc;
     int64_t *d = nullptr;
-    if ((rc = dev_alloc(c, (void **)&d, sizeof(int64_t) * (2 * ngraphs + 1) + sizeof(int),
-                        "batch sources")))
+    if ((rc = dev_alloc(c, (void **)&d, sizeof(int64_t) * (2 * ngraphs + 1), "batch sources")))
         return rc;
     struct guard {
         bd_ctx *c;
@@ -3252,18 +3265,15 @@ extern "C" int bd_bfs_multi_graph(bd_ctx *c, int ngraphs, const int64_t *vbase,
         ~guard() { dev_free(c, p); }
     } gd{c, d};
     int64_t *d_src = d, *d_vbase = d + ngraphs;
-    int *d_bad = (int *)(d + 2 * ngraphs + 1);
-    BD_HIP(c, hipMemcpy(d_src, src.data(), sizeof(int64_t) * ngraphs, hipMemcpyHostToDevice));
-    BD_HIP(c, hipMemcpy(d_vbase, vbase, sizeof(int64_t) * (ngraphs + 1), hipMemcpyHostToDevice));
-    BD_HIP(c, hipMemset(d_bad, 0, sizeof(int)));
+    const size_t each = sizeof(int64_t) * ngraphs;
+    if ((rc = stage_in(c, d, {{src.data(), each}, {vbase, each + sizeof(int64_t)}}))) return rc;
+    clear_flags(c);
     hipLaunchKernelGGL(k_check_parts, dim3(grid_for(c, c->nnz / kPartsChunk * 64 + 64, 256)),
                        dim3(256), 0, c->stream, c->d_off, c->d_cols, c->nnz, d_vbase, ngraphs,
-                       d_bad);
+                       (int *)c->h_flags);
     BD_HIP(c, hipGetLastError());
-    int bad = 0;
-    BD_HIP(c, hipMemcpyAsync(&bad, d_bad, sizeof(int), hipMemcpyDeviceToHost, c->stream));
     BD_HIP(c, hipStreamSynchronize(c->stream));
-    if (bad) return set_err(c, BD_EINVAL, "an edge joins two graphs of the batch");
+    if (c->h_flags[0]) return set_err(c, BD_EINVAL, "an edge joins two graphs of the batch");
     bd_run_stats st;
     if ((rc = run_search(c, src[0], 15, 18, BD_POLICY_BEAMER, &st, d_src, ngraphs))) return rc;
     if (ms) *ms = st.ms;

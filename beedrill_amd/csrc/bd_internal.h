@@ -6,6 +6,7 @@
 #include <stdint.h>
 
 #include <functional>
+#include <initializer_list>
 #include <string>
 #include <unordered_map>
 #include <vector>
@@ -309,6 +310,19 @@ int carry_out(bd_ctx *c, carry kind, void *dst, int64_t n, const carry_part &par
 // The same from a device array that holds the narrow form (on 16 bytes).
 int carry_copy(bd_ctx *c, carry kind, void *dst, const void *src, int64_t n);
 void free_ring(bd_ctx *c);
+// Queue a copy of words 4-byte words (src and out on 16 bytes) to pinned memory.
+int queue_to_host(bd_ctx *c, const void *src, int64_t words, void *out);
+// At least `bytes` (up to 16 MB) of the ring, for results this small.
+int host_ring(bd_ctx *c, int64_t bytes, void **p);
+// Small inputs to dst, one behind the other (sizes a multiple of 4): through
+// the ring and one launch, where each copy from ordinary memory is staged and
+// waited for by itself, some 15 us (over 1 MB they still are).  The stream has
+// to have been waited for before the ring's next use.
+struct host_piece {
+    const void *p;
+    size_t bytes;
+};
+int stage_in(bd_ctx *c, void *dst, std::initializer_list<host_piece> pieces);
 // Entries of a wave's range of the adjacency (walk_range).
 int64_t range_entries(const bd_ctx *c);
 

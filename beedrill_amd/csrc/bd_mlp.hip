@@ -508,14 +508,10 @@ int train_setup(bd_ctx *c, const float *x, const float *t, const float *mask, in
     for (int k = 0; k < 2; ++k, at += part) b->part[k] = at;
     for (int k = 0; k < 2; ++k, at += st) b->st[k] = at;
     b->sum = at;
-    BD_HIP(c, hipMemcpyAsync(b->x, x, sizeof(float) * kMlpIn * n, hipMemcpyHostToDevice, c->stream));
-    BD_HIP(c, hipMemcpyAsync(b->t, t, sizeof(float) * kMlpOut * n, hipMemcpyHostToDevice, c->stream));
-    if (mask)
-        BD_HIP(c, hipMemcpyAsync(b->mask, mask, sizeof(float) * kMlpOut * n, hipMemcpyHostToDevice,
-                                 c->stream));
-    else
-        b->mask = nullptr;
-    return BD_OK;
+    const size_t out = sizeof(float) * kMlpOut * n;  // x, t and mask lie one behind the other
+    rc = stage_in(c, b->x, {{x, sizeof(float) * kMlpIn * n}, {t, out}, {mask, mask ? out : 0}});
+    if (!mask) b->mask = nullptr;
+    return rc;
 }
 
 double mask_count(const float *mask, int64_t n) {
@@ -607,7 +603,7 @@ extern "C" int bd_mlp_infer(bd_ctx *c, const float *x, int64_t n, float *y, int 
     mlp_ws_guard g{c};
     if ((rc = mlp_ws(c, sizeof(float) * (kMlpIn + kMlpOut) * n, &dx))) return rc;
     float *dy = dx + kMlpIn * n;
-    BD_HIP(c, hipMemcpyAsync(dx, x, sizeof(float) * kMlpIn * n, hipMemcpyHostToDevice, c->stream));
+    if ((rc = stage_in(c, dx, {{x, sizeof(float) * kMlpIn * n}}))) return rc;
     const int rows = use_mfma ? 16 : 32;  // samples per wave and round
     const int64_t grid =
         std::max<int64_t>(1, std::min<int64_t>((n + rows - 1) / rows, c->cu_count * 8));
@@ -618,9 +614,8 @@ extern "C" int bd_mlp_infer(bd_ctx *c, const float *x, int64_t n, float *y, int 
         hipLaunchKernelGGL(k_mlp_infer_f32, dim3(grid), dim3(64), 0, c->stream, c->d_mlp,
                            c->mlp_h1, c->mlp_h2, (const float *)dx, n, dy);
     BD_HIP(c, hipGetLastError());
-    BD_HIP(c, hipMemcpyAsync(y, dy, sizeof(float) * 2 * n, hipMemcpyDeviceToHost, c->stream));
-    BD_HIP(c, hipStreamSynchronize(c->stream));
-    return BD_OK;
+    // the inputs have been read when the outputs take their place in the ring
+    return carry_copy(c, carry::i32_i32, y, dy, 2 * n);
 }
 
 extern "C" int bd_mlp_loss_grad(bd_ctx *c, const float *x, const float *t, const float *mask,
@@ -711,11 +706,15 @@ extern "C" int bd_mlp_train(bd_ctx *c, const float *x, const float *t, const flo
     hipLaunchKernelGGL(k_mlp_sum, dim3((np + 256) / 256), dim3(256), 0, c->stream,
                        (const float *)b.part[epochs & 1], b.grid, np, a.inv_count, b.sum);
     BD_HIP(c, hipGetLastError());
-    float h = 0.f;
-    BD_HIP(c, hipMemcpyAsync(&h, b.sum + np, sizeof(float), hipMemcpyDeviceToHost, c->stream));
-    BD_HIP(c, hipMemcpyAsync(c->h_mlp.data(), c->d_mlp, sizeof(float) * np, hipMemcpyDeviceToHost,
-                             c->stream));
-    BD_HIP(c, hipStreamSynchronize(c->stream));
-    if (loss) *loss = h;
-    return refresh_mlp_ops(c);
+    // the summed gradient with the loss at its end, and the parameters
+    void *ring;
+    BD_HIP(c, hipStreamSynchronize(c->stream));  // the samples have left the ring
+    if ((rc = host_ring(c, sizeof(float) * 2 * kPartStride, &ring))) return rc;
+    float *h = (float *)ring;
+    if ((rc = queue_to_host(c, b.sum, np + 1, h)) ||
+        (rc = queue_to_host(c, c->d_mlp, np, h + kPartStride)) || (rc = refresh_mlp_ops(c)))
+        return rc;
+    if (loss) *loss = h[np];
+    std::copy(h + kPartStride, h + kPartStride + np, c->h_mlp.begin());
+    return BD_OK;
 }

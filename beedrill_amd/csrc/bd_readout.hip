@@ -40,6 +40,14 @@ __global__ __launch_bounds__(256) void k_to_host(const uint32_t *__restrict__ sr
     if (t < n % 4) out[n - 1 - t] = src[n - 1 - t];
 }
 
+// n 4-byte words from host memory.
+__global__ __launch_bounds__(256) void k_from_host(const uint32_t *__restrict__ src, int64_t n,
+                                                   uint32_t *__restrict__ dst) {
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
+         i += (int64_t)gridDim.x * blockDim.x)
+        dst[i] = src[i];
+}
+
 size_t narrow_size(carry k) { return k == carry::u8_i32 ? 1 : k == carry::i64_i64 ? 8 : 4; }
 size_t wide_size(carry k) { return k == carry::u8_i32 || k == carry::i32_i32 ? 4 : 8; }
 
@@ -191,13 +199,49 @@ int carry_out(bd_ctx *c, carry kind, void *dst, int64_t n, const carry_part &par
 int carry_copy(bd_ctx *c, carry kind, void *dst, const void *src, int64_t n) {
     const int64_t ns = (int64_t)narrow_size(kind);
     return carry_out(c, kind, dst, n, [&](int64_t first, int64_t count, void *out) -> int {
-        const int64_t words = count * ns / 4;
-        hipLaunchKernelGGL(k_to_host, dim3(grid_for(c, (words + 3) / 4, 256)), dim3(256), 0,
-                           c->stream, (const uint32_t *)((const char *)src + first * ns), words,
-                           (uint32_t *)out);
-        BD_HIP(c, hipGetLastError());
-        return BD_OK;
+        return queue_to_host(c, (const char *)src + first * ns, count * ns / 4, out);
     });
+}
+
+int queue_to_host(bd_ctx *c, const void *src, int64_t words, void *out) {
+    hipLaunchKernelGGL(k_to_host, dim3(grid_for(c, (words + 3) / 4, 256)), dim3(256), 0, c->stream,
+                       (const uint32_t *)src, words, (uint32_t *)out);
+    BD_HIP(c, hipGetLastError());
+    return BD_OK;
+}
+
+int host_ring(bd_ctx *c, int64_t bytes, void **p) {
+    const int rc = ensure_ring(c, bytes);
+    *p = c->h_ring;
+    return rc;
+}
+
+int stage_in(bd_ctx *c, void *dst, std::initializer_list<host_piece> pieces) {
+    size_t total = 0;
+    for (const host_piece &x : pieces) total += x.bytes;
+    if (total > (size_t)kChunkBytes) {
+        char *at = (char *)dst;
+        for (const host_piece &x : pieces) {
+            if (x.bytes)
+                BD_HIP(c, hipMemcpyAsync(at, x.p, x.bytes, hipMemcpyHostToDevice, c->stream));
+            at += x.bytes;
+        }
+        return BD_OK;
+    }
+    int rc;
+    void *ring;
+    // what a call that failed half-way queued may still read the ring
+    BD_HIP(c, hipStreamSynchronize(c->stream));
+    if ((rc = host_ring(c, (int64_t)total, &ring))) return rc;
+    char *at = (char *)ring;
+    for (const host_piece &x : pieces) {
+        if (x.bytes) memcpy(at, x.p, x.bytes);
+        at += x.bytes;
+    }
+    hipLaunchKernelGGL(k_from_host, dim3(grid_for(c, (int64_t)total / 4, 256)), dim3(256), 0,
+                       c->stream, (const uint32_t *)ring, (int64_t)total / 4, (uint32_t *)dst);
+    BD_HIP(c, hipGetLastError());
+    return BD_OK;
 }
 
 void free_ring(bd_ctx *c) {
