@@ -43,7 +43,7 @@ TRAFFIC = os.path.join(ROOT, "profiles", "step_kernel_traffic_rmat_s24.json")
 # k_step<workgroup size, 2>.
 STEP_KERNEL_RE = r"k_step<\d+, 2>"
 # Connected components: the edge pass (pull or push), and its traffic file.
-CC_KERNEL_RE = r"k_cc_(hook|push|tile)"
+CC_KERNEL_RE = r"k_cc_hook"
 CC_TRAFFIC = os.path.join(ROOT, "profiles", "cc_edge_pass_traffic_rmat_s24.json")
 COPY_BYTES = 1 << 30  # calibration copy: 1 GiB read + 1 GiB written
 
@@ -382,16 +382,12 @@ def leg_components(ctx, args):
     time of each run (label initialisation, edge passes, shortcuts and the
     count; the reference times run() alone, components_main.cc:170-180),
     over args.cc_runs runs after one warm-up.  The roofline is the edge pass
-    (k_cc_hook pulls every label -- after the first pass as the long lists'
-    slices plus eight XCD-tiled k_cc_tile phases -- and k_cc_push offers the
-    labels of the vertices that changed), timed per pass with HIP events on
-    the library's stream; avg_launch_ms is that time over the passes'
-    kernel launches.  Algorithmic bytes of a pull: the column indices (4 B
-    per adjacency entry), the labels read (4 B each), the offsets and label
-    of every vertex (12 B); of a push: the changed-vertex bitmap (V/8), the
-    offsets and label of the changed vertices (12 B each, bounded by 12 B
-    per vertex), their column indices and the labels they read (4 + 4 B per
-    label read).  The reference's rate is reported too:
+    (k_cc_hook), stamped by the device from its start to the shortcut's;
+    avg_launch_ms is that time over the passes.  Algorithmic bytes: the first
+    pass reads the column indices (4 B per adjacency entry) and the offsets of
+    every vertex; a later one the label of every vertex (4 B), and the offsets
+    (8 B) and column indices and labels (4 + 4 B per label read) of those that
+    do not carry the largest component's.  The reference's rate is reported too:
     num_iters * num_edges / time (components_main.cc:179)."""
     t0 = time.perf_counter()
     m = ctx.generate_rmat(args.scale, args.edge_factor, seed=args.seed)
@@ -443,7 +439,7 @@ def components_measure(ctx, args, m):
         "reference_gteps": round(float(np.mean([r["num_iters"] * m / (r["ms"] * 1e-3) / 1e9
                                                  for r in runs])), 2),
         "check": ok, "dtype": "int32",
-        "roofline": {"kernel": "k_cc_hook + k_cc_tile + k_cc_push", "bound": "hbm",
+        "roofline": {"kernel": "k_cc_hook", "bound": "hbm",
                      "achieved": round(achieved, 1),
                      "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
@@ -453,7 +449,7 @@ def components_measure(ctx, args, m):
                      "labels_read_per_launch": round(sum(r["labels_read"] for r in runs) / launches)},
         "copy_gbs": round(copy_gbs, 1),
         # built once per graph by the warm-up run, outside `value`: slices of
-        # the long lists and the short lists regrouped by column block
+        # the long lists and the vertex of largest degree
         "regroup_once": {"ms": round(runs[0]["prep_ms"], 3),
                          "bytes": int(runs[0]["prep_bytes"])},
         "cpu_baseline": cpu,

@@ -221,16 +221,16 @@ typedef struct {
     int64_t labels_read;      /* neighbour labels the edge passes read       */
     int64_t edge_bytes;       /* algorithmic bytes of the edge passes: 8 per
                                  label read (column id + label), 4 per
-                                 column id of the first pass, 12 per vertex
-                                 of a pull, per changed vertex of a push,
-                                 and the changed-vertex bitmap              */
-    int64_t pass_launches;    /* kernel launches of the edge passes (a tiled
-                                 pull pass takes 8)                         */
-    double prep_ms;           /* device time of the per-graph regrouping the
-                                 passes use (slices of the long lists, lists
-                                 regrouped by column block), built by the
-                                 first run on a graph and not part of `ms` */
-    int64_t prep_bytes;       /* device memory that regrouping holds       */
+                                 column id of the first pass, 4 per vertex
+                                 for its label, and 8 per vertex that reads
+                                 its list                                   */
+    int64_t pass_launches;    /* kernel launches of the edge passes (one a
+                                 pass)                                      */
+    double prep_ms;           /* device time of what the passes use of the
+                                 graph (slices of the long lists, the vertex
+                                 of largest degree), built by the first run
+                                 on a graph and not part of `ms`           */
+    int64_t prep_bytes;       /* device memory that holds it               */
 } bd_cc_stats;
 
 /* components::run (components.cc:38-104) on the resident graph: label
