@@ -1066,3 +1066,24 @@ def test_bottom_up_lists_at_every_piece(ctx, orc, seed, order, head):
                 run_and_compare(ctx, orc, off, adj, m, int(root), alpha=1 << 40, beta=1 << 40)
     finally:
         ctx.set_tuning(**t0)
+
+
+def test_graphs_in_memory_other_graphs_had(ctx, orc):
+    """Memory of one graph is kept for the next: graphs of other sizes, orders
+    and kinds in turn, each searched, checked and labelled as by itself."""
+    t0 = ctx.get_tuning()
+    try:
+        for k, (scale, order) in enumerate([(15, 4), (8, 4), (13, 2), (15, 1), (10, 3), (15, 4)]):
+            ctx.set_tuning(vertex_order=order)
+            ctx.generate_rmat(scale, 8 + k, seed=k)
+            off, adj = ctx.csr()
+            roots = [int(r) for r in ctx.pick_roots(5)]
+            for root in roots:
+                run_and_compare(ctx, orc, off, adj, ctx.info()[2], root)
+                assert ctx.check(root)
+            np.testing.assert_array_equal(ctx.multi_root(roots)[0],
+                                          [orc.bfs_depth(off, adj, r) for r in roots])
+            ctx.components()
+            np.testing.assert_array_equal(ctx.component_labels(), orc.components(off, adj)[0])
+    finally:
+        ctx.set_tuning(**t0)

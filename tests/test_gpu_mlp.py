@@ -101,3 +101,19 @@ def test_grad_with_an_infinite_input_behind_an_idle_unit(ctx, orc):
     loss_inf, g_inf = ctx.mlp_loss_grad(x, t)
     assert loss_inf == pytest.approx(loss, rel=1e-6)
     np.testing.assert_allclose(g_inf, g, rtol=1e-6, atol=1e-6 * np.abs(g).max())
+
+
+@pytest.mark.parametrize("n", [21845, 21846, 32769])
+def test_samples_on_both_sides_of_the_staged_megabyte(ctx, orc, n):
+    """Samples of up to 1 MB are staged in pinned memory, more are copied; the
+    fp32 tolerances of the tests above."""
+    p = random_params(orc, 31)
+    x, t = data(n, 32)
+    mask = (np.random.default_rng(33).random((n, 2)) > 0.3).astype(np.float32)
+    ctx.mlp_set(p)
+    np.testing.assert_allclose(ctx.mlp_infer(x, mfma=False), orc.mlp_forward(p, x),
+                               rtol=1e-4, atol=1e-5)
+    loss, g = ctx.mlp_loss_grad(x, t, mask)
+    ref_loss, ref_g = orc.mlp_loss_grad(p, x, t, mask)
+    assert loss == pytest.approx(ref_loss, rel=1e-4)
+    np.testing.assert_allclose(g, ref_g, rtol=2e-3, atol=2e-5)
