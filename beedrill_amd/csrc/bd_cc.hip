@@ -122,11 +122,70 @@ __global__ __launch_bounds__(256) void k_cc_tasks(const int64_t *__restrict__ of
     }
 }
 
+// First pass: the lowest neighbour id of each of a wave's 64 light lists (lane
+// i's starts at number s of the group's `total` entries, has d, and entry q is
+// cols[base_k + q]).  As in the later passes every lane takes an entry whatever
+// the degrees, but the owner search and the segmented minimum there are 14
+// lane exchanges for 64 entries, and the LDS unit was what bound the pass.
+// Here a bitmap marks where lists start, an entry's list is the count of bits
+// up to it, and each list has a slot for its minimum: four LDS operations.
+// Scale 18: 37 -> 24 us a pass, scale 23: 536 -> 457 (1.0 GB).  With the owner
+// search kept, more rounds in flight gained nothing at scale 23.
+constexpr int kFirstRounds = 4;  // rounds of 64 entries in flight
+struct first_lds {
+    uint64_t start[kCcHeavy];  // bit q: a list starts at entry q
+    int64_t base[64];          // by rank among the lists that are not empty
+    int32_t low[64];
+};
+
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+}
+
+__device__ __forceinline__ int32_t first_min(first_lds &f, const int32_t *cols, int32_t d, int32_t s,
+                                             int32_t total, int64_t base_k, int32_t mine) {
+    const int lane = lane_id();
+    const int32_t nwords = (total + 63) >> 6;  // d < kCcHeavy: at most kCcHeavy
+    const int rank = __popcll(__ballot(d > 0) & ((1ULL << lane) - 1));
+    for (int32_t w = lane; w < nwords; w += 64) f.start[w] = 0;
+    wave_lds_order();
+    if (d > 0) {
+        atomicOr((unsigned long long *)&f.start[s >> 6], 1ULL << (s & 63));
+        f.base[rank] = base_k;
+        f.low[rank] = mine;
+    }
+    wave_lds_order();
+    const uint64_t upto = (2ULL << lane) - 1;  // this lane's entry and those before
+    int before = -1;  // rank of the list that the entry before the round is in
+    for (int32_t t = 0; t < total; t += 64 * kFirstRounds) {
+        int o[kFirstRounds];
+        int32_t c[kFirstRounds];
+#pragma unroll
+        for (int r = 0; r < kFirstRounds; ++r) {
+            const int32_t w = (t >> 6) + r, q = t + 64 * r + lane;
+            const uint64_t m = w < nwords ? f.start[w] : 0;
+            o[r] = before + __popcll(m & upto);
+            before += __popcll(m);
+            // past the end: the last entry again
+            c[r] = __builtin_nontemporal_load(cols + f.base[o[r]] + (q < total ? q : total - 1));
+        }
+#pragma unroll
+        for (int r = 0; r < kFirstRounds; ++r) atomicMin(&f.low[o[r]], c[r]);
+    }
+    wave_lds_order();
+    const int32_t got = d > 0 ? f.low[rank] : mine;
+    wave_lds_order();  // the slots are rewritten by the next group
+    return got;
+}
+
 // Edge pass.  Units [0, ntasks) are heavy slices; unit ntasks + g is
 // the vertex group [64g, 64g + 64), whose light lists are consecutive in
 // cols (heavy lists between them are skipped).  The group's light edges are
 // numbered q = 0..T-1 (light vertex i owns q in [s_i, s_i + d_i)) and taken
-// 64 at a time, one per lane, so every lane loads whatever the degrees:
+// 64 at a time, one per lane, so every lane loads whatever the degrees (the
+// first pass: first_min):
 //   owner   o(q) = the last i with s_i <= q   (binary search over lanes)
 //   edge    k    = off[base + o] + q - s_o
 //   label   l    = comp[cols[k]]
@@ -146,6 +205,7 @@ __global__ __launch_bounds__(256) void k_cc_hook(const int64_t *__restrict__ off
                                                  unsigned long long *__restrict__ labels_read,
                                                  unsigned long long *__restrict__ edge_bytes) {
     if (!FIRST && st->done) return;
+    __shared__ first_lds lds[FIRST ? 4 : 1];
     const int lane = threadIdx.x & 63;
     const int64_t wave = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
     const int64_t nwaves = ((int64_t)gridDim.x * blockDim.x) >> 6;
@@ -215,6 +275,14 @@ __global__ __launch_bounds__(256) void k_cc_hook(const int64_t *__restrict__ off
         const int32_t total = __builtin_amdgcn_readlane(s_end, 63);
         const int64_t base_k = b - s;  // k = base_k of the owner + q
         int32_t acc = mine;
+        if constexpr (FIRST) {
+            if (total > 0) acc = first_min(lds[threadIdx.x >> 6], cols, d, s, total, base_k, mine);
+            if (lane == 0) nbytes += 4 * (unsigned long long)total;
+            const bool down = acc < mine;
+            if (down) comp[v] = acc;
+            ch |= down;
+            continue;
+        }
         for (int32_t t = 0; t < total; t += 64) {
             const int32_t q = t + lane;
             const int32_t qa = q < total ? q : total - 1;

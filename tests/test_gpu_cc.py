@@ -145,3 +145,33 @@ def test_passes_that_skip_the_largest_label(ctx, orc, order):
         assert st["num_components"] > 1000
     finally:
         ctx.set_tuning(**t0)
+
+
+@pytest.mark.parametrize("degrees", [(0, 1, 2, 63, 64, 65), (254, 255, 256, 257, 0), (255,) * 64,
+                                     (1,) * 63 + (300,), (0,) * 63 + (5,), (300, 0, 1)])
+def test_first_pass_over_lists_of_every_length(ctx, orc, degrees):
+    """Consecutive lists of these lengths (up to 255 entries a wave takes them
+    together, 64 entries at a time), every vertex beside its component's
+    smallest one: the first pass finds all labels and the second changes none."""
+    r = np.random.default_rng(len(degrees))
+    n, base = 64 * 9 + 13, 1400
+    src, dst = [], []
+    for v in range(n):  # vertex base + v: its component's smallest vertex, then others of it
+        d = degrees[v % len(degrees)]
+        if d == 0:
+            continue
+        k = v % 3
+        src.append(np.full(d, base + v))
+        others = base + n + k * 400 + r.permutation(400)[:d - 1]
+        dst.append(r.permutation(np.append(others, k)))
+    src, dst = np.concatenate(src), np.concatenate(dst)
+    nv = base + n + 1200
+    used = np.unique(dst[dst >= base + n])
+    src = np.append(src, used)  # the others too
+    dst = np.append(dst, (used - base - n) // 400)
+    off, adj = orc.build_csr(nv, src, dst)
+    ctx.upload_csr(off, adj, len(src))
+    st = ctx.components()
+    labels, ncomp, _ = orc.components(off, adj)
+    np.testing.assert_array_equal(ctx.component_labels(), labels)
+    assert st["num_components"] == ncomp and st["num_iters"] == 2
