@@ -293,23 +293,12 @@ __global__ __launch_bounds__(256) void k_cc_hook(const int64_t *__restrict__ off
             const int64_t k = shfl(base_k, o) + qa;
             // one past the owner's last lane in this chunk
             const int32_t run_end = min(shfl(s_end, o) - t, 64);
-            bool live = q < total;
-            int32_t lo = 0;
-            if (!FIRST) {
-                lo = shfl(acc, o);
-                live &= lo != g;  // the owner has taken g: it reads no more
-            }
+            const int32_t lo = shfl(acc, o);
             int32_t m = 0x7fffffff;
-            if (live) {
-                const int32_t c = __builtin_nontemporal_load(cols + k);
-                if (FIRST) {
-                    m = c;
-                    nbytes += 4;
-                } else {
-                    m = comp[c];
-                    ++nread;
-                    if (m == g && lo < offer) offer = lo;
-                }
+            if (q < total && lo != g) {  // at g the owner reads no more
+                m = comp[__builtin_nontemporal_load(cols + k)];
+                ++nread;
+                if (m == g && lo < offer) offer = lo;
             }
 #pragma unroll
             for (int step = 1; step < 64; step <<= 1) {
