@@ -840,9 +840,9 @@ int run_multi_root(bd_ctx *c, const int64_t *roots, int n, int32_t *depths, doub
     if (levels) *levels = h.levels;
     const int64_t nrec = std::min<int64_t>(h.levels, c->log_cap);
     c->last_log.resize(nrec);
-    if (nrec)
-        BD_HIP(c, hipMemcpy(c->last_log.data(), c->d_log, sizeof(bd_level_rec) * nrec,
-                            hipMemcpyDeviceToHost));
+    if (nrec && (rc = copy_sync(c, c->last_log.data(), c->d_log, sizeof(bd_level_rec) * nrec,
+                                hipMemcpyDeviceToHost)))
+        return rc;
     for (int64_t i = 0; i < nrec && i < (int64_t)level_ms.size(); ++i) c->last_log[i].ms = level_ms[i];
     c->have_result = false;  // bd_bfs_levels now describes this search, not the last single one
     if (depths) {

@@ -2847,7 +2847,8 @@ extern "C" int bd_bfs_set_script(bd_ctx *c, const int32_t *dirs, int64_t n) {
     if (n == 0) return BD_OK;
     int rc = dev_alloc(c, (void **)&c->d_script, sizeof(int32_t) * n, "script");
     if (rc) return rc;
-    BD_HIP(c, hipMemcpy(c->d_script, dirs, sizeof(int32_t) * n, hipMemcpyHostToDevice));
+    if ((rc = copy_sync(c, c->d_script, dirs, sizeof(int32_t) * n, hipMemcpyHostToDevice)))
+        return rc;
     c->script.assign(dirs, dirs + n);
     c->script_len = n;
     return BD_OK;
@@ -3165,8 +3166,9 @@ extern "C" int bd_bfs_profile(bd_ctx *c, int64_t source, int64_t alpha, int64_t 
             if ((rc = launch_step(c, a, a.force_dir, 0, c->ev[2], c->ev[3]))) return rc;
             BD_HIP(c, hipEventSynchronize(c->ev[3]));
             BD_HIP(c, hipEventElapsedTime(&ms[pass], c->ev[2], c->ev[3]));
-            BD_HIP(c, hipMemcpy(lines.data(), c->d_seg->line[(L + 1) % 3],
-                                sizeof(seg_line) * lines.size(), hipMemcpyDeviceToHost));
+            if ((rc = copy_sync(c, lines.data(), c->d_seg->line[(L + 1) % 3],
+                                sizeof(seg_line) * lines.size(), hipMemcpyDeviceToHost)))
+                return rc;
             for (const seg_line &x : lines) found[pass] += x.acc[0];
         }
         if (found[0] != found[1])

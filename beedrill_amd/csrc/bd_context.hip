@@ -93,6 +93,12 @@ void dev_free(bd_ctx *c, void *p) {
     (void)hipFree(p);
 }
 
+int copy_sync(bd_ctx *c, void *dst, const void *src, size_t bytes, hipMemcpyKind kind) {
+    BD_HIP(c, hipMemcpyAsync(dst, src, bytes, kind, c->stream));
+    BD_HIP(c, hipStreamSynchronize(c->stream));
+    return BD_OK;
+}
+
 static void free_search(bd_ctx *c) {
     dev_free(c, c->d_depth);
     dev_free(c, c->d_parent);
@@ -368,7 +374,9 @@ extern "C" int bd_pick_roots(bd_ctx *c, int64_t n, int64_t *roots) {
     if (!c->d_off) return set_err(c, BD_ESTATE, "no graph");
     BD_HIP(c, hipSetDevice(c->device));
     std::vector<int64_t> off(c->nv + 1);
-    BD_HIP(c, hipMemcpy(off.data(), c->d_off, sizeof(int64_t) * (c->nv + 1), hipMemcpyDeviceToHost));
+    if (int rc = copy_sync(c, off.data(), c->d_off, sizeof(int64_t) * (c->nv + 1),
+                           hipMemcpyDeviceToHost))
+        return rc;
     if (off[c->nv] == 0 && n > 0) return set_err(c, BD_ESTATE, "graph has no edges");
     uint64_t st = 1;  // lcg(0): the skip-ahead loop leaves ran = 1
     const uint64_t mul = 6364136223846793005ULL;

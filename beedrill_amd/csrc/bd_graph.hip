@@ -770,8 +770,11 @@ extern "C" int bd_graph_upload(bd_ctx *c, const int64_t *off, const int32_t *col
     if ((rc = dev_alloc(c, (void **)&c->d_cols, sizeof(int32_t) * (nnz + kColsPad), "cols"))) return rc;
     if ((rc = dev_alloc(c, (void **)&c->d_dead, sizeof(uint64_t) * nwords, "dead bitmap")))
         return rc;
-    BD_HIP(c, hipMemcpy(c->d_off, off, sizeof(int64_t) * (nv + 1), hipMemcpyHostToDevice));
-    if (nnz) BD_HIP(c, hipMemcpy(c->d_cols, cols, sizeof(int32_t) * nnz, hipMemcpyHostToDevice));
+    if ((rc = copy_sync(c, c->d_off, off, sizeof(int64_t) * (nv + 1), hipMemcpyHostToDevice)))
+        return rc;
+    if (nnz &&
+        (rc = copy_sync(c, c->d_cols, cols, sizeof(int32_t) * nnz, hipMemcpyHostToDevice)))
+        return rc;
     dev_buf err{c};
     if ((rc = dev_alloc(c, &err.p, sizeof(int), "flag"))) return rc;
     BD_HIP(c, hipMemsetAsync(err.p, 0, sizeof(int), c->stream));
@@ -828,7 +831,7 @@ extern "C" int bd_graph_from_edges(bd_ctx *c, const int64_t *src, const int64_t 
             return rc;
     }
     int h = 0;
-    BD_HIP(c, hipMemcpy(&h, err.p, sizeof(int), hipMemcpyDeviceToHost));
+    if ((rc = copy_sync(c, &h, err.p, sizeof(int), hipMemcpyDeviceToHost))) return rc;
     if (h) {
         free_graph(c);
         return set_err(c, BD_ERANGE, "vertex id out of range");
@@ -999,7 +1002,7 @@ extern "C" int bd_graph_load_el64(bd_ctx *c, const char *path) {
     fclose(fp);
     if (e != hipSuccess) return hip_err(c, e, "hipMemsetAsync");
     int herr = 0;
-    BD_HIP(c, hipMemcpy(&herr, err.p, sizeof(int), hipMemcpyDeviceToHost));
+    if ((rc = copy_sync(c, &herr, err.p, sizeof(int), hipMemcpyDeviceToHost))) return rc;
     if (herr) {
         free_graph(c);
         return set_err(c, BD_ERANGE, "vertex id out of range");
@@ -1061,7 +1064,9 @@ extern "C" int bd_graph_generate(bd_ctx *c, int kind, int64_t nv, int64_t num_ed
             // rmat_generator.h:178-189: serial re-roll from the stream position
             // that follows the last generated edge.
             std::vector<int64_t> idx(hn);
-            BD_HIP(c, hipMemcpy(idx.data(), sidx.p, sizeof(int64_t) * hn, hipMemcpyDeviceToHost));
+            if ((rc = copy_sync(c, idx.data(), sidx.p, sizeof(int64_t) * hn,
+                                hipMemcpyDeviceToHost)))
+                return rc;
             std::sort(idx.begin(), idx.end());
             std::vector<uint64_t> val(hn);
             sitmo_reader rd;
@@ -1075,8 +1080,11 @@ extern "C" int bd_graph_generate(bd_ctx *c, int kind, int64_t nv, int64_t num_ed
             }
             dev_buf pv{c};
             if ((rc = dev_alloc(c, &pv.p, sizeof(uint64_t) * hn, "patch"))) return rc;
-            BD_HIP(c, hipMemcpy(sidx.p, idx.data(), sizeof(int64_t) * hn, hipMemcpyHostToDevice));
-            BD_HIP(c, hipMemcpy(pv.p, val.data(), sizeof(uint64_t) * hn, hipMemcpyHostToDevice));
+            if ((rc = copy_sync(c, sidx.p, idx.data(), sizeof(int64_t) * hn,
+                                hipMemcpyHostToDevice)) ||
+                (rc = copy_sync(c, pv.p, val.data(), sizeof(uint64_t) * hn,
+                                hipMemcpyHostToDevice)))
+                return rc;
             hipLaunchKernelGGL(k_patch, dim3(grid1d(c, hn)), dim3(kBlock), 0, c->stream,
                                A.as<uint64_t>(), sidx.as<int64_t>(), pv.as<uint64_t>(),
                                (int64_t)hn);
@@ -1095,8 +1103,9 @@ extern "C" int bd_graph_generate(bd_ctx *c, int kind, int64_t nv, int64_t num_ed
     if ((rc = unique_u64(c, B.as<uint64_t>(), A.as<uint64_t>(), ne, &m))) return rc;
     if (m > 0) {
         uint64_t last = 0;
-        BD_HIP(c, hipMemcpy(&last, A.as<uint64_t>() + (m - 1), sizeof(uint64_t),
-                            hipMemcpyDeviceToHost));
+        if ((rc = copy_sync(c, &last, A.as<uint64_t>() + (m - 1), sizeof(uint64_t),
+                            hipMemcpyDeviceToHost)))
+            return rc;
         if (last == ~0ULL) --m;  // the self-loop sentinel (ER)
     }
     if ((rc = finish_edges(c, A.as<uint64_t>(), m, s, nv, kind == BD_GEN_RMAT, seed, false)))
@@ -1119,8 +1128,10 @@ extern "C" int bd_graph_edges_download(bd_ctx *c, int64_t *src, int64_t *dst) {
                        s.as<int64_t>(), d.as<int64_t>());
     BD_HIP(c, hipGetLastError());
     BD_HIP(c, hipStreamSynchronize(c->stream));
-    if (src) BD_HIP(c, hipMemcpy(src, s.p, sizeof(int64_t) * m, hipMemcpyDeviceToHost));
-    if (dst) BD_HIP(c, hipMemcpy(dst, d.p, sizeof(int64_t) * m, hipMemcpyDeviceToHost));
+    if (src && (rc = copy_sync(c, src, s.p, sizeof(int64_t) * m, hipMemcpyDeviceToHost)))
+        return rc;
+    if (dst && (rc = copy_sync(c, dst, d.p, sizeof(int64_t) * m, hipMemcpyDeviceToHost)))
+        return rc;
     return BD_OK;
 }
 

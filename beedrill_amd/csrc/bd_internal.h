@@ -276,6 +276,10 @@ int hip_err(bd_ctx *c, hipError_t e, const char *what);
 // Allocate n bytes of device memory (zero-size requests allocate 256 B).
 int dev_alloc(bd_ctx *c, void **p, size_t bytes, const char *what);
 void dev_free(bd_ctx *c, void *p);
+// A copy to or from ordinary memory, done on return, behind the work queued on
+// the context's stream.  (The stream is a non-blocking one: a plain hipMemcpy
+// runs on the null stream and does not wait for it.)
+int copy_sync(bd_ctx *c, void *dst, const void *src, size_t bytes, hipMemcpyKind kind);
 // Release all graph-dependent buffers.
 void free_graph(bd_ctx *c);
 // (Re)allocate search buffers for the resident graph (and build its search

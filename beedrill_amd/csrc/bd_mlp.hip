@@ -562,7 +562,8 @@ extern "C" int bd_mlp_set(bd_ctx *c, const float *params, int h1, int h2) {
     if (!c->d_mlp &&  // one size fits every network
         (rc = dev_alloc(c, (void **)&c->d_mlp, sizeof(float) * kMaxParams, "mlp")))
         return rc;
-    BD_HIP(c, hipMemcpy(c->d_mlp, params, sizeof(float) * np, hipMemcpyHostToDevice));
+    if ((rc = copy_sync(c, c->d_mlp, params, sizeof(float) * np, hipMemcpyHostToDevice)))
+        return rc;
     c->mlp_h1 = h1;
     c->mlp_h2 = h2;
     c->h_mlp.assign(params, params + np);
@@ -581,7 +582,8 @@ extern "C" int bd_mlp_get(bd_ctx *c, float *params, int64_t cap, int *h1, int *h
     if (params) {
         if (cap < np) return set_err(c, BD_EINVAL, "buffer too small");
         BD_HIP(c, hipSetDevice(c->device));
-        BD_HIP(c, hipMemcpy(params, c->d_mlp, sizeof(float) * np, hipMemcpyDeviceToHost));
+        if ((rc = copy_sync(c, params, c->d_mlp, sizeof(float) * np, hipMemcpyDeviceToHost)))
+            return rc;
     }
     return BD_OK;
 }

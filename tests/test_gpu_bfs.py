@@ -1087,3 +1087,19 @@ def test_graphs_in_memory_other_graphs_had(ctx, orc):
             np.testing.assert_array_equal(ctx.component_labels(), orc.components(off, adj)[0])
     finally:
         ctx.set_tuning(**t0)
+
+
+def test_graph_without_edges_after_others(ctx):
+    """An edge list with no edges, in memory that other graphs had: the flag
+    that its check reads is the one cleared for it."""
+    empty = np.zeros(0, np.int64)
+    for k in range(20):
+        for n in (3, 40 + k, 500):
+            _, s, d = path_graph(n)
+            ctx.from_edges(n, s, d)
+            with pytest.raises(bd.BeedrillError) as e:  # leaves a raised flag behind
+                ctx.from_edges(n - 1, s, d)
+            assert e.value.code == -6
+        ctx.from_edges(70 + k, empty, empty)
+        assert ctx.info() == (70 + k, 0, 0)
+        assert ctx.csr()[0].tolist() == [0] * (71 + k)
