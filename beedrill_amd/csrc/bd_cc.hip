@@ -261,7 +261,7 @@ __global__ __launch_bounds__(256) void k_cc_hook(const int64_t *__restrict__ off
         int32_t mine = 0x7fffffff;
         if (v < nv) {
             mine = FIRST ? (int32_t)v : comp[v];
-            nbytes += 4;
+            if (!FIRST) nbytes += 4;
             if (FIRST || mine != g) {
                 b = off[v];
                 e = off[v + 1];

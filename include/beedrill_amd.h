@@ -221,9 +221,10 @@ typedef struct {
     int64_t labels_read;      /* neighbour labels the edge passes read       */
     int64_t edge_bytes;       /* algorithmic bytes of the edge passes: 8 per
                                  label read (column id + label), 4 per
-                                 column id of the first pass, 4 per vertex
-                                 for its label, and 8 per vertex that reads
-                                 its list                                   */
+                                 column id of the first pass, 8 per vertex
+                                 that reads its list (its bounds), and, from
+                                 the second pass on, 4 per vertex for its
+                                 label                                      */
     int64_t pass_launches;    /* kernel launches of the edge passes (one a
                                  pass)                                      */
     double prep_ms;           /* device time of what the passes use of the

@@ -175,3 +175,15 @@ def test_first_pass_over_lists_of_every_length(ctx, orc, degrees):
     labels, ncomp, _ = orc.components(off, adj)
     np.testing.assert_array_equal(ctx.component_labels(), labels)
     assert st["num_components"] == ncomp and st["num_iters"] == 2
+
+
+@pytest.mark.parametrize("nv,loops", [(1, 1), (63, 2), (64, 2), (65, 300), (1000, 255)])
+def test_bytes_of_a_first_pass_alone(ctx, nv, loops):
+    """Self-loops change no label, so the first pass is the only one: it reads
+    every column id (4 bytes) and every vertex's bounds (8), and no label."""
+    v = np.repeat(np.arange(nv), loops)
+    off = np.arange(nv + 1, dtype=np.int64) * loops
+    ctx.upload_csr(off, v.astype(np.int32), nv * loops // 2)
+    st = ctx.components()
+    assert st["num_iters"] == 1 and st["num_components"] == nv and st["labels_read"] == 0
+    assert st["edge_bytes"] == 4 * nv * loops + 8 * nv
