@@ -24,6 +24,15 @@
 // and a vertex that has taken g needs no more of its list.  At scale 23 the
 // passes after the first then cost little more than reading the labels.
 //
+// Where no component is that large (a union of many, a forest, long paths)
+// every pass reads nearly all labels, so passes have to be few: a vertex that
+// takes a lower label also lowers the root of the one it carried, and the
+// shortcut brings along every vertex that carries that root.  A label
+// that meets a lower one is then gone after the pass; those left have only
+// higher ones around, at most half of the labels of a component that has more
+// than one, so passes grow with the logarithm of its size and not with its
+// diameter (100 k paths of 200: 105 passes, 93 ms, without; 6, 6.7 ms, with).
+//
 // A run is a fixed sequence of launches with no host round trip: an edge
 // pass, a shortcut and a one-workgroup launch that closes the pass
 // (k_cc_close); launches queued past the last pass return at once.
@@ -180,6 +189,17 @@ __device__ __forceinline__ int32_t first_min(first_lds &f, const int32_t *cols, 
     return got;
 }
 
+// Vertices from which the second pass lowers roots; in smaller graphs the tenth
+// is the first to.  Where a pass brings many labels down at once, most of their
+// vertices find the root not yet lowered, and the atomics take up to 0.3 ms:
+// more than the passes they save on a small graph that needs few.  Erdos-Renyi
+// graphs of mean degree 16, a run without and with it from the second pass on:
+// 1 M vertices 414 and 656 us, 2 M 773 and 1060, 4 M 1772 and 1729, 8 M 3602 and
+// 3320; eight such graphs side by side, 4.2 M vertices in all 3150 and 2752 us,
+// 16 M 15.1 and 10.8 ms.  Of mean degree 3, 1 M vertices in nine passes: 374 us,
+// and 472 with it from the sixth on.  Graphs that take more have many to come.
+constexpr int64_t kRootsDownNv = (int64_t)1 << 22;
+
 // Edge pass.  Units [0, ntasks) are heavy slices; unit ntasks + g is
 // the vertex group [64g, 64g + 64), whose light lists are consecutive in
 // cols (heavy lists between them are skipped).  The group's light edges are
@@ -196,12 +216,14 @@ __device__ __forceinline__ int32_t first_min(first_lds &f, const int32_t *cols, 
 // is still its vertex's id when the pass starts, and a pass may read a
 // neighbour's label from before that neighbour's own update in the same pass,
 // so this is one of the pass's own outcomes, with no label gathered.  Later
-// passes skip the vertices labelled g (see the top of the file).
+// passes skip the vertices labelled g and, with lower_roots, lower the roots of
+// the labels that go (see the top of the file).
 template <bool FIRST>
 __global__ __launch_bounds__(256) void k_cc_hook(const int64_t *__restrict__ off,
                                                  const int32_t *__restrict__ cols, int32_t *comp,
                                                  int64_t nv, const td_task *__restrict__ tasks,
-                                                 int64_t ntasks, cc_state *__restrict__ st,
+                                                 int64_t ntasks, bool lower_roots,
+                                                 cc_state *__restrict__ st,
                                                  unsigned long long *__restrict__ labels_read,
                                                  unsigned long long *__restrict__ edge_bytes) {
     if (!FIRST && st->done) return;
@@ -252,8 +274,10 @@ __global__ __launch_bounds__(256) void k_cc_hook(const int64_t *__restrict__ off
             m = (uint32_t)wave_min(m);
             if (!FIRST && __ballot(saw) && mine < offer) offer = mine;
             // a slice is never empty, so m is a label; checked all the same
-            if (lane == 0 && m != 0xffffffffu && (int32_t)m < comp[src])
+            if (lane == 0 && m != 0xffffffffu && (int32_t)m < comp[src]) {
                 if ((int32_t)m < atomicMin(comp + src, (int32_t)m)) ch = true;
+                if (lower_roots && (int32_t)m < comp[mine]) atomicMin(comp + mine, (int32_t)m);
+            }
             continue;
         }
         const int64_t v = (u - ntasks) * 64 + lane;
@@ -310,7 +334,10 @@ __global__ __launch_bounds__(256) void k_cc_hook(const int64_t *__restrict__ off
             if (mine_here && acc != g && got < acc) acc = got;
         }
         const bool down = acc < mine;
-        if (down) comp[v] = acc;
+        if (down) {
+            comp[v] = acc;
+            if (lower_roots && acc < comp[mine]) atomicMin(comp + mine, acc);
+        }
         ch |= down;
     }
     if (!FIRST) {
@@ -481,16 +508,11 @@ extern "C" int bd_cc_run(bd_ctx *c, bd_cc_stats *out) {
     for (int chunk = 3;; chunk = 2) {
         if (queued > nv + 4) return set_err(c, BD_EHIP, "components did not converge");
         for (int k = 0; k < chunk; ++k, ++queued) {
-            if (queued == 0)
-                hipLaunchKernelGGL(k_cc_hook<true>, hook_grid, block, 0, c->stream,
-                                   (const int64_t *)c->d_off, (const int32_t *)c->d_cols, c->d_comp,
-                                   nv, (const td_task *)c->d_cc_tasks, c->cc_ntasks, st, nread,
-                                   ebytes);
-            else
-                hipLaunchKernelGGL(k_cc_hook<false>, hook_grid, block, 0, c->stream,
-                                   (const int64_t *)c->d_off, (const int32_t *)c->d_cols, c->d_comp,
-                                   nv, (const td_task *)c->d_cc_tasks, c->cc_ntasks, st, nread,
-                                   ebytes);
+            const bool lower_roots = queued >= (nv < kRootsDownNv ? 9 : 1);
+            hipLaunchKernelGGL((queued == 0 ? k_cc_hook<true> : k_cc_hook<false>), hook_grid, block,
+                               0, c->stream, (const int64_t *)c->d_off, (const int32_t *)c->d_cols,
+                               c->d_comp, nv, (const td_task *)c->d_cc_tasks, c->cc_ntasks,
+                               lower_roots, st, nread, ebytes);
             if (queued == 0 && c->d_head) {
                 hipLaunchKernelGGL(k_cc_shortcut, grid, block, 0, c->stream, c->d_comp, nv, st, 1,
                                    (unsigned long long *)nullptr);

@@ -238,9 +238,12 @@ typedef struct {
  * propagation (each vertex takes its neighbours' smallest label) and
  * shortcutting until an edge pass changes nothing.  Each component ends
  * labelled by its smallest vertex id.  The first pass takes neighbour ids
- * for labels (each label is still its vertex's id); once few labels change,
- * a pass offers only the changed vertices' labels to their neighbours (the
- * same pairs as a pull over changed neighbours; the outcome is unchanged). */
+ * for labels (each label is still its vertex's id); later ones leave out the
+ * vertices labelled like the vertex of largest degree, whose edges are read
+ * from their other ends, and may lower the root of a label along with the
+ * vertex that carried it, so that passes grow with the logarithm of a
+ * component's size (the outcome is unchanged; num_iters can be lower than the
+ * reference's, and differ between runs). */
 int bd_cc_run(bd_ctx *ctx, bd_cc_stats *out);
 /* components::component_ (components.h:13-14) of the last run: labels[nv]. */
 int bd_cc_fetch(bd_ctx *ctx, int64_t *labels);

@@ -187,3 +187,69 @@ def test_bytes_of_a_first_pass_alone(ctx, nv, loops):
     st = ctx.components()
     assert st["num_iters"] == 1 and st["num_components"] == nv and st["labels_read"] == 0
     assert st["edge_bytes"] == 4 * nv * loops + 8 * nv
+
+
+@pytest.mark.parametrize("fan", [0, 3, 254, 255, 2047, 2100])
+@pytest.mark.parametrize("n", [2, 65, 600, 20000])
+def test_passes_grow_with_the_logarithm_of_a_component(ctx, orc, n, fan):
+    """Relabelled paths with hubs on either side of the list cuts, beside
+    settled components, one of them with the vertex of largest degree: the
+    first pass leaves a component with labels of half its vertices at most,
+    every one from the tenth on with half of the labels, and the last changes
+    none."""
+    rng = np.random.default_rng(n + fan)
+    a, b = np.triu_indices(60, 1)
+    src, dst = [a, np.full(2200, 60)], [b, 61 + np.arange(2200)]
+    base = 2300
+    for _ in range(3):
+        src.append(base + np.arange(n - 1))
+        dst.append(base + np.arange(1, n))
+        for at in (0, n // 2, n - 1):
+            src.append(np.full(fan, base + at))
+            dst.append(base + n + np.arange(fan))
+        base += n + fan
+    perm = rng.permutation(base + 7)
+    s, d = perm[np.concatenate(src)], perm[np.concatenate(dst)]
+    off, adj = orc.build_csr(base + 7, s, d)
+    ctx.upload_csr(off, adj, len(s))
+    for _ in range(2):
+        st = compare(ctx, orc, off, adj)
+        assert st["num_iters"] <= np.ceil(np.log2(max(n + fan, 2201))) + 9
+
+
+@pytest.mark.parametrize("seed", [1, 2, 3])
+def test_components_of_many_shapes(ctx, orc, seed):
+    """Forests, unions of paths, of power-law graphs and of sparse random ones,
+    every id relabelled."""
+    r = np.random.default_rng(seed)
+    graphs = []
+    for comps in (1, 40, 3000):
+        nv = 20000
+        v = np.arange(comps, nv)
+        graphs.append((nv, v, (r.random(v.size) * v).astype(np.int64)))
+    for k, length in ((1, 3000), (50, 300), (2000, 9)):
+        v = np.arange(k * length).reshape(k, length)
+        graphs.append((k * length, v[:, :-1].ravel(), v[:, 1:].ravel()))
+    for m in (9000, 15000, 60000):
+        graphs.append((30000, r.integers(0, 30000, m), r.integers(0, 30000, m)))
+    parts = [orc.make_rmat(11, 8, seed=10 * seed + i) for i in range(12)]
+    graphs.append((12 << 11, np.concatenate([s + (i << 11) for i, (_, s, _) in enumerate(parts)]),
+                   np.concatenate([d + (i << 11) for i, (_, _, d) in enumerate(parts)])))
+    for nv, s, d in graphs:
+        p = r.permutation(nv + 5)
+        s, d = p[s], p[d]
+        off, adj = orc.build_csr(nv + 5, s, d)
+        ctx.upload_csr(off, adj, len(s))
+        compare(ctx, orc, off, adj)
+
+
+@pytest.mark.parametrize("nv", [(1 << 22) - 1, 1 << 22])
+def test_graphs_on_both_sides_of_the_root_rule(ctx, orc, nv):
+    """The second pass lowers roots from 2^22 vertices on: sparse random graphs
+    of hundreds of thousands of components."""
+    ctx.generate_er(nv, nv, seed=nv & 3)
+    off, adj = ctx.csr()
+    st = ctx.components()
+    labels, n, _ = orc.components(off, adj)
+    np.testing.assert_array_equal(ctx.component_labels(), labels)
+    assert st["num_components"] == n and st["num_iters"] <= 22 + 9
