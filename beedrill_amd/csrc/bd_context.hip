@@ -4,6 +4,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <mutex>
 
 #include "bd_internal.h"
 
@@ -23,52 +24,112 @@ int hip_err(bd_ctx *c, hipError_t e, const char *what) {
 // a call, and hipMalloc takes 37; building the graph of 3 M edges makes 34
 // pairs of them (4.8 of 6.8 ms).  So freed blocks of up to kPoolBlock are kept
 // for the next allocation of about their size, kPoolBytes of them at most,
-// until the context is destroyed or an allocation fails.  A context's work is
-// on its one stream, and a block is kept only once that stream is idle, as
-// hipFree would wait too.
+// until the context is destroyed or an allocation on the device fails, which
+// gives back what every context keeps there.  A context's work is on its one
+// stream, and a block is kept only once that stream is idle, as hipFree would
+// wait too, so any thread may free it.
 constexpr size_t kPoolBlock = (size_t)64 << 20;
 constexpr size_t kPoolBytes = (size_t)256 << 20;
 
+// The contexts and the lock of their kept blocks; never destroyed, as a program
+// may destroy its contexts late.
+struct pool_list {
+    std::mutex lock;
+    std::vector<bd_ctx *> contexts;
+};
+
+static pool_list &pools() {
+    static pool_list *p = new pool_list;
+    return *p;
+}
+
+// With the lock held.
 static void pool_release(bd_ctx *c) {
     for (auto &b : c->pool) (void)hipFree(b.p);
     c->pool.clear();
     c->pool_bytes = 0;
 }
 
-int dev_alloc(bd_ctx *c, void **p, size_t bytes, const char *what) {
-    *p = nullptr;
-    const size_t unit = bytes < ((size_t)1 << 20) ? 4096 : (size_t)64 << 10;
-    const size_t size = (std::max<size_t>(bytes, 1) + unit - 1) / unit * unit;
-    // the smallest kept block that holds it without wasting a quarter
+static void pool_join(bd_ctx *c) {
+    const std::lock_guard<std::mutex> g(pools().lock);
+    pools().contexts.push_back(c);
+}
+
+static void pool_leave(bd_ctx *c) {
+    const std::lock_guard<std::mutex> g(pools().lock);
+    pool_release(c);
+    auto &all = pools().contexts;
+    all.erase(std::remove(all.begin(), all.end(), c), all.end());
+}
+
+// A kept block of the context that holds `size` bytes without wasting a
+// quarter, the smallest of them.
+static bool pool_take(bd_ctx *c, size_t size, dev_block *out) {
+    const std::lock_guard<std::mutex> g(pools().lock);
     size_t best = c->pool.size();
     for (size_t i = 0; i < c->pool.size(); ++i)
         if (c->pool[i].bytes >= size && c->pool[i].bytes <= size + size / 4 + 4096 &&
             (best == c->pool.size() || c->pool[i].bytes < c->pool[best].bytes))
             best = i;
-    if (best < c->pool.size()) {
-        const dev_block b = c->pool[best];
-        c->pool[best] = c->pool.back();
-        c->pool.pop_back();
-        c->pool_bytes -= b.bytes;
+    if (best == c->pool.size()) return false;
+    *out = c->pool[best];
+    c->pool[best] = c->pool.back();
+    c->pool.pop_back();
+    c->pool_bytes -= out->bytes;
+    return true;
+}
+
+// False when the pool is full, or host memory is.
+static bool pool_keep(bd_ctx *c, const dev_block &b) {
+    const std::lock_guard<std::mutex> g(pools().lock);
+    if (c->pool_bytes + b.bytes > kPoolBytes) return false;
+    try {
+        c->pool.push_back(b);
+    } catch (...) {
+        return false;
+    }
+    c->pool_bytes += b.bytes;
+    return true;
+}
+
+// hipMalloc; when it fails, what every context keeps on this one's device goes
+// back first.
+static hipError_t device_malloc(bd_ctx *c, void **p, size_t bytes) {
+    hipError_t e = hipMalloc(p, bytes);
+    if (e != hipErrorOutOfMemory) return e;
+    const std::lock_guard<std::mutex> g(pools().lock);
+    bool any = false;
+    for (bd_ctx *o : pools().contexts) {
+        if (o->device != c->device || o->pool.empty()) continue;
+        pool_release(o);
+        any = true;
+    }
+    if (!any) return e;
+    (void)hipGetLastError();
+    return hipMalloc(p, bytes);
+}
+
+int dev_alloc(bd_ctx *c, void **p, size_t bytes, const char *what) {
+    *p = nullptr;
+    const size_t unit = bytes < ((size_t)1 << 20) ? 4096 : (size_t)64 << 10;
+    dev_block b{nullptr, (std::max<size_t>(bytes, 1) + unit - 1) / unit * unit};
+    if (!pool_take(c, b.bytes, &b)) {
+        const hipError_t e = device_malloc(c, &b.p, b.bytes);
+        if (e != hipSuccess) {
+            (void)hipGetLastError();
+            char buf[160];
+            snprintf(buf, sizeof(buf), "hipMalloc(%s, %zu bytes) failed: %s", what, bytes,
+                     hipGetErrorString(e));
+            return set_err(c, e == hipErrorOutOfMemory ? BD_ENOMEM : BD_EHIP, buf);
+        }
+    }
+    try {
         c->live[b.p] = b.bytes;
-        *p = b.p;
-        return BD_OK;
+    } catch (...) {
+        (void)hipFree(b.p);
+        return BD_ENOMEM;
     }
-    hipError_t e = hipMalloc(p, size);
-    if (e == hipErrorOutOfMemory && !c->pool.empty()) {
-        (void)hipGetLastError();
-        pool_release(c);
-        e = hipMalloc(p, size);
-    }
-    if (e != hipSuccess) {
-        *p = nullptr;
-        (void)hipGetLastError();
-        char buf[160];
-        snprintf(buf, sizeof(buf), "hipMalloc(%s, %zu bytes) failed: %s", what, bytes,
-                 hipGetErrorString(e));
-        return set_err(c, e == hipErrorOutOfMemory ? BD_ENOMEM : BD_EHIP, buf);
-    }
-    c->live[*p] = size;
+    *p = b.p;
     return BD_OK;
 }
 
@@ -77,18 +138,14 @@ void dev_free(bd_ctx *c, void *p) {
     const auto it = c->live.find(p);
     const size_t size = it == c->live.end() ? kPoolBlock + 1 : it->second;
     if (it != c->live.end()) c->live.erase(it);
-    if (size <= kPoolBlock && c->pool_bytes + size <= kPoolBytes) {
+    if (size <= kPoolBlock) {
         hipError_t e = hipStreamQuery(c->stream);
         if (e == hipErrorNotReady) {
             (void)hipGetLastError();
             e = hipStreamSynchronize(c->stream);
         }
-        if (e == hipSuccess) {
-            c->pool.push_back({p, size});
-            c->pool_bytes += size;
-            return;
-        }
-        (void)hipGetLastError();
+        if (e == hipSuccess && pool_keep(c, {p, size})) return;
+        if (e != hipSuccess) (void)hipGetLastError();
     }
     (void)hipFree(p);
 }
@@ -250,6 +307,7 @@ extern "C" int bd_create(bd_ctx **out, int device) {
     if (device < 0 || device >= n) return BD_EINVAL;
     bd_ctx *c = new bd_ctx();
     c->device = device;
+    pool_join(c);
     // launch shape and thresholds: beedrill_amd/autotune.py's best on MI355X
     // (RMAT scale 24, generator seed 1, models/tuning_rmat_s24.json), except
     // bu_cap (its 64 gained 0.8% there and cost an Erdos-Renyi graph 6%) and
@@ -290,8 +348,8 @@ extern "C" int bd_create(bd_ctx **out, int device) {
     for (int i = 0; i < 4 && e == hipSuccess; ++i)
         e = i < 2 ? hipEventCreate(&c->ev[i])
                   : hipEventCreateWithFlags(&c->ev[i], hipEventReleaseToDevice);
-    if (e == hipSuccess) e = hipMalloc((void **)&c->d_ctl, 2 * sizeof(ctl_block));
-    if (e == hipSuccess) e = hipMalloc((void **)&c->d_seg, sizeof(seg_counters));
+    if (e == hipSuccess) e = device_malloc(c, (void **)&c->d_ctl, 2 * sizeof(ctl_block));
+    if (e == hipSuccess) e = device_malloc(c, (void **)&c->d_seg, sizeof(seg_counters));
     if (e == hipSuccess) e = hipHostMalloc((void **)&c->h_ctl, 2 * sizeof(ctl_block), hipHostMallocDefault);
     const unsigned shared = hipHostMallocMapped | hipHostMallocCoherent;
     if (e == hipSuccess) {
@@ -304,7 +362,7 @@ extern "C" int bd_create(bd_ctx **out, int device) {
         e = hipHostMalloc((void **)&c->h_log, sizeof(bd_level_rec) * kHostRecs, shared);
     }
     if (e == hipSuccess) {
-        e = hipMalloc((void **)&c->d_log, sizeof(bd_level_rec) * c->log_cap);
+        e = device_malloc(c, (void **)&c->d_log, sizeof(bd_level_rec) * c->log_cap);
     }
     if (e != hipSuccess) {
         (void)hipGetLastError();
@@ -331,7 +389,7 @@ extern "C" int bd_destroy(bd_ctx *c) {
     dev_free(c, c->d_mlp);
     dev_free(c, c->d_mlp_ops);
     dev_free(c, c->d_mlp_ws);
-    pool_release(c);
+    pool_leave(c);
     if (c->h_ctl) (void)hipHostFree(c->h_ctl);
     if (c->h_res) (void)hipHostFree(c->h_res);
     if (c->h_flags) (void)hipHostFree(c->h_flags);

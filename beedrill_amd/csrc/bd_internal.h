@@ -153,7 +153,7 @@ struct bd_ctx {
     hipStream_t stream = nullptr;
     std::string err;
     std::unordered_map<void *, size_t> live;  // dev_alloc's blocks
-    std::vector<bd::dev_block> pool;          // freed ones kept (dev_free)
+    std::vector<bd::dev_block> pool;          // freed ones kept (dev_free), under a lock
     size_t pool_bytes = 0;
 
     // graph (flat device CSR)

@@ -1,0 +1,113 @@
+"""What the library does when an allocation fails.  Each case runs in a child
+process that loads limits.c ahead of the library, so that HIP's memory calls
+end with out-of-memory where the case says; nothing is exhausted."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+
+HEAD = """
+import ctypes, sys, threading
+sys.path.insert(0, {root!r})
+lim = ctypes.CDLL({lib!r}, ctypes.RTLD_GLOBAL)
+lim.limits_used.restype = lim.limits_peak.restype = ctypes.c_size_t
+lim.limits_set.argtypes = [ctypes.c_size_t, ctypes.c_size_t]
+NONE = 2**64 - 1
+import numpy as np
+import beedrill_amd as bd
+import oracle as orc
+
+def searched(c):
+    off, adj = c.csr()
+    root = int(c.pick_roots(1)[0])
+    c.bfs(root)
+    depth, parent = c.fetch()
+    np.testing.assert_array_equal(depth, orc.bfs_depth(off, adj, root))
+    assert orc.check(off, adj, root, parent)
+"""
+
+
+@pytest.fixture(scope="module")
+def limited(tmp_path_factory):
+    lib = str(tmp_path_factory.mktemp("limits") / "limits.so")
+    subprocess.run(["gcc", "-O1", "-shared", "-fPIC", "-o", lib, os.path.join(HERE, "limits.c"),
+                    "-ldl", "-lpthread"], check=True)
+
+    def run(code):
+        r = subprocess.run([sys.executable, "-c", HEAD.format(root=ROOT, lib=lib) + code],
+                           capture_output=True, text=True, timeout=100)
+        assert r.returncode == 0, r.stdout + r.stderr
+        return r.stdout
+    return run
+
+
+def test_memory_kept_by_another_context(limited):
+    """What a context keeps of its freed blocks goes back when another's
+    allocation fails, and what it has in use stays."""
+    limited("""
+c = bd.Context(0)
+before = lim.limits_used()
+assert before > 0  # the calls go through the limits
+lim.limits_peak()
+c.generate_er(300000, 1500000, seed=2)
+need = lim.limits_peak() - before
+c.close()
+a, b = bd.Context(0), bd.Context(0)
+a.generate_er(1000000, 4000000, seed=1)
+held = lim.limits_used()
+a.generate_er(1000, 4000, seed=1)
+a.components()
+used = lim.limits_used()
+assert used - before > need  # most of it kept
+lim.limits_set(used + need // 4, NONE)
+b.generate_er(300000, 1500000, seed=2)
+searched(b)
+searched(a)
+assert a.component_labels().size == 1000
+lim.limits_set(lim.limits_used(), NONE)
+try:
+    b.generate_er(3000000, 15000000, seed=2)
+    raise SystemExit("over the limit")
+except bd.BeedrillError as e:
+    assert e.code == -2, e
+lim.limits_set(NONE, NONE)
+b.generate_er(1000, 3000, seed=2)
+searched(b)
+searched(a)
+print("done")
+""")
+
+
+def test_memory_kept_by_contexts_of_several_threads(limited):
+    """Contexts of three threads build and search graphs under a limit that
+    holds what they have in use, but not what they keep as well."""
+    limited("""
+c = bd.Context(0)
+before = lim.limits_used()
+lim.limits_peak()
+c.generate_er(200000, 1000000, seed=2)
+need = lim.limits_peak() - before
+c.close()
+lim.limits_set(lim.limits_used() + 4 * need, NONE)
+bad = []
+def work(k):
+    try:
+        with bd.Context(0) as x:
+            for i in range(6):
+                x.generate_er(200000 // (1 + (i + k) % 3), 1000000 // (1 + (i + k) % 3), seed=i)
+                searched(x)
+    except BaseException as e:
+        bad.append(e)
+        raise
+ts = [threading.Thread(target=work, args=(k,)) for k in range(3)]
+[t.start() for t in ts]
+[t.join() for t in ts]
+assert not bad, bad
+print("done")
+""")
