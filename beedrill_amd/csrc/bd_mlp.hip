@@ -562,12 +562,14 @@ extern "C" int bd_mlp_set(bd_ctx *c, const float *params, int h1, int h2) {
     if (!c->d_mlp &&  // one size fits every network
         (rc = dev_alloc(c, (void **)&c->d_mlp, sizeof(float) * kMaxParams, "mlp")))
         return rc;
-    if ((rc = copy_sync(c, c->d_mlp, params, sizeof(float) * np, hipMemcpyHostToDevice)))
-        return rc;
+    BD_HIP(c, hipMemcpyAsync(c->d_mlp, params, sizeof(float) * np, hipMemcpyHostToDevice, c->stream));
     c->mlp_h1 = h1;
     c->mlp_h2 = h2;
     c->h_mlp.assign(params, params + np);
-    if ((rc = refresh_mlp_ops(c))) return rc;
+    if ((rc = refresh_mlp_ops(c))) {  // which waits for the stream
+        (void)hipStreamSynchronize(c->stream);
+        return rc;
+    }
     c->has_mlp = true;
     return BD_OK;
 }
