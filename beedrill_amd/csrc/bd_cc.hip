@@ -457,15 +457,11 @@ extern "C" int bd_cc_run(bd_ctx *c, bd_cc_stats *out) {
     // read, algorithmic bytes of the edge passes
     constexpr int kBlockWords = kSlots * kLine;
     static_assert(sizeof(cc_state) <= sizeof(unsigned long long) * kLine, "state line");
+    static_assert(sizeof(cc_result) <= kFlagLine, "result's place");
     if (!c->d_cc_flag &&
         (rc = dev_alloc(c, (void **)&c->d_cc_flag,
                         sizeof(unsigned long long) * (kLine + 3 * kBlockWords), "label flags")))
         return rc;
-    if (!c->h_cc) {
-        BD_HIP(c, hipHostMalloc(&c->h_cc, sizeof(cc_result),
-                                hipHostMallocMapped | hipHostMallocCoherent));
-        ((cc_result *)c->h_cc)->seq = 0;
-    }
     c->have_cc = false;
     cc_state *st = (cc_state *)c->d_cc_flag;
     unsigned long long *count = (unsigned long long *)c->d_cc_flag + kLine;

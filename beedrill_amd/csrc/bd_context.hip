@@ -356,7 +356,11 @@ extern "C" int bd_create(bd_ctx **out, int device) {
         e = hipHostMalloc((void **)&c->h_res, sizeof(search_result), shared);
         if (e == hipSuccess) c->h_res->seq = 0;
     }
-    if (e == hipSuccess) e = hipHostMalloc((void **)&c->h_flags, 4 * sizeof(int32_t), shared);
+    if (e == hipSuccess) e = hipHostMalloc((void **)&c->h_flags, kFlagBytes, shared);
+    if (e == hipSuccess) {
+        memset(c->h_flags, 0, kFlagBytes);
+        c->h_cc = (char *)c->h_flags + kFlagLine;
+    }
     if (e == hipSuccess) {
         c->log_cap = 1 << 16;
         e = hipHostMalloc((void **)&c->h_log, sizeof(bd_level_rec) * kHostRecs, shared);
@@ -393,7 +397,6 @@ extern "C" int bd_destroy(bd_ctx *c) {
     if (c->h_ctl) (void)hipHostFree(c->h_ctl);
     if (c->h_res) (void)hipHostFree(c->h_res);
     if (c->h_flags) (void)hipHostFree(c->h_flags);
-    if (c->h_cc) (void)hipHostFree(c->h_cc);
     if (c->h_log) (void)hipHostFree(c->h_log);
     free_ring(c);
     for (auto &e : c->ev)

@@ -138,6 +138,9 @@ struct search_result {
     uint32_t seq;
 };
 
+// The readout kernels' flags (on a line), then a component run's result.
+constexpr size_t kFlagLine = 128, kFlagBytes = 2 * kFlagLine;
+
 // Device memory a context has, or keeps for its next allocations.
 struct dev_block {
     void *p;
@@ -194,7 +197,7 @@ struct bd_ctx {
     int32_t *d_comp = nullptr;    // connected-component labels (components_)
     int32_t *d_cc_flag = nullptr; // a component run's state and counters
     bool have_cc = false;         // d_comp holds a finished run
-    void *h_cc = nullptr;         // pinned: a component run's result, written by the device
+    void *h_cc = nullptr;         // a component run's result, written by the device (behind h_flags)
     int32_t cc_hub = 0;           // the vertex of largest degree
     bd::td_task *d_cc_tasks = nullptr;  // slices of the long lists of the edge pass
     int64_t cc_ntasks = -1;             // -1: not built for the resident graph
@@ -227,7 +230,7 @@ struct bd_ctx {
     uint64_t *d_tree = nullptr;   // ancestors of a deep parent tree
     int32_t *d_out = nullptr;     // check(): nv parents in graph ids, then nv depths
     uint8_t *d_marks = nullptr;   // check: per range, its spanning list's parent was found
-    int32_t *h_flags = nullptr;   // pinned: faults a readout kernel found
+    int32_t *h_flags = nullptr;   // pinned, kFlagBytes: faults a readout kernel found
     void *h_ring = nullptr;       // pinned: results on their way to the caller (bd_readout.hip)
     int64_t ring_bytes = 0;
     hipEvent_t ring_ev[bd::kRing] = {};
@@ -316,7 +319,8 @@ int carry_copy(bd_ctx *c, carry kind, void *dst, const void *src, int64_t n);
 void free_ring(bd_ctx *c);
 // Queue a copy of words 4-byte words (src and out on 16 bytes) to pinned memory.
 int queue_to_host(bd_ctx *c, const void *src, int64_t words, void *out);
-// At least `bytes` (up to 16 MB) of the ring, for results this small.
+// At least `bytes` (up to 16 MB) of the ring, for results this small; BD_ENOMEM
+// when they cannot be pinned.
 int host_ring(bd_ctx *c, int64_t bytes, void **p);
 // Small inputs to dst, one behind the other (sizes a multiple of 4): through
 // the ring and one launch, where each copy from ordinary memory is staged and

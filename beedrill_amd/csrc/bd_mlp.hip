@@ -713,11 +713,19 @@ extern "C" int bd_mlp_train(bd_ctx *c, const float *x, const float *t, const flo
     // the summed gradient with the loss at its end, and the parameters
     void *ring;
     BD_HIP(c, hipStreamSynchronize(c->stream));  // the samples have left the ring
-    if ((rc = host_ring(c, sizeof(float) * 2 * kPartStride, &ring))) return rc;
-    float *h = (float *)ring;
-    if ((rc = queue_to_host(c, b.sum, np + 1, h)) ||
-        (rc = queue_to_host(c, c->d_mlp, np, h + kPartStride)) || (rc = refresh_mlp_ops(c)))
+    float own[2 * kPartStride], *h = own;
+    if ((rc = host_ring(c, sizeof(own), &ring)) == BD_OK) {
+        h = (float *)ring;
+        if ((rc = queue_to_host(c, b.sum, np + 1, h)) ||
+            (rc = queue_to_host(c, c->d_mlp, np, h + kPartStride)))
+            return rc;
+    } else if (rc != BD_ENOMEM ||
+               (rc = copy_sync(c, h, b.sum, sizeof(float) * (np + 1), hipMemcpyDeviceToHost)) ||
+               (rc = copy_sync(c, h + kPartStride, c->d_mlp, sizeof(float) * np,
+                               hipMemcpyDeviceToHost))) {
         return rc;
+    }
+    if ((rc = refresh_mlp_ops(c))) return rc;
     if (loss) *loss = h[np];
     std::copy(h + kPartStride, h + kPartStride + np, c->h_mlp.begin());
     return BD_OK;

@@ -12,6 +12,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <new>
 #include <thread>
 #include <vector>
 
@@ -73,6 +74,7 @@ int helper_threads() {
 }
 
 // The pinned ring, at least `bytes` and at most kRing chunks, and its events.
+// BD_ENOMEM when it cannot be pinned: results then go the plain way.
 int ensure_ring(bd_ctx *c, int64_t bytes) {
     if (c->ring_bytes < bytes) {
         // what a small graph needs is pinned in no time; a whole ring takes about 2 ms
@@ -86,13 +88,41 @@ int ensure_ring(bd_ctx *c, int64_t bytes) {
         if (e != hipSuccess) {
             c->h_ring = nullptr;
             (void)hipGetLastError();
-            return set_err(c, BD_ENOMEM, "pinned result buffer");
+            return BD_ENOMEM;
         }
         c->ring_bytes = want;
     }
     if (bytes > kChunkBytes)
         for (auto &ev : c->ring_ev)
             if (!ev) BD_HIP(c, hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+    return BD_OK;
+}
+
+// Without the ring: a chunk at a time through device memory and a plain copy.
+int carry_plain(bd_ctx *c, carry kind, void *dst, int64_t n, const carry_part &part) {
+    const int64_t ns = (int64_t)narrow_size(kind), ws = (int64_t)wide_size(kind);
+    const int64_t per = std::min<int64_t>(n, kChunkBytes / ns);
+    struct buffers {
+        bd_ctx *c;
+        void *dev = nullptr;
+        char *host = nullptr;
+        ~buffers() {
+            dev_free(c, dev);
+            delete[] host;
+        }
+    } b{c};
+    int rc;
+    if ((rc = dev_alloc(c, &b.dev, per * ns, "result chunk"))) return rc;
+    if (ns != ws && !(b.host = new (std::nothrow) char[per * ns]))
+        return set_err(c, BD_ENOMEM, "result chunk");
+    for (int64_t first = 0; first < n; first += per) {
+        const int64_t cnt = std::min(per, n - first);
+        char *to = (char *)dst + first * ws;
+        if ((rc = part(first, cnt, b.dev)) ||
+            (rc = copy_sync(c, b.host ? b.host : to, b.dev, cnt * ns, hipMemcpyDeviceToHost)))
+            return rc;
+        if (b.host) widen(kind, b.host, to, cnt);
+    }
     return BD_OK;
 }
 
@@ -103,7 +133,8 @@ int carry_out(bd_ctx *c, carry kind, void *dst, int64_t n, const carry_part &par
     const int64_t ns = (int64_t)narrow_size(kind), ws = (int64_t)wide_size(kind);
     const int64_t per = kChunkBytes / ns, chunks = (n + per - 1) / per;
     int rc;
-    if ((rc = ensure_ring(c, std::min<int64_t>(n * ns, kRing * kChunkBytes)))) return rc;
+    if ((rc = ensure_ring(c, std::min<int64_t>(n * ns, kRing * kChunkBytes))))
+        return rc == BD_ENOMEM ? carry_plain(c, kind, dst, n, part) : rc;
     char *ring = (char *)c->h_ring;
     if (chunks == 1) {
         if ((rc = part(0, n, ring))) return rc;
@@ -219,7 +250,14 @@ int host_ring(bd_ctx *c, int64_t bytes, void **p) {
 int stage_in(bd_ctx *c, void *dst, std::initializer_list<host_piece> pieces) {
     size_t total = 0;
     for (const host_piece &x : pieces) total += x.bytes;
-    if (total > (size_t)kChunkBytes) {
+    int rc = BD_ENOMEM;
+    void *ring;
+    if (total <= (size_t)kChunkBytes) {
+        // what a call that failed half-way queued may still read the ring
+        BD_HIP(c, hipStreamSynchronize(c->stream));
+        if ((rc = host_ring(c, (int64_t)total, &ring)) && rc != BD_ENOMEM) return rc;
+    }
+    if (rc) {  // too large, or nothing to be pinned
         char *at = (char *)dst;
         for (const host_piece &x : pieces) {
             if (x.bytes)
@@ -228,11 +266,6 @@ int stage_in(bd_ctx *c, void *dst, std::initializer_list<host_piece> pieces) {
         }
         return BD_OK;
     }
-    int rc;
-    void *ring;
-    // what a call that failed half-way queued may still read the ring
-    BD_HIP(c, hipStreamSynchronize(c->stream));
-    if ((rc = host_ring(c, (int64_t)total, &ring))) return rc;
     char *at = (char *)ring;
     for (const host_piece &x : pieces) {
         if (x.bytes) memcpy(at, x.p, x.bytes);

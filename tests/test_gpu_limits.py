@@ -111,3 +111,51 @@ ts = [threading.Thread(target=work, args=(k,)) for k in range(3)]
 assert not bad, bad
 print("done")
 """)
+
+
+def test_results_where_nothing_can_be_pinned(limited):
+    """Results and small inputs then go by plain copies: chunks of every form
+    (bytes, ints, ids; short and in several pieces), batches, components and
+    training; and again through pinned memory once there is some."""
+    limited("""
+def everything(c, deep):
+    for nv, m in ((700, 3000), (300000, 900000), (1100003, 2500000)):
+        c.generate_er(nv, m, seed=nv & 7)
+        searched(c)
+        off, adj = c.csr()
+        r = c.components()
+        labels, n, _ = orc.components(off, adj)
+        assert r["num_components"] == n
+        np.testing.assert_array_equal(c.component_labels(), labels)
+        roots = [int(v) for v in c.pick_roots(3)]
+        np.testing.assert_array_equal(c.multi_root(roots)[0],
+                                      [orc.bfs_depth(off, adj, v) for v in roots])
+    s = np.arange(deep - 1)
+    c.from_edges(deep, s, s + 1)
+    searched(c)  # past 250 levels: depths as ints
+    depth, _ = c.multi_graph([0, deep], [0])
+    np.testing.assert_array_equal(depth, np.arange(deep))
+    rng = np.random.default_rng(1)
+    x, t = rng.random((500, 8), np.float32), rng.random((500, 2), np.float32)
+    p = rng.standard_normal(32 * 8 + 32 + 32 * 32 + 32 + 64 + 2).astype(np.float32) / 8
+    c.mlp_set(p, 32, 32)
+    loss = c.mlp_train(x, t, epochs=5, lr=3e-3)
+    return loss, c.mlp_get()[0], c.mlp_infer(x, mfma=False), c.mlp_infer(x), c.mlp_loss_grad(x, t)[1]
+
+free = bd.Context(0)
+want = everything(free, 700)
+c = bd.Context(0)
+lim.limits_set(NONE, 0)
+got = [everything(c, 700), everything(c, 700)]
+lim.limits_set(NONE, NONE)
+c.generate_er(2000, 9000, seed=1)
+searched(c)  # a small ring
+lim.limits_set(NONE, 0)
+got.append(everything(c, 400000 // 1000))
+lim.limits_set(NONE, NONE)
+got.append(everything(c, 300))
+for g in got:
+    for a, b in zip(g, want):
+        np.testing.assert_array_equal(a, b)
+print("done")
+""")
