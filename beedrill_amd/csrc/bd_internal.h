@@ -234,6 +234,7 @@ struct bd_ctx {
     void *h_ring = nullptr;       // pinned: results on their way to the caller (bd_readout.hip)
     int64_t ring_bytes = 0;
     hipEvent_t ring_ev[bd::kRing] = {};
+    int cpus = 0;                 // CPUs the process may keep busy (0: not read yet)
     bool split_off = false;    // profiling: top-down steps never run with remote writes
     bool cand_clean = false;   // d_cand is all -1 (set when a search finishes)
     int chunk_hint = 0;        // first chunk of device-driven launches (0: 16)

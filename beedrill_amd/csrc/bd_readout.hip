@@ -8,7 +8,6 @@
 // pinned chunks, and a few host threads widen chunks into the caller's pages
 // while later ones are on their way.
 #include <string.h>
-#include <sched.h>
 
 #include <algorithm>
 #include <atomic>
@@ -16,6 +15,7 @@
 #include <thread>
 #include <vector>
 
+#include "bd_cpus.h"
 #include "bd_internal.h"
 
 namespace bd {
@@ -67,10 +67,12 @@ void widen(carry k, const void *src, void *dst, int64_t n) {
     }
 }
 
-int helper_threads() {
-    cpu_set_t set;
-    const int n = sched_getaffinity(0, sizeof(set), &set) == 0 ? CPU_COUNT(&set) : 1;
-    return std::min(kMaxHelpers, n / 2);
+// Helpers spin while their chunk is on its way, so they may be half of the CPUs
+// that the process has the use of.  Those that its quota leaves are read once a
+// context (7 to 23 us).
+int helper_threads(bd_ctx *c) {
+    if (c->cpus == 0) c->cpus = usable_cpus();
+    return std::min(kMaxHelpers, std::min(c->cpus, affinity_cpus()) / 2);
 }
 
 // The pinned ring, at least `bytes` and at most kRing chunks, and its events.
@@ -184,7 +186,7 @@ int carry_out(bd_ctx *c, carry kind, void *dst, int64_t n, const carry_part &par
     std::vector<std::thread> helpers;
     while (!rc && issued < std::min<int64_t>(chunks, kRing)) rc = issue();
     if (!rc && n * ws >= kThreadBytes) {
-        const int64_t nh = std::min<int64_t>(helper_threads(), nunits - 1);
+        const int64_t nh = std::min<int64_t>(helper_threads(c), nunits - 1);
         try {
             helpers.reserve(nh);
             for (int64_t i = 0; i < nh; ++i) helpers.emplace_back(help);
