@@ -1103,3 +1103,66 @@ def test_graph_without_edges_after_others(ctx):
         ctx.from_edges(70 + k, empty, empty)
         assert ctx.info() == (70 + k, 0, 0)
         assert ctx.csr()[0].tolist() == [0] * (71 + k)
+
+
+def top_down_levels(off, depth, m):
+    """Records of a search of top-down steps alone, from its depths."""
+    deg = np.diff(off)
+    n = depth.max() + 1
+    seen = depth >= 0
+    count = np.bincount(depth[seen], minlength=n + 1)
+    dsum = np.bincount(depth[seen], weights=deg[seen], minlength=n + 1).astype(np.int64)
+    left, left_deg = len(deg) - np.cumsum(count), int(off[-1]) - np.cumsum(dsum)
+    return [dict(level=k, dir=0, frontier=count[k], frontier_deg=dsum[k], unvisited=left[k],
+                 unvisited_deg=left_deg[k], edges_to_check=2 * m, result=dsum[k + 1],
+                 next=count[k + 1], next_deg=dsum[k + 1], edges_examined=dsum[k],
+                 max_frontier_deg=deg[depth == k].max()) for k in range(n)]
+
+
+@pytest.mark.parametrize("paths", [1, 64, 2047, 2048, 2049, 3100])
+def test_records_of_small_frontiers_under_other_policies(orc, paths):
+    """Steps run many to a launch leave the same records: top-down alone what
+    the depths and degrees give, learned without a network Beamer's."""
+    nv, s, d = bundle_graph(paths, 40)
+    off, adj, m = oracle_csr(orc, nv, s, d)
+    with bd.Context(0) as c:  # no network in it
+        c.upload_csr(off, adj, m)
+        for root in (0, nv - 1, nv // 2):
+            for _ in range(2):
+                run_and_compare(c, orc, off, adj, m, root, policy="td_only")
+                assert_same_levels(c.levels(), top_down_levels(off, c.fetch()[0], m))
+                assert _launches_follow(c.levels())
+            for alpha in (3, 15, 1 << 40):
+                run_and_compare(c, orc, off, adj, m, root, policy="learned", alpha=alpha)
+                _, _, ref = orc.beamer(off, adj, m, root, alpha, head=orc.head_index(off, adj))
+                assert_same_levels(c.levels(), ref)
+
+
+@pytest.mark.parametrize("split", [1, 16, 299, 599, 600, 601, 1200])
+@pytest.mark.parametrize("shape", ["bundle", "lattice"])
+def test_small_frontiers_between_remote_writes(ctx, orc, shape, split):
+    """Steps of `split` frontier edges or more are run with remote writes: the
+    launch that runs many stops before one and goes on after it.  The bundle's
+    paths have frontiers of 600 edges, the lattice's grow to that and shrink."""
+    if shape == "bundle":
+        nv, s, d = bundle_graph(300, 60)
+        off, adj, m = oracle_csr(orc, nv, s, d)
+        ctx.upload_csr(off, adj, m)
+    else:
+        ctx.generate_lattice(150, 170)
+        off, adj = ctx.csr()
+        nv, m = len(off) - 1, len(adj) // 2
+    t0 = ctx.get_tuning()
+    try:
+        ctx.set_tuning(td_split_edges=split)
+        for root in (0, nv // 2, nv - 1):
+            for alpha in (15, 1 << 40):
+                for _ in range(2):
+                    run_and_compare(ctx, orc, off, adj, m, root, alpha=alpha)
+                    lv = ctx.levels()
+                    assert _launches_follow(lv) and ctx.check(root)
+                    for r in lv:
+                        if r["dir"] == 0:
+                            assert r["launches"] == (2 if r["frontier_deg"] >= split else 1)
+    finally:
+        ctx.set_tuning(**t0)

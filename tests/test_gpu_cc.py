@@ -253,3 +253,19 @@ def test_graphs_on_both_sides_of_the_root_rule(ctx, orc, nv):
     labels, n, _ = orc.components(off, adj)
     np.testing.assert_array_equal(ctx.component_labels(), labels)
     assert st["num_components"] == n and st["num_iters"] <= 22 + 9
+
+
+@pytest.mark.parametrize("scale", [14, 17])
+def test_one_launch_a_pass_and_few_labels_read(ctx, scale):
+    """An edge pass is one launch.  Where one component holds nearly all edges,
+    the passes after the first read few labels: a vertex that carries its label
+    reads none, and one that takes it no more."""
+    ctx.generate_rmat(scale, 16, seed=scale)
+    off, adj = ctx.csr()
+    for _ in range(3):
+        st = ctx.components()
+        labels = ctx.component_labels()
+        big = np.bincount(labels).max()
+        assert big > 0.9 * np.count_nonzero(np.diff(off))
+        assert st["pass_launches"] == st["num_iters"] >= 2
+        assert st["labels_read"] <= 0.25 * (st["num_iters"] - 1) * len(adj)
