@@ -38,9 +38,10 @@
 // flushed once per block into the block's segment), task slices for
 // high-degree vertices, and the depth-(L+1) bitmap; a bottom-up step writes
 // only the bitmap, and a top-down step after it reads the bitmap.  The
-// direction is
-// picked on the device, so a search is a stream of launches with no host
-// round trip.
+// direction is picked on the device, so a search is a stream of launches with
+// no host round trip.  On a graph without long lists, k_solo goes before the
+// step launch and runs the levels whose frontiers are small, as many as there
+// are in a row, on one workgroup.
 #include <hip/hip_ext.h>
 #include <math.h>
 #include <stdio.h>
@@ -127,9 +128,7 @@ struct step_args {
     bd_level_rec *hlog, *log;  // the first kHostRecs records (host memory), the others
     search_result *res;    // host memory
     const int32_t *script;
-    const float *mlp;
     const uint4 *mlp_ops;  // the network's operands in MFMA lane order
-    int64_t nwords;
     int64_t live_nwords;   // words holding every vertex with edges (the sweeps cover these)
     int64_t task_cap;
     int64_t qseg_cap, tseg_cap;
@@ -145,7 +144,7 @@ struct step_args {
     int32_t bu_words, bu_cap, bu_head, bu_batch;
     int32_t policy, script_len, log_cap;
     uint32_t seq;          // the search's number
-    int32_t mlp_h1, mlp_h2, has_mlp;
+    int32_t has_mlp;
     float mlp_margin;      // log2-cost margin for the network to override Beamer
     int64_t mlp_near;      // also consulted at top-down steps this close to Beamer's switch
 };
@@ -2476,9 +2475,7 @@ step_args make_args(bd_ctx *c, int32_t level, int64_t alpha, int64_t beta, int p
     a.res = c->h_res;
     a.seq = c->search_seq;
     a.script = c->d_script;
-    a.mlp = c->d_mlp;
     a.mlp_ops = c->d_mlp_ops;
-    a.nwords = c->nwords;
     // vertices past nv_active have no edges when the layout is renumbered:
     // clear() sets their visited bits, no step finds them, and only an
     // isolated source (whose search ends after one step) is ever in a
@@ -2508,8 +2505,6 @@ step_args make_args(bd_ctx *c, int32_t level, int64_t alpha, int64_t beta, int p
     a.policy = policy;
     a.script_len = (int32_t)c->script_len;
     a.log_cap = (int32_t)c->log_cap;
-    a.mlp_h1 = c->mlp_h1;
-    a.mlp_h2 = c->mlp_h2;
     // The network was trained on graphs with hubs; on a graph whose largest
     // degree is under learned_min_skew times the mean, LEARNED runs Beamer.
     const bool skewed = (double)c->max_deg * (double)c->nv >=

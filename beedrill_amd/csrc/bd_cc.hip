@@ -60,7 +60,7 @@ struct cc_state {
 struct cc_result {
     int64_t iters, components, labels_read, edge_bytes;
     uint64_t ticks, pass_ticks;
-    int32_t done, bad;
+    int32_t bad;
     uint32_t seq;
 };
 
@@ -499,7 +499,8 @@ extern "C" int bd_cc_run(bd_ctx *c, bd_cc_stats *out) {
     const uint32_t seq = res->seq + 1;
     hipLaunchKernelGGL(k_cc_init, grid, block, 0, c->stream, c->d_comp, nv, st, count,
                        3 * kBlockWords);
-    // passes queued at a time: the fewest a graph with edges takes, then two
+    // passes queued at a time: three (most graphs take two to four, and one that
+    // is not needed returns at once), then two
     int64_t queued = 0;
     for (int chunk = 3;; chunk = 2) {
         if (queued > nv + 4) return set_err(c, BD_EHIP, "components did not converge");
