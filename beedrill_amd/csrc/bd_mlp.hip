@@ -216,9 +216,11 @@ struct train_args {
 // a launch's latency, the parameter update and ~110 MFMAs per wave, 16.0 us
 // (27.4 with one parameter's partials loaded after another's and the waves'
 // gradients added up in turn).  All of a thread's parameters are loaded
-// together, up to 24 partials of each, and the first tile's samples before
-// them.  The update is still 6 us of it; twice the threads for it alone leave
-// the others half the registers, which spilled (21 us).
+// together, up to 16 partials of each, and the first tile's samples before
+// them (32 epochs of 300 to 20000 samples: 8 partials at a time 0 to 2% longer,
+// 24 the same, 32 from 1% longer at 3000 to 3% less at 8000, 48 longer).  The
+// update is still 6 us of it; twice the threads for it alone leave the others
+// half the registers, which spilled (21 us).
 __global__ __launch_bounds__(kTrainBlock) void k_mlp_train(train_args a) {
     __shared__ mlp_lds s;
     // per wave: activations and gradients of its samples, [sample][unit]
@@ -273,7 +275,7 @@ __global__ __launch_bounds__(kTrainBlock) void k_mlp_train(train_args a) {
                 }
                 b += N;
             };
-            while (b + 24 <= a.nparts) add(std::integral_constant<int, 24>{});
+            while (b + 16 <= a.nparts) add(std::integral_constant<int, 16>{});
             while (b + 8 <= a.nparts) add(std::integral_constant<int, 8>{});
             while (b < a.nparts) add(std::integral_constant<int, 1>{});
         }
