@@ -450,7 +450,7 @@ def components_measure(ctx, args, m):
         "copy_gbs": round(copy_gbs, 1),
         # built once per graph by the warm-up run, outside `value`: slices of
         # the long lists and the vertex of largest degree
-        "regroup_once": {"ms": round(runs[0]["prep_ms"], 3),
+        "prep_once": {"ms": round(runs[0]["prep_ms"], 3),
                          "bytes": int(runs[0]["prep_bytes"])},
         "cpu_baseline": cpu,
     }
