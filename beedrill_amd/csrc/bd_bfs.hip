@@ -672,8 +672,12 @@ __device__ __forceinline__ void td_bitmap_body(const step_args &a, step_smem<BLO
     // workgroup had up to 64 * BLOCK of them to expand (scale 20: 38 k
     // vertices of 45 k edges in 44.8 us, 13.7 with even ranges).  For a light
     // frontier the ranks of the empty ranges cost more than they spread (a
-    // lattice's levels: 9.8 us, 11.8 with even ranges).
-    const int rw = s.st.frontier >= kEvenRanges ? a.bu_words * (BLOCK / 64) : BLOCK;
+    // lattice's levels: 9.8 us, 11.8 with even ranges), and a frontier of fewer
+    // vertices than there would be ranges is light (8000 x 8000: 672 ms with
+    // even ranges from 4096 vertices on, 487 with this).
+    const int even = a.bu_words * (BLOCK / 64);
+    const int rw = s.st.frontier >= kEvenRanges && s.st.frontier * even >= a.live_nwords ? even
+                                                                                        : BLOCK;
     for (int64_t w0 = (int64_t)blockIdx.x * rw; w0 < a.live_nwords; w0 += (int64_t)gridDim.x * rw) {
         const int64_t wi = w0 + tid;
         uint64_t w = tid < rw && wi < a.live_nwords ? a.front[wi] : 0ULL;

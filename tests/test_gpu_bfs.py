@@ -1166,3 +1166,23 @@ def test_small_frontiers_between_remote_writes(ctx, orc, shape, split):
                             assert r["launches"] == (2 if r["frontier_deg"] >= split else 1)
     finally:
         ctx.set_tuning(**t0)
+
+
+def test_levels_of_a_wide_lattice_cost_the_same_past_4096_vertices(ctx):
+    """A frontier of 4096 vertices or more is ranked in even ranges only where
+    they hold a vertex each: on a large lattice levels on either side of that
+    number take the same time (a fifth longer with a range for each 32 words)."""
+    ctx.generate_lattice(3600, 4600)
+    t0 = ctx.get_tuning()
+    try:
+        ctx.set_tuning(time_steps=3)
+        root = 1800 * 4600 + 2300
+        ctx.bfs(root)
+        ctx.bfs(root)
+        lv = ctx.levels()
+        below = [r["ms"] for r in lv if 3500 <= r["frontier"] < 4096]
+        above = [r["ms"] for r in lv if 4096 <= r["frontier"] < 4700]
+        assert len(below) > 50 and len(above) > 50
+        assert np.median(above) < 1.1 * np.median(below)
+    finally:
+        ctx.set_tuning(**t0)
