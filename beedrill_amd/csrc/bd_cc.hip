@@ -457,7 +457,7 @@ extern "C" int bd_cc_run(bd_ctx *c, bd_cc_stats *out) {
     // read, algorithmic bytes of the edge passes
     constexpr int kBlockWords = kSlots * kLine;
     static_assert(sizeof(cc_state) <= sizeof(unsigned long long) * kLine, "state line");
-    static_assert(sizeof(cc_result) <= kFlagLine, "result's place");
+    static_assert(sizeof(cc_result) <= sizeof(host_state::cc), "result's place");
     if (!c->d_cc_flag &&
         (rc = dev_alloc(c, (void **)&c->d_cc_flag,
                         sizeof(unsigned long long) * (kLine + 3 * kBlockWords), "label flags")))

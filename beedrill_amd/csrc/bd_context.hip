@@ -1,5 +1,6 @@
 // bd_context.hip -- context lifetime, errors, buffers and small queries.
 #include <hip/hip_ext.h>
+#include <stddef.h>
 #include <stdio.h>
 #include <string.h>
 
@@ -351,20 +352,17 @@ extern "C" int bd_create(bd_ctx **out, int device) {
                   : hipEventCreateWithFlags(&c->ev[i], hipEventReleaseToDevice);
     if (e == hipSuccess) e = device_malloc(c, (void **)&c->d_ctl, 2 * sizeof(ctl_block));
     if (e == hipSuccess) e = device_malloc(c, (void **)&c->d_seg, sizeof(seg_counters));
-    if (e == hipSuccess) e = hipHostMalloc((void **)&c->h_ctl, 2 * sizeof(ctl_block), hipHostMallocDefault);
-    const unsigned shared = hipHostMallocMapped | hipHostMallocCoherent;
+    if (e == hipSuccess)
+        e = hipHostMalloc((void **)&c->h_state, sizeof(host_state),
+                          hipHostMallocMapped | hipHostMallocCoherent);
     if (e == hipSuccess) {
-        e = hipHostMalloc((void **)&c->h_res, sizeof(search_result), shared);
-        if (e == hipSuccess) c->h_res->seq = 0;
-    }
-    if (e == hipSuccess) e = hipHostMalloc((void **)&c->h_flags, kFlagBytes, shared);
-    if (e == hipSuccess) {
-        memset(c->h_flags, 0, kFlagBytes);
-        c->h_cc = (char *)c->h_flags + kFlagLine;
-    }
-    if (e == hipSuccess) {
+        memset((void *)c->h_state, 0, offsetof(host_state, log));
+        c->h_ctl = c->h_state->ctl;
+        c->h_res = &c->h_state->res;
+        c->h_flags = c->h_state->flags;
+        c->h_cc = c->h_state->cc;
+        c->h_log = c->h_state->log;
         c->log_cap = 1 << 16;
-        e = hipHostMalloc((void **)&c->h_log, sizeof(bd_level_rec) * kHostRecs, shared);
     }
     if (e == hipSuccess) {
         e = device_malloc(c, (void **)&c->d_log, sizeof(bd_level_rec) * c->log_cap);
@@ -395,10 +393,7 @@ extern "C" int bd_destroy(bd_ctx *c) {
     dev_free(c, c->d_mlp_ops);
     dev_free(c, c->d_mlp_ws);
     pool_leave(c);
-    if (c->h_ctl) (void)hipHostFree(c->h_ctl);
-    if (c->h_res) (void)hipHostFree(c->h_res);
-    if (c->h_flags) (void)hipHostFree(c->h_flags);
-    if (c->h_log) (void)hipHostFree(c->h_log);
+    if (c->h_state) (void)hipHostFree(c->h_state);
     free_ring(c);
     for (auto &e : c->ev)
         if (e) (void)hipEventDestroy(e);

@@ -138,8 +138,15 @@ struct search_result {
     uint32_t seq;
 };
 
-// The readout kernels' flags (on a line), then a component run's result.
-constexpr size_t kFlagLine = 128, kFlagBytes = 2 * kFlagLine;
+// What a context pins when it is made, in one piece (each takes 25 us): the
+// mirror of both control blocks, and what the device writes.
+struct host_state {
+    ctl_block ctl[2];
+    alignas(128) search_result res;
+    alignas(128) int32_t flags[32];  // faults a readout kernel found
+    alignas(128) char cc[128];       // a component run's result
+    alignas(128) bd_level_rec log[kHostRecs];
+};
 
 // Device memory a context has, or keeps for its next allocations.
 struct dev_block {
@@ -197,7 +204,7 @@ struct bd_ctx {
     int32_t *d_comp = nullptr;    // connected-component labels (components_)
     int32_t *d_cc_flag = nullptr; // a component run's state and counters
     bool have_cc = false;         // d_comp holds a finished run
-    void *h_cc = nullptr;         // a component run's result, written by the device (behind h_flags)
+    void *h_cc = nullptr;         // h_state's cc
     int32_t cc_hub = 0;           // the vertex of largest degree
     bd::td_task *d_cc_tasks = nullptr;  // slices of the long lists of the edge pass
     int64_t cc_ntasks = -1;             // -1: not built for the resident graph
@@ -213,9 +220,10 @@ struct bd_ctx {
     int64_t tseg_cap = 0;    // entries per task segment (overflow holds task_cap)
     bd::seg_counters *d_seg = nullptr;
     bd::ctl_block *d_ctl = nullptr;  // two published copies (see ctl_block)
-    bd::ctl_block *h_ctl = nullptr;  // pinned mirror of both copies
-    bd::search_result *h_res = nullptr;  // pinned, written by the device
-    bd_level_rec *h_log = nullptr;       // pinned: the first kHostRecs step records
+    bd::host_state *h_state = nullptr;   // pinned, with the parts that the next three name
+    bd::ctl_block *h_ctl = nullptr;      // mirror of both copies
+    bd::search_result *h_res = nullptr;  // written by the device
+    bd_level_rec *h_log = nullptr;       // the first kHostRecs step records
     uint32_t search_seq = 0;             // number of the last search started
     bd_level_rec *d_log = nullptr;       // records past those, and the bit-parallel search's
     int64_t log_cap = 0;
@@ -230,7 +238,7 @@ struct bd_ctx {
     uint64_t *d_tree = nullptr;   // ancestors of a deep parent tree
     int32_t *d_out = nullptr;     // check(): nv parents in graph ids, then nv depths
     uint8_t *d_marks = nullptr;   // check: per range, its spanning list's parent was found
-    int32_t *h_flags = nullptr;   // pinned, kFlagBytes: faults a readout kernel found
+    int32_t *h_flags = nullptr;   // h_state's flags
     void *h_ring = nullptr;       // pinned: results on their way to the caller (bd_readout.hip)
     int64_t ring_bytes = 0;
     hipEvent_t ring_ev[bd::kRing] = {};

@@ -13,7 +13,7 @@ enum { kOutOfMemory = 2, kBlocks = 1 << 16 }; /* hipErrorOutOfMemory */
 static pthread_mutex_t lock = PTHREAD_MUTEX_INITIALIZER;
 static struct { void *p; size_t n; } blocks[kBlocks];
 static size_t device_used, device_peak;
-static size_t device_limit = (size_t)-1, pin_limit = (size_t)-1;
+static size_t device_limit = (size_t)-1, pin_limit = (size_t)-1, pins;
 
 static void *hip(const char *name) {
     static void *lib;
@@ -34,6 +34,8 @@ size_t limits_peak(void) {
     device_peak = device_used;
     return n;
 }
+/* Allocations of pinned memory so far. */
+size_t limits_pins(void) { return pins; }
 void limits_set(size_t device, size_t pin) {
     device_limit = device;
     pin_limit = pin;
@@ -72,5 +74,6 @@ int hipFree(void *p) {
 
 int hipHostMalloc(void **p, size_t n, unsigned flags) {
     if (n > pin_limit) return kOutOfMemory;
+    ++pins;
     return ((int (*)(void **, size_t, unsigned))hip("hipHostMalloc"))(p, n, flags);
 }

@@ -16,7 +16,7 @@ HEAD = """
 import ctypes, sys, threading
 sys.path.insert(0, {root!r})
 lim = ctypes.CDLL({lib!r}, ctypes.RTLD_GLOBAL)
-lim.limits_used.restype = lim.limits_peak.restype = ctypes.c_size_t
+lim.limits_used.restype = lim.limits_peak.restype = lim.limits_pins.restype = ctypes.c_size_t
 lim.limits_set.argtypes = [ctypes.c_size_t, ctypes.c_size_t]
 NONE = 2**64 - 1
 import numpy as np
@@ -158,4 +158,13 @@ for g in got:
     for a, b in zip(g, want):
         np.testing.assert_array_equal(a, b)
 print("done")
+""")
+
+
+def test_a_context_pins_memory_once(limited):
+    limited("""
+for k in range(3):
+    c = bd.Context(0)
+    assert lim.limits_pins() == k + 1
+    c.close()
 """)
